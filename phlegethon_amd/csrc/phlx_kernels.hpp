@@ -17,6 +17,8 @@
 // contraction, so there is no MFMA here; every kernel is HBM/VALU work.
 #pragma once
 
+#include <algorithm>
+
 #include "phlx_internal.hpp"
 
 namespace phlx {
@@ -275,26 +277,31 @@ struct CellW {
 };
 
 // x2 / x3 sweeps with the 2nd-order reconstructions: one thread per
-// (x1, transverse) column walks kSegFaces consecutive faces along DIR,
+// (x1, transverse) column walks segf consecutive faces along DIR,
 // loading each cell once and reconstructing it once; the right edges of
 // cell f-1 are carried to face f.  k_flux builds every face from four cell
 // loads and two reconstructions.  Each face's arithmetic is that of k_flux.
-#ifndef PHLX_SEG_FACES
-#define PHLX_SEG_FACES 32
-#endif
-constexpr int kSegFaces = PHLX_SEG_FACES;
-#ifndef PHLX_FLUX_SEG
-#define PHLX_FLUX_SEG 1
-#endif
-// the mixed-precision sweeps' own choice (their faces cost fewer
-// instructions, which shifts the balance towards more, shorter threads)
-#ifndef PHLX_FLUX_SEG_MX
-#define PHLX_FLUX_SEG_MX PHLX_FLUX_SEG
-#endif
-#ifndef PHLX_SEG_FACES_MX
-#define PHLX_SEG_FACES_MX PHLX_SEG_FACES
-#endif
-constexpr int kSegFacesMx = PHLX_SEG_FACES_MX;
+// This thread's column (x1 cell i, transverse cell o) and the first face f0
+// of its segment, the same in all lanes of a wave.  3D: the columns are
+// numbered along the flattened (x1, x3) or (x1, x2) plane, one segment per
+// blockIdx.y (rows of n1 cells in 64-wide tiles would leave lanes idle at
+// every row end, a third of them at n1 = 133).  2D, where a row is all there
+// is: 64 cells of it per wave, one segment per wave of the block.  False past
+// the grid.
+template <int DIR, int SD>
+__device__ __forceinline__ bool seg_coords(const Grid &g, int segf, int &i, int &o, int &f0) {
+  if (SD == 2) {
+    i = blockIdx.x * 64 + (threadIdx.x & 63);
+    o = 0;
+    f0 = __builtin_amdgcn_readfirstlane((int)(blockIdx.y * 4 + (threadIdx.x >> 6))) * segf;
+    return i < g.n1 && f0 <= g.n2;
+  }
+  const unsigned t = blockIdx.x * 256u + threadIdx.x, n1 = (unsigned)g.n1;
+  o = (int)(t / n1);
+  i = (int)(t - (unsigned)o * n1);
+  f0 = (int)blockIdx.y * segf;
+  return o < ((DIR == 1) ? g.n3 : g.n2);
+}
 
 // SF: USE_SHOCK_FLATTENING -- a flagged cell takes the LIM2ND edges, a face
 // beside one the HLL flux (as k_flux<..., SF>).
@@ -377,15 +384,13 @@ __device__ __forceinline__ void seg_walk(const Grid &g, int i, int o, int f0, in
 }
 
 template <int DIR, int SD, int NAS, bool MHD, int EK, bool SF = false>
-__global__ void __launch_bounds__(256) k_flux_seg(Grid g) {
+__global__ void __launch_bounds__(256) k_flux_seg(Grid g, int segf) {
   static_assert(DIR == 1 || DIR == 2, "x2 / x3 sweeps");
   if (!g.sc->active) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int o = blockIdx.y * blockDim.y + threadIdx.y;  // x3 cell (DIR 1) / x2 cell (DIR 2)
+  int i, o, f0;
+  if (!seg_coords<DIR, SD>(g, segf, i, o, f0)) return;
   const int n = (DIR == 1) ? g.n2 : g.n3;                // cells along DIR
-  if (i >= g.n1 || o >= ((DIR == 1) ? g.n3 : g.n2)) return;
-  const int f0 = blockIdx.z * kSegFaces;
-  const int f1 = min(f0 + kSegFaces, n + 1);
+  const int f1 = min(f0 + segf, n + 1);
   // cells f0 - 2 .. f1 are read
   if (__all(f0 - 2 >= 0 && f1 <= n - 1))
     seg_walk<DIR, SD, NAS, MHD, EK, true, SF>(g, i, o, f0, f1);
@@ -574,15 +579,13 @@ __device__ __forceinline__ void seg_walk_mx(const Grid &g, int i, int o, int f0,
 }
 
 template <int DIR, int SD, int NAS, bool MHD, bool HELM>
-__global__ void __launch_bounds__(256) k_flux_seg_mx(Grid g) {
+__global__ void __launch_bounds__(256) k_flux_seg_mx(Grid g, int segf) {
   static_assert(DIR == 1 || DIR == 2, "x2 / x3 sweeps");
   if (!g.sc->active) return;
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  const int o = blockIdx.y * blockDim.y + threadIdx.y;
+  int i, o, f0;
+  if (!seg_coords<DIR, SD>(g, segf, i, o, f0)) return;
   const int n = (DIR == 1) ? g.n2 : g.n3;
-  if (i >= g.n1 || o >= ((DIR == 1) ? g.n3 : g.n2)) return;
-  const int f0 = blockIdx.z * kSegFacesMx;
-  const int f1 = min(f0 + kSegFacesMx, n + 1);
+  const int f1 = min(f0 + segf, n + 1);
   if (__all(f0 - 2 >= 0 && f1 <= n - 1))
     seg_walk_mx<DIR, SD, NAS, MHD, HELM, true>(g, i, o, f0, f1);
   else
@@ -2036,6 +2039,38 @@ static inline dim3 grid_flat(int e1, int e2, int e3, dim3 blk) {
   return dim3(gr.x * gr.y * gr.z, 1, 1);
 }
 
+// Launch shape of a column-segment sweep: 256 columns per block, segments of
+// segf faces.  A longer segment loads and reconstructs less twice (three
+// cells and one reconstruction per segment), more segments fill the chip:
+//   - at least kSegWavesMin waves (4 per SIMD), down to one face each: with 32
+//     faces a 2D grid had a handful of waves walking in a row (x2 sweep, FP64:
+//     101 x 93 hydro 56 -> 8 us, 333 x 250 MHD 80 -> 11 us; 3D 64 x 60 x 50
+//     MHD 100 -> 20 us);
+//   - up to kSegWaves while a segment keeps 8 faces (150 x 201 x 130 MHD +
+//     Helmholtz: 261 -> 250 us from 4096 to 8192 waves; shorter segments lose
+//     again, 133 x 120 x 97 hydro: 39 us at 6 faces, 43 at 3);
+//   - at most kSegFaces faces (256^3 mixed MHD: 283 us at 29, 259 at 22; FP64
+//     701 and 696).
+constexpr int kSegFaces = 24, kSegLong = 8, kSegWavesMin = 4096, kSegWaves = 8192;
+struct SegShape {
+  dim3 grd;
+  int segf;
+};
+static inline SegShape seg_shape(const Grid &g, int dir) {
+  const int nf = 1 + (dir == 1 ? g.n2 : g.n3);  // faces of a column
+  const int no = g.sd == 2 ? 1 : (dir == 1 ? g.n3 : g.n2);
+  const long long cols = (long long)g.n1 * no, waves = (cols + 63) / 64;
+  auto segs = [&](long long w) { return (int)std::min<long long>((w + waves - 1) / waves, nf); };
+  int nseg = std::max((nf + kSegFaces - 1) / kSegFaces, segs(kSegWavesMin));
+  nseg = std::max(nseg, std::min(segs(kSegWaves), nf / kSegLong));
+  SegShape s;
+  s.segf = (nf + nseg - 1) / nseg;
+  nseg = (nf + s.segf - 1) / s.segf;
+  s.grd = g.sd == 2 ? dim3((g.n1 + 63) / 64, (nseg + 3) / 4)
+                    : dim3((unsigned)((cols + 255) / 256), nseg);
+  return s;
+}
+
 template <int SD, int NAS, bool MHD, int EK, bool MIX, bool R5>
 static void launch_flux(const Grid &g, int dir, hipStream_t st) {
   constexpr bool HELM = EK != EK_IDEAL;
@@ -2046,16 +2081,15 @@ static void launch_flux(const Grid &g, int dir, hipStream_t st) {
       k_flux_x1c<SD, NAS, MHD, EK, true><<<grid_x1_cells(g), 256, 0, st>>>(g);
     } else if (dir == 0) {
       k_flux_mx<0, SD, NAS, MHD, HELM, R5><<<grid_x1_faces(g), blk, 0, st>>>(g);
-    } else if (!R5 && PHLX_FLUX_SEG_MX) {
-      const int n = dir == 1 ? g.n2 : g.n3, no = dir == 1 ? g.n3 : g.n2;
-      const dim3 grd((g.n1 + 63) / 64, (no + 3) / 4, (n + 1 + kSegFacesMx - 1) / kSegFacesMx);
+    } else if constexpr (!R5) {
+      const SegShape s = seg_shape(g, dir);
       if (dir == 1)
-        k_flux_seg_mx<1, SD, NAS, MHD, HELM><<<grd, blk, 0, st>>>(g);
-      else if (SD == 3)
-        k_flux_seg_mx<2, SD, NAS, MHD, HELM><<<grd, blk, 0, st>>>(g);
+        k_flux_seg_mx<1, SD, NAS, MHD, HELM><<<s.grd, 256, 0, st>>>(g, s.segf);
+      else if constexpr (SD == 3)
+        k_flux_seg_mx<2, SD, NAS, MHD, HELM><<<s.grd, 256, 0, st>>>(g, s.segf);
     } else if (dir == 1) {
       k_flux_mx<1, SD, NAS, MHD, HELM, R5><<<grid_for(g.n1, g.n2 + 1, g.n3, blk), blk, 0, st>>>(g);
-    } else if (SD == 3) {
+    } else if constexpr (SD == 3) {
       k_flux_mx<2, SD, NAS, MHD, HELM, R5><<<grid_for(g.n1, g.n2, g.n3 + 1, blk), blk, 0, st>>>(g);
     }
   } else {
@@ -2067,17 +2101,15 @@ static void launch_flux(const Grid &g, int dir, hipStream_t st) {
     }
     if (dir == 0) {
       k_flux<0, SD, NAS, MHD, EK, R5><<<grid_x1_faces(g), blk, 0, st>>>(g);
-    } else if (!R5 && PHLX_FLUX_SEG) {
-      // column segments: (x1 cells, transverse cells, segments of kSegFaces)
-      const int n = dir == 1 ? g.n2 : g.n3, no = dir == 1 ? g.n3 : g.n2;
-      const dim3 grd((g.n1 + 63) / 64, (no + 3) / 4, (n + 1 + kSegFaces - 1) / kSegFaces);
+    } else if constexpr (!R5) {
+      const SegShape s = seg_shape(g, dir);
       if (dir == 1)
-        k_flux_seg<1, SD, NAS, MHD, EK><<<grd, blk, 0, st>>>(g);
-      else if (SD == 3)
-        k_flux_seg<2, SD, NAS, MHD, EK><<<grd, blk, 0, st>>>(g);
+        k_flux_seg<1, SD, NAS, MHD, EK><<<s.grd, 256, 0, st>>>(g, s.segf);
+      else if constexpr (SD == 3)
+        k_flux_seg<2, SD, NAS, MHD, EK><<<s.grd, 256, 0, st>>>(g, s.segf);
     } else if (dir == 1) {
       k_flux<1, SD, NAS, MHD, EK, R5><<<grid_for(g.n1, g.n2 + 1, g.n3, blk), blk, 0, st>>>(g);
-    } else if (SD == 3) {
+    } else if constexpr (SD == 3) {
       k_flux<2, SD, NAS, MHD, EK, R5><<<grid_for(g.n1, g.n2, g.n3 + 1, blk), blk, 0, st>>>(g);
     }
   }
@@ -2090,17 +2122,17 @@ static void launch_flux_sf(const Grid &g, int dir, hipStream_t st) {
   const dim3 blk(64, 4, 1);
   if (dir == 0) {
     k_flux<0, SD, NAS, MHD, EK, R5, true><<<grid_x1_faces(g), blk, 0, st>>>(g);
-  } else if (!R5 && PHLX_FLUX_SEG) {
-    const int n = dir == 1 ? g.n2 : g.n3, no = dir == 1 ? g.n3 : g.n2;
-    const dim3 grd((g.n1 + 63) / 64, (no + 3) / 4, (n + 1 + kSegFaces - 1) / kSegFaces);
+  } else if constexpr (!R5) {
+    const SegShape s = seg_shape(g, dir);
     if (dir == 1)
-      k_flux_seg<1, SD, NAS, MHD, EK, true><<<grd, blk, 0, st>>>(g);
-    else if (SD == 3)
-      k_flux_seg<2, SD, NAS, MHD, EK, true><<<grd, blk, 0, st>>>(g);
-  } else if (dir == 1)
+      k_flux_seg<1, SD, NAS, MHD, EK, true><<<s.grd, 256, 0, st>>>(g, s.segf);
+    else if constexpr (SD == 3)
+      k_flux_seg<2, SD, NAS, MHD, EK, true><<<s.grd, 256, 0, st>>>(g, s.segf);
+  } else if (dir == 1) {
     k_flux<1, SD, NAS, MHD, EK, R5, true><<<grid_for(g.n1, g.n2 + 1, g.n3, blk), blk, 0, st>>>(g);
-  else if (SD == 3)
+  } else if constexpr (SD == 3) {
     k_flux<2, SD, NAS, MHD, EK, R5, true><<<grid_for(g.n1, g.n2, g.n3 + 1, blk), blk, 0, st>>>(g);
+  }
 }
 
 template <int SD, int NAS, bool MHD, bool HELM, bool MIX, bool R5 = false,
