@@ -156,17 +156,18 @@ int phlx_sweep(phlx_ctx *ctx, int32_t dir);
 int phlx_ct(phlx_ctx *ctx, int32_t irk, double a1, double a2, double a3);
 int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, double a3,
                    int32_t last_stage);
-/* Whether phlx_hydro_step / phlx_run fuse each stage's three directional
- * sweeps and flux divergence (the work of sweep(0..2) and the divergence
- * and RK combine of rk_update) into one pass that stages a pencil tile in
- * LDS and keeps the face fluxes out of HBM: mode 1 wherever the run admits
- * it, 0 never, -1 (the default) where it is the faster form: runs without
- * MHD.  It applies to 3D runs with LIM2ND or PPH, the ideal or
- * the FASTEOS Helmholtz state, no shock flattening and nx1, nx2 multiples
- * of 16 (other runs take the separate sweeps).  Either way the results are
- * bit for bit the same.  No counterpart in the reference (its hydro_step is
- * one routine either way): for A/B timing and for callers that want the
- * per-direction kernels. */
+/* Whether phlx_hydro_step / phlx_run fuse each stage's directional sweeps
+ * and flux divergence (the work of sweep(0..2) and the divergence and RK
+ * combine of rk_update; without MHD and with the ideal gas the whole stage,
+ * cons -> prim and the CFL maximum included) into one pass that stages a
+ * pencil tile in LDS and keeps the face fluxes out of HBM: mode 1 wherever the
+ * run admits it, 0 never, -1 (the default) where it is the faster form: runs
+ * without MHD.  It applies with LIM2ND or PPH and no shock flattening to 3D
+ * runs with the ideal or the FASTEOS Helmholtz state and to 2D runs of the
+ * ideal gas without MHD; with MHD, nx1 has to be a multiple of 16 (other runs
+ * take the separate sweeps).  Either way the results are bit for bit the
+ * same.  No counterpart in the reference (its hydro_step is one routine either
+ * way): for A/B timing and for callers that want the per-direction kernels. */
 int phlx_set_fused_sweep(phlx_ctx *ctx, int32_t mode);
 /* Whether phlx_run replays one captured HIP graph per step (on = 1) instead
  * of launching the step's kernels one by one (0, the default).  The step is
@@ -346,7 +347,7 @@ int phlx_compute_dt_noalloc(const phlx_config *cfg, const double *prim, const do
 /* Per-kernel device time accumulated while profiling is on (HIP events on
  * the context stream).  kernel ids: 0 flux x1, 1 flux x2, 2 flux x3,
  * 3 corner EMF, 4 face-B, 5 update, 6 misc (shock flags), 7 thermal
- * diffusion. */
+ * diffusion, 8 fused sweep. */
 int phlx_profile_enable(phlx_ctx *ctx, int32_t on);
 int phlx_profile_read(phlx_ctx *ctx, int32_t kernel, double *total_ms, int64_t *launches);
 /* Bandwidth probe: copies nbytes between two fresh device buffers `reps`

@@ -236,6 +236,12 @@ extern "C" int phlx_create(const phlx_config *cfg, phlx_ctx **out) {
   e |= dalloc(ctx, &g.U0, nv * N);
   e |= dalloc(ctx, &g.eint, N);
   if (cfg->precision == PHLX_PREC_MIXED) e |= dalloc(ctx, &g.Pf, (nv + 5) * N);
+  if (ctx->kt.sweep && !ctx->kt.update_swept) {
+    if (cfg->precision == PHLX_PREC_MIXED)
+      e |= dalloc(ctx, &g.Pfn, nv * N);
+    else
+      e |= dalloc(ctx, &g.Pn, nv * N);
+  }
   for (int d = 0; d < g.sd; d++) {
     e |= dalloc(ctx, &g.F[d], nv * (size_t)g.nf[d]);
     g.Ff[d] = (float *)g.F[d];  // the mixed path stores FP32 fluxes in the same buffer
@@ -276,7 +282,10 @@ extern "C" int phlx_create(const phlx_config *cfg, phlx_ctx **out) {
   e |= dalloc(ctx, &g.sc, 1);
   e |= dalloc(ctx, &ctx->scratch_val, 1);
   g.nred = cell_grid_blocks(g);
-  e |= dalloc(ctx, &g.red, (size_t)g.nred);
+  // partials of a cell-grid launch, or of a fused sweep of one plane per block
+  const size_t nsw = (size_t)((g.n1 + kSweepT - 1) / kSweepT) *
+                     ((g.n2 + kSweepTy - 1) / kSweepTy) * g.n3;
+  e |= dalloc(ctx, &g.red, std::max((size_t)g.nred, nsw));
   if (helm) {
     e |= dalloc(ctx, &g.eos_part, 3 * (size_t)g.nred);
     e |= dalloc(ctx, &g.mlp_y, N);
@@ -673,9 +682,10 @@ extern "C" int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, 
   return rk_update(ctx, irk, a1, a2, a3, last_stage, false);
 }
 
-// Whether hydro_step takes the fused sweep: a family that has one, no shock
-// flattening (its flagged cells switch scheme per face), and x1 tiles that
-// divide the grid.
+// Whether hydro_step takes the fused sweep: a family that has one and no shock
+// flattening (its flagged cells switch scheme per face); with MHD, x1 tiles
+// that divide the grid.  A captured step keeps its buffers, so an odd number
+// of whole-stage passes, which ends in the other one, is not captured.
 static bool use_fused_sweep(const phlx_ctx *ctx) {
   const Grid &g = ctx->g;
   // measured on MI355X: without MHD the fused stage is 5-19 % faster (FP64
@@ -683,7 +693,9 @@ static bool use_fused_sweep(const phlx_ctx *ctx) {
   // column segments prefetch a cell ahead at 3-4 waves/SIMD; FP64: the
   // fused MHD sweep spills)
   const bool want = ctx->fused_sweep < 0 ? !ctx->g.mhd : ctx->fused_sweep != 0;
-  return want && ctx->kt.sweep && !g.sflat && g.sd == 3 && g.n1 % kSweepT == 0 &&
+  if (!want || !ctx->kt.sweep || g.sflat) return false;
+  if (!ctx->kt.update_swept) return !(ctx->step_graph && ctx->stages % 2);
+  return (!g.mhd || g.n1 % kSweepT == 0) &&
          (!ctx->kt.update_guess || ctx->kt.update_swept_guess);
 }
 
@@ -707,8 +719,11 @@ static int materialize(phlx_ctx *ctx) {
   return check_launch();
 }
 
-static int do_hydro_step(phlx_ctx *ctx, bool with_cfl) {
+// n_cfl: the partials of the CFL maximum that the last stage leaves.
+static int do_hydro_step(phlx_ctx *ctx, bool with_cfl, int *n_cfl = nullptr) {
   const bool fused = use_fused_sweep(ctx);
+  const bool whole = fused && !ctx->kt.update_swept;
+  if (n_cfl) *n_cfl = ctx->g.nred;
   for (int irk = 0; irk < ctx->stages; irk++) {
     int rc = phlx_stage_begin(ctx, irk);
     if (rc) return rc;
@@ -716,11 +731,23 @@ static int do_hydro_step(phlx_ctx *ctx, bool with_cfl) {
     if (fused) {
       ProfRec r;
       int on = kbegin(ctx, KID_SWEEP, r);
-      ctx->kt.sweep(ctx->g, irk == 0 ? 1 : 0, irk == ctx->stages - 1 ? 1 : 0, a1, a2, a3,
-                    ctx->stream);
+      const int fin = irk == ctx->stages - 1;
+      const int blocks = ctx->kt.sweep(ctx->g, irk == 0 ? 1 : 0, with_cfl && fin, fin, a1, a2, a3,
+                                       ctx->stream);
       kend(ctx, on, r);
       rc = check_launch();
       if (rc) return rc;
+      if (whole) {
+        Grid &g = ctx->g;
+        if (g.Pfn)
+          std::swap(g.Pf, g.Pfn);
+        else
+          std::swap(g.P, g.Pn);
+        ctx->tdiff_valid = false;
+        if (fin && ctx->kt.prims) ctx->prim_stale = true;
+        if (n_cfl) *n_cfl = blocks;
+        continue;
+      }
     } else {
       for (int d = 0; d < ctx->g.sd; d++) {
         rc = phlx_sweep(ctx, d);
@@ -788,7 +815,7 @@ extern "C" int phlx_compute_dt(phlx_ctx *ctx, double *dt_out, double *smax_out) 
   if (!ctx->initialized) return PHLX_E_STATE;
   if (const int m = materialize(ctx)) return m;
   ctx->kt.cfl(ctx->g, ctx->stream);
-  launch_step_end(ctx->g, 0, ctx->stream);
+  launch_step_end(ctx->g, ctx->g.nred, 0, 0, ctx->stream);
   int rc = check_launch();
   if (rc) return rc;
   if (dt_out || smax_out) {
@@ -834,8 +861,9 @@ static int step_graph_ready(phlx_ctx *ctx) {
   drop_step_graph(ctx);
   HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   launch_step_begin(ctx->g.sc, ctx->stream);
-  const int rc = do_hydro_step(ctx, true);
-  launch_step_end(ctx->g, 1, ctx->stream);
+  int n_cfl;
+  const int rc = do_hydro_step(ctx, true, &n_cfl);
+  launch_step_end(ctx->g, n_cfl, 1, 0, ctx->stream);
   hipGraph_t gr = nullptr;
   const hipError_t e = hipStreamEndCapture(ctx->stream, &gr);
   if (rc || e != hipSuccess) {
@@ -869,22 +897,23 @@ extern "C" int phlx_run(phlx_ctx *ctx, int32_t nsteps) {
     if (ctx->kt.prims) ctx->prim_stale = true;
     return PHLX_OK;
   }
+  if (nsteps > 0) launch_step_begin(ctx->g.sc, ctx->stream);
   for (int s = 0; s < nsteps; s++) {
-    launch_step_begin(ctx->g.sc, ctx->stream);
-    int rc;
+    int rc, n_cfl;
     if (diff) {
       // THERMAL_DIFFUSION_STS around hydro_step (source/source.F90:6672-6688);
       // the hyperbolic dt follows the second half (:6716)
       if (ctx->diff_eval && (rc = parabolic_dt(ctx))) return rc;
       if ((rc = diffusion_step(ctx, 1))) return rc;
     }
-    rc = do_hydro_step(ctx, !diff);
+    rc = do_hydro_step(ctx, !diff, &n_cfl);
     if (rc) return rc;
     if (diff) {
       if ((rc = diffusion_step(ctx, 2))) return rc;
       ctx->kt.cfl(ctx->g, ctx->stream);
+      n_cfl = ctx->g.nred;
     }
-    launch_step_end(ctx->g, 1, ctx->stream);
+    launch_step_end(ctx->g, n_cfl, 1, s + 1 < nsteps, ctx->stream);
     rc = check_launch();
     if (rc) return rc;
   }

@@ -55,6 +55,11 @@ struct Grid {
   // the cell-centred B, nv+3 / nv+4 gamma_e (deviation) / gamma_c; written by
   // the update (and k_pack_f), read by the mixed flux kernels
   float *Pf;
+  // ideal hydro in whole-stage passes (k_sweep): the buffer the next stage's
+  // primitives go to (FP64; the FP32 sweep inputs in the mixed path); the
+  // host swaps it with P / Pf after the launch
+  double *Pn;
+  float *Pfn;
   double *bf[3], *b0f[3];
   double *F[3];
   float *Ff[3];            // FP32 view of F[d] (mixed precision: fluxes stored as FP32)

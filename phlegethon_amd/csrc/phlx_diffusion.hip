@@ -203,7 +203,8 @@ __global__ void __launch_bounds__(256) k_parabolic(Grid g, double inv_dl2) {
   // block maximum (max is exact, so the order does not matter)
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = fmax(v, __shfl_xor(v, o));
-  if (threadIdx.x == 0) red[threadIdx.y] = v;
+  const int tid = threadIdx.y * blockDim.x + threadIdx.x;
+  if ((tid & 63) == 0) red[tid >> 6] = v;
   __syncthreads();
   if (threadIdx.x == 0 && threadIdx.y == 0) {
     const double m = fmax(fmax(red[0], red[1]), fmax(red[2], red[3]));
@@ -212,18 +213,19 @@ __global__ void __launch_bounds__(256) k_parabolic(Grid g, double inv_dl2) {
 }
 
 static dim3 diff_grid(const Grid &g) {
-  return dim3((g.n1 + 63) / 64, (g.n2 + 3) / 4, g.n3);
+  const dim3 b = cell_block(g);
+  return dim3((g.n1 + b.x - 1) / b.x, (g.n2 + b.y - 1) / b.y, g.n3);
 }
 
 void launch_diff_t_from_p(const Grid &g, hipStream_t st) {
-  const dim3 blk(64, 4, 1);
+  const dim3 blk = cell_block(g);
   if (g.sd == 3) k_diff_t_from_p<3><<<diff_grid(g), blk, 0, st>>>(g);
   else k_diff_t_from_p<2><<<diff_grid(g), blk, 0, st>>>(g);
 }
 
 void launch_diff_stage(const Grid &g, bool first, double mu, double nu, double c0, double hm,
                        double hg, hipStream_t st) {
-  const dim3 blk(64, 4, 1);
+  const dim3 blk = cell_block(g);
   if (g.sd == 3) {
     if (first) k_diff_stage<3, true><<<diff_grid(g), blk, 0, st>>>(g, mu, nu, c0, hm, hg);
     else k_diff_stage<3, false><<<diff_grid(g), blk, 0, st>>>(g, mu, nu, c0, hm, hg);
@@ -234,7 +236,7 @@ void launch_diff_stage(const Grid &g, bool first, double mu, double nu, double c
 }
 
 void launch_diff_temp(const Grid &g, bool helm, hipStream_t st) {
-  const dim3 blk(64, 4, 1);
+  const dim3 blk = cell_block(g);
   if (g.sd == 3) {
     if (helm) k_diff_temp<3, true><<<diff_grid(g), blk, 0, st>>>(g);
     else k_diff_temp<3, false><<<diff_grid(g), blk, 0, st>>>(g);
@@ -245,7 +247,7 @@ void launch_diff_temp(const Grid &g, bool helm, hipStream_t st) {
 }
 
 void launch_diff_final(const Grid &g, bool helm, hipStream_t st) {
-  const dim3 blk(64, 4, 1);
+  const dim3 blk = cell_block(g);
   if (g.sd == 3) {
     if (helm) k_diff_final<3, true><<<diff_grid(g), blk, 0, st>>>(g);
     else k_diff_final<3, false><<<diff_grid(g), blk, 0, st>>>(g);
@@ -256,7 +258,7 @@ void launch_diff_final(const Grid &g, bool helm, hipStream_t st) {
 }
 
 void launch_parabolic(const Grid &g, double inv_dl2, hipStream_t st) {
-  const dim3 blk(64, 4, 1);
+  const dim3 blk = cell_block(g);
   if (g.sd == 3) k_parabolic<3><<<diff_grid(g), blk, 0, st>>>(g, inv_dl2);
   else k_parabolic<2><<<diff_grid(g), blk, 0, st>>>(g, inv_dl2);
 }

@@ -7,8 +7,8 @@
 
 namespace phlx {
 
-// x1 tile edge of the fused sweep: it runs where it divides the grid
-constexpr int kSweepT = 16;
+// the fused sweep's (x1, x2) tile
+constexpr int kSweepT = 16, kSweepTy = 15;
 
 // Where k_faceb takes b0 and puts the new face field (its comment has the
 // four cases); RK2 steps alternate the face-field buffers instead of
@@ -28,10 +28,13 @@ struct KernelTable {
   // mixed precision: refresh the FP32 sweep inputs from the FP64 state
   void (*pack)(const Grid &, hipStream_t);
   void (*prims)(const Grid &, hipStream_t);   // mixed: FP64 prim / eint / b_cc from U
-  // fused sweep (3D, 2nd-order reconstructions, ideal / FASTEOS states;
-  // null otherwise): one pass forms the stage's conserved state, the swept
-  // updates finish it after CT
-  void (*sweep)(const Grid &, int, int, double, double, double, hipStream_t);
+  // fused sweep (2nd-order reconstructions, ideal / FASTEOS states, 3D or 2D
+  // ideal hydro; null otherwise): one pass forms the stage's conserved state
+  // and the swept updates finish it after CT; without update_swept (ideal
+  // hydro) the pass is the whole stage, its new primitives in the other
+  // buffer (Grid::Pn / Pfn).  Returns the blocks launched (partials of the CFL
+  // maximum).
+  int (*sweep)(const Grid &, int, int, int, double, double, double, hipStream_t);
   void (*update_swept)(const Grid &, int, int, double, double, double, int, hipStream_t);
   void (*update_swept_guess)(const Grid &, int, int, double, double, double, int, hipStream_t);
 };
@@ -46,8 +49,19 @@ bool select_mixed_r5(int sd, int nas, bool mhd, bool helm, bool fasteos, KernelT
 void launch_step_begin(Scalars *sc, hipStream_t st);
 // device state flags: flags = (flags & keep) | set
 void launch_flags(Scalars *sc, int keep, int set, hipStream_t st);
-void launch_step_end(const Grid &g, int advance, hipStream_t st);
+// n: partials of the CFL maximum in g.red; begin: another step follows at once
+// (launch_step_begin's work in the same launch)
+void launch_step_end(const Grid &g, int n, int advance, int begin, hipStream_t st);
 void launch_reduce_to(const Grid &g, double *out, hipStream_t st);
+// Block of the cell-grid kernels: (64, 4), or (32, 8) where that leaves fewer
+// idle lanes (n1 = 150: 160 lanes per row instead of 192).  All launches whose
+// block maxima g.red collects (Grid::nred of them) take it.
+inline dim3 cell_block(const Grid &g) {
+  auto lanes = [&](int w, int h) {
+    return (long long)((g.n1 + w - 1) / w * w) * ((g.n2 + h - 1) / h * h);
+  };
+  return lanes(32, 8) < lanes(64, 4) ? dim3(32, 8, 1) : dim3(64, 4, 1);
+}
 int cell_grid_blocks(const Grid &g);
 void launch_stream_copy(const void *src, void *dst, long long n16, hipStream_t st);
 // USE_SHOCK_FLATTENING flags of the current primitive state (g.sf_flag)

@@ -7,9 +7,11 @@
 //   k_faceb                              face-B update (FP64)         (MHD)
 //   k_update                             flux divergence + sources + RK combine
 //                                        + cons->prim (+ CFL max at the last stage)
-// or, fused (k_sweep, 3D with the 2nd-order reconstructions),
-//   k_sweep                              the three sweeps + divergence + sources
-//                                        + RK combine in one pass over LDS tiles
+// or, fused (k_sweep, the 2nd-order reconstructions),
+//   k_sweep                              the sweeps + divergence + sources
+//                                        + RK combine in one pass over LDS tiles;
+//                                        ideal hydro: also cons->prim and CFL,
+//                                        the whole stage
 //   k_corner, k_faceb                    as above (MHD)
 //   k_update<..., SWEPT>                 cons->prim (+ CFL max at the last stage)
 // Ghost zones are never stored: loads outside the interior go through the
@@ -1234,7 +1236,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
     for (int v = 0; v < NV; v++) {
       if (!MIX && (!HELM || v != IE)) g.P[v * N + c] = p[v];
-      out[v * N + c] = S[v];
+      if (!SWEPT) out[v * N + c] = S[v];
     }
     if (!MIX) g.eint[c] = eint;
     if constexpr (MIX) {
@@ -1579,9 +1581,10 @@ __global__ void __launch_bounds__(256) k_divb(Grid g) {
 
 // ------------------------------------------------------------ fused sweep
 // One RK stage's reconstruction, Riemann fluxes and flux divergence in one
-// pass (3D, the 2nd-order reconstructions, ideal or FASTEOS states; FP64 or
-// the mixed-precision policy).  A block of 256 threads owns a 16 x 15
-// (x1, x2) tile of columns and walks a chunk of kSweepK planes along x3.
+// pass (the 2nd-order reconstructions, ideal or FASTEOS states; FP64 or the
+// mixed-precision policy; 3D, and 2D ideal hydro as the one plane).  A block of
+// 256 threads owns a 16 x 15 (x1, x2) tile of columns and walks a chunk of kc
+// planes along x3 (sweep_grid).
 // Per plane the tile plus a 2-cell halo of sweep inputs (WB deviations,
 // cell B, FASTEOS gammas: what load_cell / load_cell_f return) is staged in
 // LDS, SoA.  The tile's 17 x 15 x1 faces, 16 x 16 x2 faces and 16 x 15 x3
@@ -1601,13 +1604,16 @@ __global__ void __launch_bounds__(256) k_divb(Grid g) {
 // combination a1 S0 + a2 S + a3 dt R is written where k_update would write
 // it (stage 1 also rebuilds state0 as k_update does, or, mixed, takes it
 // from U when the device flags say U is current).  k_update<..., SWEPT>
-// then runs cons -> prim, the EoS and the CFL after CT.
-// Requires n1 % 16 == 0 (checked by the host); a last x2 tile past n2
-// masks its missing rows.
-#ifndef PHLX_SWEEP_KC
-#define PHLX_SWEEP_KC 32
-#endif
-constexpr int kSweepK = PHLX_SWEEP_KC, kSweepTy = 15;
+// then runs cons -> prim, the EoS and the CFL after CT (it leaves U as it is:
+// 100 -> 60 B per cell of the mixed ideal gas).
+// FUSE (the ideal gas without a field, where nothing stands between the RK
+// combination and cons -> prim): the pass is the whole stage.  The new
+// primitives go to a second buffer, since neighbouring blocks still read the
+// old ones, and the host swaps the two.  A 2D step is then three launches of
+// ~10 us (101 x 93 FP64: 36 -> 22 us, 256^2 mixed 31 -> 20), and a 3D one reads
+// and writes U once less (384^3 LHLLC: FP64 12.5 -> 10.25 ms per step, mixed
+// 6.14 -> 5.89, where the mixed pass is bound by its face solves).
+// Last tiles past n1 or n2 mask their missing columns.
 template <int D>
 struct SweepDir {
   static constexpr int value = D;
@@ -1620,13 +1626,15 @@ struct SweepDir {
 #define PHLX_SWEEP_WAVES_MX 2
 #endif
 
-template <int NAS, bool MHD, int EK, bool MIX>
+template <int SD, int NAS, bool MHD, int EK, bool MIX, bool FUSE>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(MIX ? PHLX_SWEEP_WAVES_MX : PHLX_SWEEP_WAVES)))
-    k_sweep(Grid g, int first, int fin, double a1, double a2, double c3) {
-  constexpr int SD = 3, NV = SD + 2 + NAS, IE = SD + 1, IA = SD + 2;
+    k_sweep(Grid g, int first, int last, int fin, double a1, double a2, double c3, int kc) {
+  constexpr int NV = SD + 2 + NAS, IE = SD + 1, IA = SD + 2;
   constexpr bool GAM = EK == EK_FASTEOS;
   static_assert(EK != EK_HELM_FACE, "per-face Newton states are not staged");
+  static_assert(!FUSE || (!MHD && EK == EK_IDEAL), "the stage's end without CT and EoS solve");
+  static_assert(SD == 3 || FUSE, "2D stages are fused ones");
   using Re = typename std::conditional<MIX, float, double>::type;
   constexpr int TX = kSweepT, TY = kSweepTy;     // cells per tile
   constexpr int W = TX + 4, WW = W * (TY + 4);   // LDS row, cells per variable
@@ -1637,16 +1645,38 @@ __global__ void __launch_bounds__(256)
   // interior is then staged while plane k is solved, and no cell of the x3
   // window stays in registers across the in-plane solves
   constexpr int kTileB = NC * WW * (int)sizeof(Re), kFaceB = NV * (NF1 + NF2) * (int)sizeof(Re);
-  constexpr bool DB = 2 * kTileB + kFaceB <= 53 * 1024;
+  constexpr bool DB = SD == 3 && 2 * kTileB + kFaceB <= 53 * 1024;
   __shared__ Re tile[(DB ? 2 : 1) * NC * WW];
   __shared__ Re f1[NV * NF1];  // x1 faces: [v][row b][face a = 0..16]
   __shared__ Re f2[NV * NF2];  // x2 faces: [v][face b = 0..15][column a]
-  if (!g.sc->active) return;
   const int tid = threadIdx.x;
-  const int ntx = g.n1 / TX;
+  const int ntx = (g.n1 + TX - 1) / TX;
   const int i0 = (blockIdx.x % ntx) * TX, j0 = (blockIdx.x / ntx) * TY;
-  const int k0 = blockIdx.y * kSweepK, k1 = min(k0 + kSweepK, g.n3);
+  const int k0 = blockIdx.y * kc, k1 = min(k0 + kc, g.n3);
   const long long N = g.N;
+  if (!g.sc->active) {
+    if constexpr (FUSE) {
+      // the other buffer becomes the current one (sweep_swap): it takes the
+      // state unchanged
+      const int i = i0 + (tid & (TX - 1)), j = j0 + (tid >> 4);
+      if ((tid >> 4) < TY && i < g.n1 && j < g.n2) {
+        for (int kk = k0; kk < k1; kk++)
+          for (int v = 0; v < NV; v++) {
+            const long long x = v * N + cix(g, i, j, kk);
+            if (MIX)
+              g.Pfn[x] = g.Pf[x];
+            else
+              g.Pn[x] = g.P[x];
+          }
+      }
+    }
+    return;
+  }
+  if (FUSE && MIX && fin && !first && blockIdx.x == 0 && blockIdx.y == 0 && tid == 0) {
+    // as k_update: no thread of this launch reads the flags
+    g.sc->flags = SC_U_CUR | SC_P_STALE;
+  }
+  double smax_local = 0.0;
   // thread (a, b): column (i0 + a, j0 + b) for b < TY (the last thread row
   // has no column; it takes the tile's upper x1 faces)
   const bool own = (tid >> 4) < TY;
@@ -1655,9 +1685,11 @@ __global__ void __launch_bounds__(256)
   struct Cell {
     Re q[NV], b[3], ga[2];
   };
-  // rows past n2 + 1 (a partial last tile) are read as row n2 + 1: no
-  // face inside the grid reaches them, and the ghost map covers two rows
+  // cells past n1 + 1 and n2 + 1 (partial last tiles) are read as cell
+  // n1 + 1 and row n2 + 1: no face inside the grid reaches them, and the
+  // ghost map covers two cells
   auto load = [&](int ii, int jj, int kk, Cell &c) {
+    ii = min(ii, g.n1 + 1);
     jj = min(jj, g.n2 + 1);
     const bool in = ii >= 0 && ii < g.n1 && jj >= 0 && jj < g.n2 && kk >= 0 && kk < g.n3;
     if constexpr (MIX) {
@@ -1743,10 +1775,14 @@ __global__ void __launch_bounds__(256)
   if (own) {
     const int a = tid & (TX - 1), b = tid >> 4, i = i0 + a, j = j0 + b;
     Cell cA, cB, cC;
-    load(i, j, k0 - 2, cA);
-    load(i, j, k0 - 1, cB);
     load(i, j, k0, cC);
-    load(i, j, k0 + 1, nxt);
+    if constexpr (SD == 2) {
+      cA = cB = nxt = cC;  // no x3 stencil
+    } else {
+      load(i, j, k0 - 2, cA);
+      load(i, j, k0 - 1, cB);
+      load(i, j, k0 + 1, nxt);
+    }
     Re l, qL[NV], qR[NV], bL[3] = {0, 0, 0}, bR[3] = {0, 0, 0}, gL[2] = {0, 0}, gR[2] = {0, 0};
 #pragma unroll
     for (int v = 0; v < NV; v++) {
@@ -1767,7 +1803,8 @@ __global__ void __launch_bounds__(256)
         edges(false, cB.ga[c], cC.ga[c], nxt.ga[c], gR[c], rg[c]);
       }
     }
-    if (j < g.n2) solve(SweepDir<2>{}, i, j, k0, qL, qR, bL, bR, gL, gR, F3m);
+    if constexpr (SD == 3)
+      if (i < g.n1 && j < g.n2) solve(SweepDir<2>{}, i, j, k0, qL, qR, bL, bR, gL, gR, F3m);
     put(plane(k0), (b + 2) * W + a + 2, cC);
   }
 
@@ -1787,7 +1824,7 @@ __global__ void __launch_bounds__(256)
     int lt = tid;
     asm volatile("" : "+v"(lt));
     const int la = lt & (TX - 1), lb = lt >> 4, li = i0 + la, lj = j0 + lb;
-    const bool col = lb < TY && lj < g.n2;  // a column inside the grid
+    const bool col = lb < TY && li < g.n1 && lj < g.n2;  // a column inside the grid
     Re *const tk = plane(k);
     const int mine = (lb + 2) * W + la + 2;
     // double tile: cell k+1 of this column into plane k+1's tile (whose
@@ -1817,17 +1854,19 @@ __global__ void __launch_bounds__(256)
     // the lower face of row lb (16 faces: row 15's is the tile's upper face)
     {
       const int fa = lb < TY ? la : TX, fb = lb < TY ? lb : la;
-      if (fb < TY && j0 + fb < g.n2) plane_face(SweepDir<0>{}, tk, fa, fb, k);
+      if (fb < TY && i0 + fa <= g.n1 && j0 + fb < g.n2) plane_face(SweepDir<0>{}, tk, fa, fb, k);
     }
-    if (lj <= g.n2) plane_face(SweepDir<1>{}, tk, la, lb, k);
+    if (li < g.n1 && lj <= g.n2) plane_face(SweepDir<1>{}, tk, la, lb, k);
     // cell k+2 of this column, in flight across the barrier
     Cell cp;
-    if (lb < TY) load(li, lj, k + 2, cp);
+    if constexpr (SD == 3)
+      if (lb < TY) load(li, lj, k + 2, cp);
     __syncthreads();
     if (lb < TY) {
       // x3: face k+1 of this column from cells k (LDS), k+1, k+2
       Re qL[NV], qR[NV], bL[3] = {0, 0, 0}, bR[3] = {0, 0, 0}, gL[2] = {0, 0}, gR[2] = {0, 0};
       Re F3p[NV];
+      if constexpr (SD == 3) {
       const Re *qm = tk + mine;
       const Re *q1 = plane(k + 1) + mine;
 #pragma unroll
@@ -1851,10 +1890,13 @@ __global__ void __launch_bounds__(256)
                 rg[c]);
         }
       }
+      }
       // single tile: plane k's reads are done (this thread's own cell k was
       // the last, just above), so cell k+1 takes its slot
-      if (!DB && k + 1 < k1) put(tk, mine, nxt);
-      nxt = cp;
+      if (SD == 3) {
+        if (!DB && k + 1 < k1) put(tk, mine, nxt);
+        nxt = cp;
+      }
       if (col) {
         // the stage's state (state0 and stage state, or state0 rebuilt from
         // the primitives) first: its loads are in flight during the x3 solve
@@ -1871,11 +1913,11 @@ __global__ void __launch_bounds__(256)
           double p[NV];
 #pragma unroll
           for (int v = 0; v < NV; v++) p[v] = g.P[v * N + c];
-          const double rho = p[0], v1 = p[1], v2 = p[2], v3 = p[3];
+          const double rho = p[0], v1 = p[1], v2 = p[2], v3 = (SD == 3) ? p[3] : 0.0;
           S0[0] = rho;
           S0[1] = rho * v1;
           S0[2] = rho * v2;
-          S0[3] = rho * v3;
+          if (SD == 3) S0[3] = rho * v3;
           double E = g.eint[c] + 0.5 * rho * (v1 * v1 + v2 * v2 + v3 * v3);
           if (MHD) {
             const double b1 = g.bcc[c], b2 = g.bcc[N + c], b3 = g.bcc[2 * N + c];
@@ -1897,7 +1939,7 @@ __global__ void __launch_bounds__(256)
             S[v] = s_buf[v * N + c];
           }
         }
-        solve(SweepDir<2>{}, li, lj, k + 1, qL, qR, bL, bR, gL, gR, F3p);
+        if constexpr (SD == 3) solve(SweepDir<2>{}, li, lj, k + 1, qL, qR, bL, bR, gL, gR, F3p);
         // divergence (x1 overwrites, x2 and x3 accumulate), sources, RK
 #pragma unroll
         for (int v = 0; v < NV; v++) {
@@ -1905,8 +1947,10 @@ __global__ void __launch_bounds__(256)
           const Re *F2 = f2 + v * NF2 + lb * TX + la;
           R[v] = ((double)F1[1] - (double)F1[0]) * g.inv_dx[0];
           R[v] = R[v] + ((double)F2[TX] - (double)F2[0]) * g.inv_dx[1];
-          R[v] = R[v] + ((double)F3p[v] - (double)F3m[v]) * g.inv_dx[2];
-          F3m[v] = F3p[v];
+          if (SD == 3) {
+            R[v] = R[v] + ((double)F3p[v] - (double)F3m[v]) * g.inv_dx[2];
+            F3m[v] = F3p[v];
+          }
         }
         if (g.grav) {
           const double r0 = S[0];
@@ -1918,10 +1962,45 @@ __global__ void __launch_bounds__(256)
         if (g.edot) R[IE] = R[IE] - g.edot_cc[lj];
         const double a3 = c3 * g.sc->dt;
 #pragma unroll
-        for (int v = 0; v < NV; v++) out[v * N + c] = a1 * S0[v] + a2 * S[v] + a3 * R[v];
+        for (int v = 0; v < NV; v++) {
+          S[v] = a1 * S0[v] + a2 * S[v] + a3 * R[v];
+          out[v * N + c] = S[v];
+        }
+        if constexpr (FUSE) {
+          // cons -> prim and the CFL speed, as k_update (the ideal gas without
+          // a field), into the buffer that no block reads in this launch
+          const double rho = S[0], m1 = S[1], m2 = S[2], m3 = (SD == 3) ? S[3] : 0.0;
+          const double ir = 1.0 / rho;
+          double p[NV];
+          double eint = S[IE] - 0.5 * (m1 * m1 + m2 * m2 + m3 * m3) * ir;
+          if (g.etot) eint = eint - rho * g.phi_cc[lj];
+          p[0] = rho;
+          p[1] = m1 * ir;
+          p[2] = m2 * ir;
+          if (SD == 3) p[3] = m3 * ir;
+#pragma unroll
+          for (int v = IA; v < NV; v++) p[v] = S[v] * ir;
+          p[IE] = g.gmm1 * eint;
+          if constexpr (MIX) {
+#pragma unroll
+            for (int v = 0; v < NV; v++) {
+              double x = p[v];
+              if (g.wb && v == 0) x = x - g.eq_rho_cc[lj];
+              if (g.wb && v == IE) x = x - g.eq_p_cc[lj];
+              g.Pfn[v * N + c] = (float)x;
+            }
+          } else {
+            g.eint[c] = eint;
+#pragma unroll
+            for (int v = 0; v < NV; v++) g.Pn[v * N + c] = p[v];
+          }
+          if (last)
+            smax_local = fmax(smax_local, cell_speed<SD, false, false>(g, p, nullptr, 0.0));
+        }
       }
     }
   }
+  if (FUSE && last) block_max_to(smax_local, g.red);
 }
 
 // ------------------------------------------------------- shock flattening
@@ -2135,6 +2214,24 @@ static void launch_flux_sf(const Grid &g, int dir, hipStream_t st) {
   }
 }
 
+// Grid of the fused sweep: 16 x 15 tiles by chunks of kc planes.  A chunk
+// solves one x3 face and loads three cells of every column more than its
+// planes need, and a launch of few long chunks leaves CUs idle at its end:
+// about kSweepBlocks blocks (4-6 per CU slot), at most kSweepK planes each.
+// Sweep times, us, by planes per chunk (FP64 hydro):
+//   384^3 LHLLC         3: 5533   5: 5301   12: 5136   16: 5132   32: 5219
+//   192 x 256 x 192 Helmholtz  3: 1399  5: 1345  12: 1342  16: 1398  32: 1531
+//   150 x 100 x 120     3: 223    5: 226    8: 251    12: 230     32: 365
+//   64 x 60 x 50        1: 39     2: 36     3: 39     6: 67       32: 308
+constexpr int kSweepK = 12, kSweepBlocks = 3072;
+static inline dim3 sweep_grid(const Grid &g, int &kc) {
+  const int tiles = ((g.n1 + kSweepT - 1) / kSweepT) * ((g.n2 + kSweepTy - 1) / kSweepTy);
+  const long long planes = (long long)tiles * g.n3;
+  kc = (int)std::min<long long>((planes + kSweepBlocks / 2) / kSweepBlocks, kSweepK);
+  kc = std::max(kc, 1);
+  return dim3((unsigned)tiles, (unsigned)((g.n3 + kc - 1) / kc), 1);
+}
+
 template <int SD, int NAS, bool MHD, bool HELM, bool MIX, bool R5 = false,
           int EK = HELM ? EK_FASTEOS : EK_IDEAL>
 struct Kern {
@@ -2158,31 +2255,36 @@ struct Kern {
   }
   static void update(const Grid &g, int first, int last, double a1, double a2, double c3,
                      int fin, hipStream_t st) {
-    const dim3 blk(64, 4, 1);
+    const dim3 blk = cell_block(g);
     k_update<SD, NAS, MHD, HELM, MIX><<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(
         g, first, last, a1, a2, c3, fin);
   }
   static void update_guess(const Grid &g, int first, int last, double a1, double a2, double c3,
                            int fin, hipStream_t st) {
-    const dim3 blk(64, 4, 1);
+    const dim3 blk = cell_block(g);
     k_update<SD, NAS, MHD, HELM, MIX, true><<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(
         g, first, last, a1, a2, c3, fin);
   }
-  // the fused sweep and the update that finishes its stage after CT
-  // (3D FP64 with the 2nd-order reconstructions and ideal / FASTEOS states)
-  static constexpr bool kSwept = SD == 3 && !R5 && EK != EK_HELM_FACE;
-  static void sweep(const Grid &g, int first, int fin, double a1, double a2, double c3,
-                    hipStream_t st) {
+  // the fused sweep, whole stages of it where nothing but cons -> prim follows
+  // the RK combination (kWhole), else the sweep and the update that finishes
+  // its stage after CT (2nd-order reconstructions, ideal / FASTEOS states)
+  static constexpr bool kWhole = !R5 && !MHD && EK == EK_IDEAL;
+  static constexpr bool kSwept = (SD == 3 || kWhole) && !R5 && EK != EK_HELM_FACE;
+  static int sweep(const Grid &g, int first, int last, int fin, double a1, double a2, double c3,
+                   hipStream_t st) {
     if constexpr (kSwept) {
-      const dim3 grd((unsigned)((g.n1 / kSweepT) * ((g.n2 + kSweepTy - 1) / kSweepTy)),
-                     (unsigned)((g.n3 + kSweepK - 1) / kSweepK), 1);
-      k_sweep<NAS, MHD, EK, MIX><<<grd, 256, 0, st>>>(g, first, fin, a1, a2, c3);
+      int kc;
+      const dim3 grd = sweep_grid(g, kc);
+      k_sweep<SD, NAS, MHD, EK, MIX, kWhole>
+          <<<grd, 256, 0, st>>>(g, first, last, fin, a1, a2, c3, kc);
+      return (int)(grd.x * grd.y);
     }
+    return 0;
   }
   static void update_swept(const Grid &g, int first, int last, double a1, double a2, double c3,
                            int fin, hipStream_t st) {
-    if constexpr (kSwept) {
-      const dim3 blk(64, 4, 1);
+    if constexpr (kSwept && !kWhole) {
+      const dim3 blk = cell_block(g);
       k_update<SD, NAS, MHD, HELM, MIX, false, true>
           <<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g, first, last, a1, a2, c3, fin);
     }
@@ -2190,32 +2292,32 @@ struct Kern {
   static void update_swept_guess(const Grid &g, int first, int last, double a1, double a2,
                                  double c3, int fin, hipStream_t st) {
     if constexpr (kSwept && HELM) {
-      const dim3 blk(64, 4, 1);
+      const dim3 blk = cell_block(g);
       k_update<SD, NAS, MHD, HELM, MIX, true, true>
           <<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g, first, last, a1, a2, c3, fin);
     }
   }
   static void cfl(const Grid &g, hipStream_t st) {
-    const dim3 blk(64, 4, 1);
+    const dim3 blk = cell_block(g);
     k_cfl<SD, MHD, HELM><<<grid_for(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g);
   }
   static void init(const Grid &g, int restart, hipStream_t st) {
-    const dim3 blk(64, 4, 1);
+    const dim3 blk = cell_block(g);
     k_init<SD, MHD, HELM><<<grid_for(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g, restart);
   }
   static void divb(const Grid &g, hipStream_t st) {
-    const dim3 blk(64, 4, 1);
+    const dim3 blk = cell_block(g);
     k_divb<SD><<<grid_for(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g);
   }
   static void prims(const Grid &g, hipStream_t st) {
     if constexpr (MIX) {
-      const dim3 blk(64, 4, 1);
+      const dim3 blk = cell_block(g);
       k_prim_from_u<SD, NAS, MHD, HELM><<<grid_for(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g);
     }
   }
   static void pack(const Grid &g, hipStream_t st) {
     if constexpr (MIX) {
-      const dim3 blk(64, 4, 1);
+      const dim3 blk = cell_block(g);
       k_pack_f<SD, NAS, MHD, HELM><<<grid_for(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g);
     }
   }
@@ -2242,7 +2344,7 @@ static KernelTable make_table() {
   t.prims = MIX ? &K::prims : nullptr;
   if constexpr (K::kSwept) {
     t.sweep = &K::sweep;
-    t.update_swept = &K::update_swept;
+    t.update_swept = K::kWhole ? nullptr : &K::update_swept;
     t.update_swept_guess = HELM ? &K::update_swept_guess : nullptr;
   }
   return t;
