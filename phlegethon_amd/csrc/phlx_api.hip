@@ -1043,6 +1043,8 @@ static int load_table(phlx_ctx *ctx, const double *f9, const double *c4, int32_t
   h.nt = nT;
   h.dt = (lthi - ltlo) / (double)(nT - 1);
   h.dr = (ldhi - ldlo) / (double)(nrho - 1);
+  h.idt = 1.0 / h.dt;
+  h.idr = 1.0 / h.dr;
   std::vector<double> nodes((size_t)nrho + nT);
   for (int i = 0; i < nrho; i++) nodes[i] = std::pow(10.0, ldlo + (double)i * h.dr);
   for (int j = 0; j < nT; j++) nodes[nrho + j] = std::pow(10.0, ltlo + (double)j * h.dt);

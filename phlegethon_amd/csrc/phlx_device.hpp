@@ -278,7 +278,7 @@ __device__ __forceinline__ void rec_lim2nd(double qm, double qc, double qp, doub
   // harmonic-mean limited slope, source/source.F90:8141-8181
   double sf = qp - qc, sb = qc - qm;
   double prod = sf * sb, slope = 0.0;
-  if (prod > 0.0) slope = prod / (sf + sb);
+  if (prod > 0.0) slope = Recip(sf + sb).div(prod);
   double h = 0.5 * slope;
   l = qc - h;
   r = qc + h;
@@ -418,7 +418,7 @@ __device__ __forceinline__ void face_helm(const Grid &g, const double *q, double
   double ye = 1.0, abar = 1.0;   // PIG_EOS without scalars ignores both
   if constexpr (NAS >= 2) {
     ye = q[IA];
-    abar = 1.0 / q[IA + 1];
+    abar = Recip(q[IA + 1]).inv();
   }
   const double zbar = ye * abar;
   double T = Tg, eint;
@@ -434,33 +434,33 @@ __device__ __forceinline__ void riemann_hydro(const Grid &g, const double *qL,
                                               const double *gR, double Tg, double *F,
                                               bool hll = false) {
   constexpr int IE = SD + 1, IA = SD + 2, NV = SD + 2 + NAS;
-  const double rhoL = qL[0], irL = 1.0 / rhoL;
+  const double rhoL = qL[0], irL = Recip(rhoL).inv();
   const double uL = qL[1], vL = qL[2], wL = (SD == 3) ? qL[3] : 0.0;
   const double v2L = uL * uL + vL * vL + wL * wL;
   const double pL = qL[IE];
   double eL, cL, eR, cR;
   if (EK == EK_FASTEOS) {
-    eL = pL / (gL[0] - 1.0);
-    cL = sqrt(gL[1] * pL * irL);
+    eL = Recip(gL[0] - 1.0).div(pL);
+    cL = dsqrt(gL[1] * pL * irL);
   } else if (EK == EK_HELM_FACE) {
     face_helm<SD, NAS>(g, qL, Tg, eL, cL);
   } else {
     eL = g.igmm1 * pL;
-    cL = sqrt(g.gm * pL * irL);
+    cL = dsqrt(g.gm * pL * irL);
   }
   const double EL = eL + 0.5 * rhoL * v2L;
-  const double rhoR = qR[0], irR = 1.0 / rhoR;
+  const double rhoR = qR[0], irR = Recip(rhoR).inv();
   const double uR = qR[1], vR = qR[2], wR = (SD == 3) ? qR[3] : 0.0;
   const double v2R = uR * uR + vR * vR + wR * wR;
   const double pR = qR[IE];
   if (EK == EK_FASTEOS) {
-    eR = pR / (gR[0] - 1.0);
-    cR = sqrt(gR[1] * pR * irR);
+    eR = Recip(gR[0] - 1.0).div(pR);
+    cR = dsqrt(gR[1] * pR * irR);
   } else if (EK == EK_HELM_FACE) {
     face_helm<SD, NAS>(g, qR, Tg, eR, cR);
   } else {
     eR = g.igmm1 * pR;
-    cR = sqrt(g.gm * pR * irR);
+    cR = dsqrt(g.gm * pR * irR);
   }
   const double ER = eR + 0.5 * rhoR * v2R;
   const double cmax = fmax(cL, cR);
@@ -489,21 +489,22 @@ __device__ __forceinline__ void riemann_hydro(const Grid &g, const double *qL,
       fL[v] = UL[v] * uL;
       fR[v] = UR[v] * uR;
     }
-    const double idn = 1.0 / (s1 - s0), ss = s0 * s1;
+    const double idn = Recip(s1 - s0).inv(), ss = s0 * s1;
 #pragma unroll
     for (int v = 0; v < NV; v++) F[v] = idn * (s1 * fL[v] - s0 * fR[v] + ss * (UR[v] - UL[v]));
     return;
   }
   const double dL = sL - uL, dR = sR - uR;
-  const double us = (pR - pL + rhoL * uL * dL - rhoR * uR * dR) / (rhoL * dL - rhoR * dR);
-  const double rsL = rhoL * (dL / (sL - us));
-  const double EsL = rsL * (EL * irL + (us - uL) * (us + pL * irL / dL));
-  const double rsR = rhoR * (dR / (sR - us));
-  const double EsR = rsR * (ER * irR + (us - uR) * (us + pR * irR / dR));
+  const double us =
+      Recip(rhoL * dL - rhoR * dR).div(pR - pL + rhoL * uL * dL - rhoR * uR * dR);
+  const double rsL = rhoL * Recip(sL - us).div(dL);
+  const double EsL = rsL * (EL * irL + (us - uL) * (us + Recip(dL).div(pL * irL)));
+  const double rsR = rhoR * Recip(sR - us).div(dR);
+  const double EsR = rsR * (ER * irR + (us - uR) * (us + Recip(dR).div(pR * irR)));
 
   if (g.flux == FLUX_LHLLC) {
     // low-dissipation pressure, source/source.F90:16014-16030
-    double chi = fmin(1.0, fmax(sqrt(v2L) / cL, sqrt(v2R) / cR));
+    double chi = fmin(1.0, fmax(Recip(cL).div(dsqrt(v2L)), Recip(cR).div(dsqrt(v2R))));
     chi = fmax(g.mach_cutoff, chi);
     const double phi = chi * (2.0 - chi);
     const double rbar = 0.5 * (rhoL + rhoR), cbar = 0.5 * (cL + cR);
@@ -582,13 +583,13 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
                                             const double *gR, double Tg, double *F,
                                             double *Fb, bool hll = false) {
   constexpr int IE = SD + 1, IA = SD + 2, NV = SD + 2 + NAS;
-  const double rhoL = qL[0], irL = 1.0 / rhoL;
+  const double rhoL = qL[0], irL = Recip(rhoL).inv();
   const double uL = qL[1], vL = qL[2], wL = (SD == 3) ? qL[3] : 0.0;
   const double v2L = uL * uL + vL * vL + wL * wL;
   const double pL = qL[IE];
   double e, c2L, c2R;
   if (EK == EK_FASTEOS) {
-    e = pL / (gL[0] - 1.0);
+    e = Recip(gL[0] - 1.0).div(pL);
     c2L = gL[1] * pL * irL;
   } else if (EK == EK_HELM_FACE) {
     double sound;
@@ -600,12 +601,12 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
   }
   double EL = e + 0.5 * rhoL * v2L;
   const double byL = bL[1], bzL = (SD == 3) ? bL[2] : 0.0;
-  const double rhoR = qR[0], irR = 1.0 / rhoR;
+  const double rhoR = qR[0], irR = Recip(rhoR).inv();
   const double uR = qR[1], vR = qR[2], wR = (SD == 3) ? qR[3] : 0.0;
   const double v2R = uR * uR + vR * vR + wR * wR;
   const double pR = qR[IE];
   if (EK == EK_FASTEOS) {
-    e = pR / (gR[0] - 1.0);
+    e = Recip(gR[0] - 1.0).div(pR);
     c2R = gR[1] * pR * irR;
   } else if (EK == EK_HELM_FACE) {
     double sound;
@@ -627,9 +628,9 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
   const double a2L = 2.0 * pbL * irL, a2R = 2.0 * pbR * irR;
   const double an2L = bx2 * irL, an2R = bx2 * irR;
   double t = c2L + a2L;
-  const double cL = sqrt(0.5 * (c2L + a2L + sqrt(t * t - 4.0 * c2L * an2L)));
+  const double cL = dsqrt(0.5 * (c2L + a2L + dsqrt(t * t - 4.0 * c2L * an2L)));
   t = c2R + a2R;
-  const double cR = sqrt(0.5 * (c2R + a2R + sqrt(t * t - 4.0 * c2R * an2R)));
+  const double cR = dsqrt(0.5 * (c2R + a2R + dsqrt(t * t - 4.0 * c2R * an2R)));
   const double cmax = fmax(cL, cR);
   const double sL = fmin(uL, uR) - cmax;
   const double sR = fmax(uL, uR) + cmax;
@@ -663,7 +664,7 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
     const double UbL[3] = {bx, byL, bzL}, UbR[3] = {bx, byR, bzR};
     const double fbL[3] = {0.0, uL * byL - vL * bx, uL * bzL - wL * bx};
     const double fbR[3] = {0.0, uR * byR - vR * bx, uR * bzR - wR * bx};
-    const double idn = 1.0 / (s1 - s0), ss = s0 * s1;
+    const double idn = Recip(s1 - s0).inv(), ss = s0 * s1;
 #pragma unroll
     for (int v = 0; v < NV; v++) F[v] = idn * (s1 * fL[v] - s0 * fR[v] + ss * (UR[v] - UL[v]));
 #pragma unroll
@@ -672,17 +673,17 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
     return;
   }
   const double dL = sL - uL, dR = sR - uR;
-  const double it1 = 1.0 / (dR * rhoR - dL * rhoL);
+  const double it1 = Recip(dR * rhoR - dL * rhoL).inv();
   const double us = (dR * rhoR * uR - dL * rhoL * uL - ptR + ptL) * it1;
   const double dmL = sL - us, dmR = sR - us;
   double phi = 1.0;
   if (g.flux == FLUX_LHLLD) {
     // source/source.F90:14364-14384
     t = v2L + a2L;
-    const double cu2L = 0.5 * (v2L + a2L + sqrt(t * t - 4.0 * v2L * an2L));
+    const double cu2L = 0.5 * (v2L + a2L + dsqrt(t * t - 4.0 * v2L * an2L));
     t = v2R + a2R;
-    const double cu2R = 0.5 * (v2R + a2R + sqrt(t * t - 4.0 * v2R * an2R));
-    const double mL = sqrt(cu2L) / cL, mR = sqrt(cu2R) / cR;
+    const double cu2R = 0.5 * (v2R + a2R + dsqrt(t * t - 4.0 * v2R * an2R));
+    const double mL = Recip(cL).div(dsqrt(cu2L)), mR = Recip(cR).div(dsqrt(cu2R));
     if (fmax(mL, mR) < 0.6) {
       double chi = fmin(1.0, fmax(mL, mR));
       chi = fmax(g.mach_cutoff, chi);
@@ -690,8 +691,9 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
     }
   }
   const double ps = (dR * rhoR * ptL - dL * rhoL * ptR - phi * rhoL * rhoR * dR * dL * (uL - uR)) * it1;
-  const double rsL = rhoL * dL / dmL;
-  const double rsR = rhoR * dR / dmR;
+  const Recip idmL(dmL), idmR(dmR);
+  const double rsL = idmL.div(rhoL * dL);
+  const double rsR = idmR.div(rhoR * dR);
   const double ia1 = 1.0 / (rhoL * dL * dmL - bx2);
   const double vsL = vL - bx * byL * (us - uL) * ia1;
   const double bysL = byL * (rhoL * dL * dL - bx2) * ia1;
@@ -706,13 +708,13 @@ __device__ __forceinline__ void riemann_mhd(const Grid &g, const double *qL,
   const double vbR = uR * bx + vR * byR + wR * bzR;
   const double vbsL = us * bx + vsL * bysL + wsL * bzsL;
   const double vbsR = us * bx + vsR * bysR + wsR * bzsR;
-  const double EsL = (dL * EL - ptL * uL + ps * us + bx * (vbL - vbsL)) / dmL;
-  const double EsR = (dR * ER - ptR * uR + ps * us + bx * (vbR - vbsR)) / dmR;
-  const double sqL = sqrt(rsL), sqR = sqrt(rsR);
+  const double EsL = idmL.div(dL * EL - ptL * uL + ps * us + bx * (vbL - vbsL));
+  const double EsR = idmR.div(dR * ER - ptR * uR + ps * us + bx * (vbR - vbsR));
+  const double sqL = dsqrt(rsL), sqR = dsqrt(rsR);
   const double abx = fabs(bx);
-  const double ssL = us - abx / sqL;
-  const double ssR = us + abx / sqR;
-  const double isq = 1.0 / (sqL + sqR);
+  const double ssL = us - Recip(sqL).div(abx);
+  const double ssR = us + Recip(sqR).div(abx);
+  const double isq = Recip(sqL + sqR).inv();
   const double sg = copysign(1.0, bx);
   const double vss = (sqL * vsL + sqR * vsR + (bysR - bysL) * sg) * isq;
   const double byss = (sqL * bysR + sqR * bysL + sqL * sqR * (vsR - vsL) * sg) * isq;

@@ -37,6 +37,7 @@ struct HelmDev {
   int nr, nt;
   double lrho1, lT1;  // log10 of the first nodes
   double dr, dt;      // log10 spacings
+  double idr, idt;    // their reciprocals (helm_index's estimate)
   double tl, th;      // Tl_eos, Th_eos (source/source.F90:750-751)
   // PIG_EOS table (pig_rhoT_given_*, source/source.F90:25457-26731): the free
   // energy of the whole gas at rho, i.e. Ye = 1 and no ion terms; the
@@ -55,11 +56,53 @@ struct HelmCell {
 // which holds every table value of the evaluation live at once.
 __device__ __forceinline__ void helm_pin(double &v) { asm volatile("" : "+v"(v)); }
 
+// Correctly rounded FP64 quotients of one denominator, the bits of a / b, in
+// fewer instructions than the compiler's expansion of it (v_div_scale twice,
+// reciprocal, four FMAs, product, remainder, v_div_fmas, v_div_fixup: 11 per
+// quotient, nothing shared).  The hardware reciprocal (relative error e <
+// 2^-24.4) is refined in one third-order step, r (1 + e + e^2), to half an ulp;
+// each quotient is the product with it corrected by its exact FMA remainder
+// (Markstein's theorem).  4 instructions and 3 per quotient (2 for 1 / b).
+// Without the scaling the remainder must stay a normal number: b normal and
+// finite, |a| in [2^-960, 2^960] or 0 and a / b in that range too.  No operand
+// of a physical state leaves it (b = 0 gives NaN where a / b is inf: the
+// callers' denominators are densities, speeds, cell widths, temperatures).
+// Checked bit for bit against a / b and 1 / b on 1.6e10 pairs with exponents
+// to +-480, mantissas next to all-ones and all-zeros among them.
+struct Recip {
+  double b, r;
+  __device__ __forceinline__ explicit Recip(double v) : b(v) {
+    const double r0 = __builtin_amdgcn_rcp(v);
+    const double e = fma(-v, r0, 1.0);
+    r = fma(r0, fma(e, e, e), r0);
+  }
+  __device__ __forceinline__ double div(double a) const {
+    const double q = a * r;
+    return fma(fma(-b, q, a), r, q);
+  }
+  __device__ __forceinline__ double inv() const { return fma(fma(-b, r, 1.0), r, r); }
+};
+// The correctly rounded square root, the bits of sqrt(x), for x = 0 or x in
+// [2^-960, 2^960] (NaN for x < 0): Goldschmidt's iteration from the hardware's
+// reciprocal root and two exact-remainder corrections, without the compiler's
+// rescaling and its tests of the ends of the range (13 instructions instead
+// of 19).  Checked on the same sample.
+__device__ __forceinline__ double dsqrt(double x) {
+  const double y = __builtin_amdgcn_rsq(x);
+  double s = x * y, h = 0.5 * y;
+  const double r = fma(-h, s, 0.5);
+  s = fma(s, r, s);
+  h = fma(h, r, h);
+  s = fma(fma(-s, s, x), h, s);
+  s = fma(fma(-s, s, x), h, s);
+  return x == 0.0 ? x : s;
+}
+
 // a / b; FAST (the mixed-precision EoS step only): the hardware reciprocal
-// refined by two Newton steps (~1 ulp) instead of the IEEE-rounded sequence.
+// refined by two Newton steps (~1 ulp) instead of the correctly rounded form.
 template <bool FAST>
 __device__ __forceinline__ double hdiv(double a, double b) {
-  if (!FAST) return a / b;
+  if (!FAST) return Recip(b).div(a);
   double r = __builtin_amdgcn_rcp(b);
   double e = fma(-b, r, 1.0);
   r = fma(r, e, r);
@@ -74,12 +117,28 @@ struct HelmBasis {
   double a[3], am[3];
 };
 
-// cell index int((log10(rhoYe) - log10(rho_1)) / dlog) (source/source.F90
-// :23773-23784), kept inside the table.  FAST (the mixed-precision EoS step
-// only): the index from the FP32 base-2 logarithm (v_log_f32) instead of two
-// FP64 log10; within ~1e-5 of a node it may pick the neighbouring cell, whose
-// quintic Hermite interpolant matches value, slope and curvature there, and
-// the offsets x, y are still formed in FP64 from the table's nodes.
+// Cell index int((log10(x) - l1) / d) (source/source.F90:23773-23784), kept
+// inside the table of n nodes.  The index only needs the logarithm to less than
+// its distance from the next node: the base-2 logarithm as the exact exponent
+// plus v_log_f32 of the mantissa is good to 6e-8 in log10, and only a lane
+// within 5e-7 of a node takes the FP64 log10 and its quotient (~100
+// instructions).  Both give the same index elsewhere, so the result is that of
+// the FP64 form bit for bit (a NaN, an infinity, x <= 0 take it too).
+__device__ __forceinline__ int helm_index(double x, double l1, double d, double id, int n) {
+  constexpr double kLog10of2 = 0.301029995663981195;
+  const double lg = (double)__builtin_amdgcn_frexp_exp(x) +
+                    (double)__builtin_amdgcn_logf((float)__builtin_amdgcn_frexp_mant(x));
+  const double t = (lg * kLog10of2 - l1) * id, fl = __builtin_floor(t), fr = t - fl;
+  const double tol = 5e-7 * id;
+  int i = (int)fl;
+  if (!(fr > tol && fr < 1.0 - tol)) i = (int)((log10(x) - l1) / d);
+  return i < 0 ? 0 : (i > n - 2 ? n - 2 : i);
+}
+
+// FAST (the mixed-precision EoS step only): the index from the FP32 base-2
+// logarithm (v_log_f32); within ~1e-5 of a node it may pick the neighbouring
+// cell, whose quintic Hermite interpolant matches value, slope and curvature
+// there, and the offsets x, y are still formed in FP64 from the table's nodes.
 template <bool FAST = false>
 __device__ __forceinline__ HelmCell helm_locate(const HelmDev &h, double rhos, double T) {
   HelmCell c;
@@ -89,12 +148,12 @@ __device__ __forceinline__ HelmCell helm_locate(const HelmDev &h, double rhos, d
     const float lt = __builtin_amdgcn_logf((float)T) * kLog10of2;
     c.ih = (int)((lr - (float)h.lrho1) * __builtin_amdgcn_rcpf((float)h.dr));
     c.jh = (int)((lt - (float)h.lT1) * __builtin_amdgcn_rcpf((float)h.dt));
+    c.ih = c.ih < 0 ? 0 : (c.ih > h.nr - 2 ? h.nr - 2 : c.ih);
+    c.jh = c.jh < 0 ? 0 : (c.jh > h.nt - 2 ? h.nt - 2 : c.jh);
   } else {
-    c.ih = (int)((log10(rhos) - h.lrho1) / h.dr);
-    c.jh = (int)((log10(T) - h.lT1) / h.dt);
+    c.ih = helm_index(rhos, h.lrho1, h.dr, h.idr, h.nr);
+    c.jh = helm_index(T, h.lT1, h.dt, h.idt, h.nt);
   }
-  c.ih = c.ih < 0 ? 0 : (c.ih > h.nr - 2 ? h.nr - 2 : c.ih);
-  c.jh = c.jh < 0 ? 0 : (c.jh > h.nt - 2 ? h.nt - 2 : c.jh);
   double tmp = h.rho[c.ih];
   c.drho = h.rho[c.ih + 1] - tmp;
   c.x = hdiv<FAST>(rhos - tmp, c.drho);
@@ -119,9 +178,8 @@ __device__ __forceinline__ void helm_basis(double x, double d, HelmBasis &v) {
   v.am[2] = (0.5 * (-o5 + 3.0 * o4 - 3.0 * o3 + o2)) * d2;
 }
 
-template <bool FAST = false>
-__device__ __forceinline__ void helm_dbasis(double x, double d, HelmBasis &v) {
-  const double id = hdiv<FAST>(1.0, d);
+// id = 1 / d
+__device__ __forceinline__ void helm_dbasis(double x, double d, double id, HelmBasis &v) {
   const double x2 = x * x, x3 = x2 * x, x4 = x3 * x;
   const double o = 1.0 - x;
   const double o2 = o * o, o3 = o2 * o, o4 = o3 * o;
@@ -133,9 +191,8 @@ __device__ __forceinline__ void helm_dbasis(double x, double d, HelmBasis &v) {
   v.am[2] = -(0.5 * (-5.0 * o4 + 12.0 * o3 - 9.0 * o2 + 2.0 * o)) * d;
 }
 
-template <bool FAST = false>
-__device__ __forceinline__ void helm_ddbasis(double x, double d, HelmBasis &v) {
-  const double id = hdiv<FAST>(1.0, d), id2 = id * id;
+__device__ __forceinline__ void helm_ddbasis(double x, double d, double id, HelmBasis &v) {
+  const double id2 = id * id;
   const double x2 = x * x, x3 = x2 * x;
   const double o = 1.0 - x;
   const double o2 = o * o, o3 = o2 * o;
@@ -147,18 +204,17 @@ __device__ __forceinline__ void helm_ddbasis(double x, double d, HelmBasis &v) {
   v.am[2] = (0.5 * (-20.0 * o3 + 36.0 * o2 - 18.0 * o + 2.0));
 }
 
+// rho and T orders of the nine entries
+constexpr int kHelmRX[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2};
+constexpr int kHelmTY[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
+
 // NS biquintic sums over the cell in ONE pass over the table: sum k pairs
 // the rho basis R[k] with the T basis T[k].  Each sum keeps the reference's
-// term order: entry v pairs the rho basis of order (0,0,0,1,2,1,2,1,2)[v]
-// with the T basis of order (0,1,2,0,0,1,1,2,2)[v]; per entry the corners
-// (i,j) (i+1,j) (i,j+1) (i+1,j+1) are added in that order.  Reading each
-// table value once for all sums keeps ~4 values in flight per lane instead
-// of the whole 36-value block per sum.
-// FMA (the mixed-precision EoS step only): the basis products are formed
-// once per entry and the four corner terms accumulated with fused
-// multiply-adds (8 instead of 12 operations per entry and sum); the FP64
-// path keeps the reference's unfused order.
-template <int NS, bool FMA = false>
+// term order: entry v pairs the rho basis of order kHelmRX[v] with the T basis
+// of order kHelmTY[v]; per entry the corners (i,j) (i+1,j) (i,j+1) (i+1,j+1)
+// are added in that order.  Reading each table value once for all sums keeps
+// ~4 values in flight per lane instead of the whole 36-value block per sum.
+template <int NS>
 __device__ __forceinline__ void helm_sums36(const HelmDev &h, const HelmCell &c,
                                             const HelmBasis *const (&R)[NS],
                                             const HelmBasis *const (&T)[NS], double (&s)[NS]) {
@@ -166,29 +222,63 @@ __device__ __forceinline__ void helm_sums36(const HelmDev &h, const HelmCell &c,
   const double *n10 = n00 + kHelmRec;
   const double *n01 = n00 + (size_t)kHelmRec * h.nr;
   const double *n11 = n01 + kHelmRec;
-  constexpr int RX[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2};
-  constexpr int TY[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
 #pragma unroll
   for (int v = 0; v < 9; v++) {
     const double q0 = n00[v], q1 = n10[v], q2 = n01[v], q3 = n11[v];
 #pragma unroll
     for (int k = 0; k < NS; k++) {
-      const double a = R[k]->a[RX[v]], am = R[k]->am[RX[v]];
-      const double b = T[k]->a[TY[v]], bm = T[k]->am[TY[v]];
-      if (FMA) {
-        const double ab = a * b, amb = am * b, abm = a * bm, ambm = am * bm;
-        s[k] = (v == 0) ? q0 * ab : fma(q0, ab, s[k]);
-        s[k] = fma(q1, amb, s[k]);
-        s[k] = fma(q2, abm, s[k]);
-        s[k] = fma(q3, ambm, s[k]);
-      } else {
-        const double t0 = q0 * a * b, t1 = q1 * am * b;
-        const double t2 = q2 * a * bm, t3 = q3 * am * bm;
-        s[k] = (v == 0) ? t0 : s[k] + t0;
-        s[k] = s[k] + t1;
-        s[k] = s[k] + t2;
-        s[k] = s[k] + t3;
-      }
+      const double a = R[k]->a[kHelmRX[v]], am = R[k]->am[kHelmRX[v]];
+      const double b = T[k]->a[kHelmTY[v]], bm = T[k]->am[kHelmTY[v]];
+      const double t0 = q0 * a * b, t1 = q1 * am * b;
+      const double t2 = q2 * a * bm, t3 = q3 * am * bm;
+      s[k] = (v == 0) ? t0 : s[k] + t0;
+      s[k] = s[k] + t1;
+      s[k] = s[k] + t2;
+      s[k] = s[k] + t3;
+    }
+  }
+}
+
+// The first products of those terms, table value times rho basis, for the 9 x
+// 4 values of one cell, kept in registers over a Newton solve: rho does not
+// move in it, its iterates mostly share the cell, and a lane reads the records
+// again only when its T leaves it.  Points in no particular order (the batch
+// calls) put every lane on lines of its own, and a load instruction then takes
+// the L1 one lane a cycle: with 20-28 of them per evaluation the loads, not
+// the arithmetic, were the time (10^6 points, T(rho, e) from 5 % off: 262 us).
+struct HelmTab {
+  double q[9][4];
+  int jh = -1;
+};
+__device__ __forceinline__ void helm_tab_load(const HelmDev &h, const HelmCell &c,
+                                              const HelmBasis &R, HelmTab &tab) {
+  tab.jh = c.jh;
+  const double *n00 = h.tab + (size_t)kHelmRec * ((size_t)c.jh * h.nr + c.ih);
+  const double *n01 = n00 + (size_t)kHelmRec * h.nr;
+#pragma unroll
+  for (int v = 0; v < 9; v++) {
+    const double a = R.a[kHelmRX[v]], am = R.am[kHelmRX[v]];
+    tab.q[v][0] = n00[v] * a;
+    tab.q[v][1] = n00[kHelmRec + v] * am;
+    tab.q[v][2] = n01[v] * a;
+    tab.q[v][3] = n01[kHelmRec + v] * am;
+  }
+}
+// helm_sums36 of one rho basis from its products
+template <int NS>
+__device__ __forceinline__ void helm_sums_T(const HelmTab &tab, const HelmBasis *const (&T)[NS],
+                                            double (&s)[NS]) {
+#pragma unroll
+  for (int v = 0; v < 9; v++) {
+#pragma unroll
+    for (int k = 0; k < NS; k++) {
+      const double b = T[k]->a[kHelmTY[v]], bm = T[k]->am[kHelmTY[v]];
+      const double t0 = tab.q[v][0] * b, t1 = tab.q[v][1] * b;
+      const double t2 = tab.q[v][2] * bm, t3 = tab.q[v][3] * bm;
+      s[k] = (v == 0) ? t0 : s[k] + t0;
+      s[k] = s[k] + t1;
+      s[k] = s[k] + t2;
+      s[k] = s[k] + t3;
     }
   }
 }
@@ -208,15 +298,13 @@ __device__ __forceinline__ void helm_contract_rho(const HelmDev &h, const HelmCe
   const double *n10 = n00 + kHelmRec;
   const double *n01 = n00 + (size_t)kHelmRec * h.nr;
   const double *n11 = n01 + kHelmRec;
-  constexpr int RX[9] = {0, 0, 0, 1, 2, 1, 2, 1, 2};
-  constexpr int TY[9] = {0, 1, 2, 0, 0, 1, 1, 2, 2};
 #pragma unroll
   for (int v = 0; v < 9; v++) {
     const double q0 = n00[v], q1 = n10[v], q2 = n01[v], q3 = n11[v];
-    const int lo = 2 * TY[v], hi = lo + 1;
+    const int lo = 2 * kHelmTY[v], hi = lo + 1;
 #pragma unroll
     for (int k = 0; k < NR; k++) {
-      const double a = R[k]->a[RX[v]], am = R[k]->am[RX[v]];
+      const double a = R[k]->a[kHelmRX[v]], am = R[k]->am[kHelmRX[v]];
       // entries 0..2 (rho order 0) are the first of their T order
       G[k][lo] = (v < 3) ? q0 * a : fma(q0, a, G[k][lo]);
       G[k][lo] = fma(q1, am, G[k][lo]);
@@ -276,36 +364,30 @@ __device__ __forceinline__ double helm_sum16(const HelmDev &h, const HelmCell &c
 }
 
 // helm_rhoT_given_full: P, E (specific), sound speed (relativistic form), c_v;
-// dPdT (when non-null) receives dP/dT.  FMA: fused table sums (mixed path).
-template <bool FMA = false>
-__device__ __forceinline__ void helm_full(const HelmDev &h, double rho, double T, double abar,
-                                          double zbar, double &P, double &E, double &sound,
-                                          double &cv, double *dPdT_out = nullptr) {
-  const double Ye = h.pig ? 1.0 : hdiv<FMA>(zbar, abar), rhos = rho * Ye;
-  const HelmCell c = helm_locate<FMA>(h, rhos, T);
+// dPdT (when non-null) receives dP/dT.  With the fused table sums and refined
+// reciprocals of the mixed path (helm_rhoe_lin).
+__device__ __forceinline__ void helm_full_fma(const HelmDev &h, double rho, double T, double abar,
+                                              double zbar, double &P, double &E, double &sound,
+                                              double &cv, double *dPdT_out) {
+  const double Ye = h.pig ? 1.0 : hdiv<true>(zbar, abar), rhos = rho * Ye;
+  const HelmCell c = helm_locate<true>(h, rhos, T);
   HelmBasis r, dr, t, dt, ddt;
   helm_basis(c.x, c.drho, r);
-  helm_dbasis<FMA>(c.x, c.drho, dr);
+  helm_dbasis(c.x, c.drho, hdiv<true>(1.0, c.drho), dr);
   helm_basis(c.y, c.dT, t);
-  helm_dbasis<FMA>(c.y, c.dT, dt);
-  helm_ddbasis<FMA>(c.y, c.dT, ddt);
-  double sm[5];
-  if constexpr (FMA) {
-    const HelmBasis *const RR[2] = {&r, &dr};
-    double G[2][6];
-    helm_contract_rho<2>(h, c, RR, G);
-    sm[0] = helm_contract_T(G[0], t);
-    sm[1] = helm_contract_T(G[1], t);
-    sm[2] = helm_contract_T(G[0], dt);
-    sm[3] = helm_contract_T(G[1], dt);
-    sm[4] = helm_contract_T(G[0], ddt);
-  } else {
-    const HelmBasis *const RR[5] = {&r, &dr, &r, &dr, &r};
-    const HelmBasis *const TT[5] = {&t, &t, &dt, &dt, &ddt};
-    helm_sums36<5, FMA>(h, c, RR, TT, sm);
-  }
+  const double idT = hdiv<true>(1.0, c.dT);
+  helm_dbasis(c.y, c.dT, idT, dt);
+  helm_ddbasis(c.y, c.dT, idT, ddt);
+  const HelmBasis *const RR[2] = {&r, &dr};
+  double G[2][6], sm[5];
+  helm_contract_rho<2>(h, c, RR, G);
+  sm[0] = helm_contract_T(G[0], t);
+  sm[1] = helm_contract_T(G[1], t);
+  sm[2] = helm_contract_T(G[0], dt);
+  sm[3] = helm_contract_T(G[1], dt);
+  sm[4] = helm_contract_T(G[0], ddt);
   const double f = sm[0], df_drho = sm[1], df_dT = sm[2], df_drhodT = sm[3], df_dT2 = sm[4];
-  double dP_drho = helm_sum16<FMA>(h, c);
+  double dP_drho = helm_sum16<true>(h, c);
   dP_drho = Ye * dP_drho;
   double tmp = rhos * rhos;
   double p = tmp * df_drho;
@@ -314,7 +396,7 @@ __device__ __forceinline__ void helm_full(const HelmDev &h, double rho, double T
   const double ds_dT = -Ye * df_dT2;
   double e = Ye * f + T * s;
   double dE_dT = T * ds_dT;
-  tmp = h.pig ? 0.0 : hdiv<FMA>(1.0, abar);
+  tmp = h.pig ? 0.0 : hdiv<true>(1.0, abar);
   const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
   const double pion = kHelmRgas * rho * T * tmp;
   const double dpiondt = kHelmRgas * rho * tmp;
@@ -322,18 +404,18 @@ __device__ __forceinline__ void helm_full(const HelmDev &h, double rho, double T
   p = p + pion + kHelmCrad * T4 * (1.0 / 3.0);
   dP_dT = dP_dT + dpiondt + (4.0 / 3.0) * kHelmCrad * T3;
   dP_drho = dP_drho + dpiondd;
-  e = e + 1.5 * kHelmRgas * T * tmp + hdiv<FMA>(kHelmCrad * T4, rho);
-  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv<FMA>(4.0 * kHelmCrad * T3, rho);
-  const double zz = hdiv<FMA>(p, rho);
-  const double chiT = hdiv<FMA>(T, p) * dP_dT;
-  const double chirho = hdiv<FMA>(dP_drho, zz);
-  const double x = hdiv<FMA>(zz * chiT, T * dE_dT);
+  e = e + 1.5 * kHelmRgas * T * tmp + hdiv<true>(kHelmCrad * T4, rho);
+  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv<true>(4.0 * kHelmCrad * T3, rho);
+  const double zz = hdiv<true>(p, rho);
+  const double chiT = hdiv<true>(T, p) * dP_dT;
+  const double chirho = hdiv<true>(dP_drho, zz);
+  const double x = hdiv<true>(zz * chiT, T * dE_dT);
   const double gam1 = chiT * x + chirho;
-  const double z = 1.0 + hdiv<FMA>(e + kHelmClight2, zz);
+  const double z = 1.0 + hdiv<true>(e + kHelmClight2, zz);
   P = p;
   E = e;
   cv = dE_dT;
-  sound = kHelmClight * sqrt(hdiv<FMA>(gam1, z));
+  sound = kHelmClight * sqrt(hdiv<true>(gam1, z));
   if (dPdT_out) *dPdT_out = dP_dT;
 }
 
@@ -365,7 +447,7 @@ __device__ __forceinline__ void helm_mx_contract(const HelmDev &h, double T, Hel
   m.Tj = h.T[c.jh];
   HelmBasis r, dr;
   helm_basis(c.x, c.drho, r);
-  helm_dbasis<true>(c.x, c.drho, dr);
+  helm_dbasis(c.x, c.drho, hdiv<true>(1.0, c.drho), dr);
   {
     const HelmBasis *const RR[2] = {&r, &dr};
     double G[2][6];
@@ -426,8 +508,9 @@ __device__ __forceinline__ void helm_mx_energy(const HelmDev &h, HelmMx &m, doub
   a.y = y;
   HelmBasis ddt;
   helm_basis(y, m.dT, a.t);
-  helm_dbasis<true>(y, m.dT, a.dt);
-  helm_ddbasis<true>(y, m.dT, ddt);
+  const double idT = hdiv<true>(1.0, m.dT);
+  helm_dbasis(y, m.dT, idT, a.dt);
+  helm_ddbasis(y, m.dT, idT, ddt);
   const double f = helm_contract_T(m.Gr, a.t);
   const double df_dT = helm_contract_T(m.Gr, a.dt);
   const double df_dT2 = helm_contract_T(m.Gr, ddt);
@@ -476,77 +559,171 @@ __device__ __forceinline__ void helm_mx_pressure(const HelmMx &m, double rho, do
   sound = kHelmClight * sqrt(hdiv<true>(gam1, z));
 }
 
-// helm_rhoT_given1: P and (when ret) dP/dT.
-__device__ __forceinline__ void helm_given1(const HelmDev &h, double rho, double T, double abar,
-                                            double zbar, double &P, double &dPdT, bool ret) {
-  const double Ye = h.pig ? 1.0 : zbar / abar, rhos = rho * Ye;
-  const HelmCell c = helm_locate(h, rhos, T);
-  HelmBasis dr, t, dt;
-  helm_dbasis(c.x, c.drho, dr);
+// ---------------------------------------------------------------------------
+// The FP64 evaluations.  Everything that depends on rho, Ye and abar alone is
+// formed once per solve (HelmRho) and shared by the Newton iterates and the
+// closing evaluation; the reference forms it again in each call, with the same
+// operands, so the bits are the same.
+struct HelmRho {
+  double rho, Ye, rhos, iabar;  // iabar = 1/abar (PIG: 0)
+  int ih;
+  double x, drho, idrho;
+  Recip rrho;
+  __device__ __forceinline__ HelmRho(const HelmDev &h, double rho_, double abar, double zbar)
+      : rho(rho_), rrho(rho_) {
+    Ye = 1.0;
+    iabar = 0.0;
+    if (!h.pig) {
+      const Recip ra(abar);
+      Ye = ra.div(zbar);
+      iabar = ra.inv();
+    }
+    rhos = rho * Ye;
+    ih = helm_index(rhos, h.lrho1, h.dr, h.idr, h.nr);
+    const double lo = h.rho[ih];
+    drho = h.rho[ih + 1] - lo;
+    const Recip rd(drho);
+    x = rd.div(rhos - lo);
+    idrho = rd.inv();
+  }
+};
+
+// The cell of an evaluation at T and 1 / dT.
+__device__ __forceinline__ HelmCell helm_cell(const HelmDev &h, const HelmRho &m, double T,
+                                              double &idT) {
+  HelmCell c;
+  c.ih = m.ih;
+  c.x = m.x;
+  c.drho = m.drho;
+  c.jh = helm_index(T, h.lT1, h.dt, h.idt, h.nt);
+  const double lo = h.T[c.jh];
+  c.dT = h.T[c.jh + 1] - lo;
+  const Recip rd(c.dT);
+  c.y = rd.div(T - lo);
+  idT = rd.inv();
+  return c;
+}
+
+// helm_rhoT_given_full: P, E (specific), sound speed (relativistic form), c_v.
+__device__ __forceinline__ void helm_full_at(const HelmDev &h, const HelmRho &m, double T,
+                                             double &P, double &E, double &sound, double &cv) {
+  const double rho = m.rho, Ye = m.Ye, rhos = m.rhos, iabar = m.iabar;
+  double idT;
+  const HelmCell c = helm_cell(h, m, T, idT);
+  HelmBasis r, dr, t, dt, ddt;
+  helm_basis(c.x, c.drho, r);
+  helm_dbasis(c.x, c.drho, m.idrho, dr);
+  helm_basis(c.y, c.dT, t);
+  helm_dbasis(c.y, c.dT, idT, dt);
+  helm_ddbasis(c.y, c.dT, idT, ddt);
+  const HelmBasis *const RR[5] = {&r, &dr, &r, &dr, &r};
+  const HelmBasis *const TT[5] = {&t, &t, &dt, &dt, &ddt};
+  double sm[5];
+  helm_sums36<5>(h, c, RR, TT, sm);
+  const double f = sm[0], df_drho = sm[1], df_dT = sm[2], df_drhodT = sm[3], df_dT2 = sm[4];
+  double dP_drho = helm_sum16(h, c);
+  dP_drho = Ye * dP_drho;
+  const double rr = rhos * rhos;
+  double p = rr * df_drho;
+  double dP_dT = rr * df_drhodT;
+  const double s = -Ye * df_dT;
+  const double ds_dT = -Ye * df_dT2;
+  double e = Ye * f + T * s;
+  double dE_dT = T * ds_dT;
+  const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
+  const double pion = kHelmRgas * rho * T * iabar;
+  const double dpiondt = kHelmRgas * rho * iabar;
+  const double dpiondd = kHelmRgas * T * iabar;
+  p = p + pion + kHelmCrad * T4 * (1.0 / 3.0);
+  dP_dT = dP_dT + dpiondt + (4.0 / 3.0) * kHelmCrad * T3;
+  dP_drho = dP_drho + dpiondd;
+  e = e + 1.5 * kHelmRgas * T * iabar + m.rrho.div(kHelmCrad * T4);
+  dE_dT = dE_dT + 1.5 * kHelmRgas * iabar + m.rrho.div(4.0 * kHelmCrad * T3);
+  const double zz = m.rrho.div(p);
+  const double chiT = Recip(p).div(T) * dP_dT;
+  const Recip rz(zz);
+  const double chirho = rz.div(dP_drho);
+  const double x = Recip(T * dE_dT).div(zz * chiT);
+  const double gam1 = chiT * x + chirho;
+  const double z = 1.0 + rz.div(e + kHelmClight2);
+  P = p;
+  E = e;
+  cv = dE_dT;
+  sound = kHelmClight * dsqrt(Recip(z).div(gam1));
+}
+__device__ __forceinline__ void helm_full(const HelmDev &h, double rho, double T, double abar,
+                                          double zbar, double &P, double &E, double &sound,
+                                          double &cv) {
+  helm_full_at(h, HelmRho(h, rho, abar, zbar), T, P, E, sound, cv);
+}
+
+// helm_rhoT_given1: P and (when ret) dP/dT.  tab: the products of dr/d(rho Ye)'s
+// basis (a solve's own, empty at its start).
+__device__ __forceinline__ void helm_given1(const HelmDev &h, const HelmRho &m, HelmTab &tab,
+                                            double T, double &P, double &dPdT, bool ret) {
+  const double rho = m.rho, rhos = m.rhos;
+  double idT;
+  const HelmCell c = helm_cell(h, m, T, idT);
+  if (tab.jh != c.jh) {
+    HelmBasis dr;
+    helm_dbasis(c.x, c.drho, m.idrho, dr);
+    helm_tab_load(h, c, dr, tab);
+  }
+  HelmBasis t, dt;
   helm_basis(c.y, c.dT, t);
   double df_drho, df_drhodT = 0.0;
   if (ret) {
-    helm_dbasis(c.y, c.dT, dt);
-    const HelmBasis *const RR[2] = {&dr, &dr};
+    helm_dbasis(c.y, c.dT, idT, dt);
     const HelmBasis *const TT[2] = {&t, &dt};
     double sm[2];
-    helm_sums36<2>(h, c, RR, TT, sm);
+    helm_sums_T<2>(tab, TT, sm);
     df_drho = sm[0];
     df_drhodT = sm[1];
   } else {
-    const HelmBasis *const RR[1] = {&dr};
     const HelmBasis *const TT[1] = {&t};
     double sm[1];
-    helm_sums36<1>(h, c, RR, TT, sm);
+    helm_sums_T<1>(tab, TT, sm);
     df_drho = sm[0];
   }
-  double tmp = rhos * rhos;
-  double p = tmp * df_drho;
-  double dP_dT = tmp * df_drhodT;
+  const double rr = rhos * rhos;
+  double p = rr * df_drho;
+  double dP_dT = rr * df_drhodT;
   const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
-  tmp = h.pig ? 0.0 : 1.0 / abar;
-  const double pion = kHelmRgas * rho * T * tmp;
-  const double dpiondt = kHelmRgas * rho * tmp;
+  const double pion = kHelmRgas * rho * T * m.iabar;
+  const double dpiondt = kHelmRgas * rho * m.iabar;
   p = p + pion + kHelmCrad * T4 * (1.0 / 3.0);
   dP_dT = dP_dT + dpiondt + (4.0 / 3.0) * kHelmCrad * T3;
   P = p;
   dPdT = dP_dT;
 }
 
-// helm_rhoT_given2: E and (when ret) dE/dT.  FMA (the mixed-precision EoS
-// only): the separable contraction, refined reciprocals, FP32 cell lookup.
-template <bool FMA = false>
-__device__ __forceinline__ void helm_given2(const HelmDev &h, double rho, double T, double abar,
-                                            double zbar, double &E, double &dEdT, bool ret) {
-  const double Ye = h.pig ? 1.0 : hdiv<FMA>(zbar, abar), rhos = rho * Ye;
-  const HelmCell c = helm_locate<FMA>(h, rhos, T);
-  HelmBasis r, t, dt, ddt;
-  helm_basis(c.x, c.drho, r);
+// helm_rhoT_given2: E and (when ret) dE/dT.  tab: the products of the rho basis.
+__device__ __forceinline__ void helm_given2(const HelmDev &h, const HelmRho &m, HelmTab &tab,
+                                            double T, double &E, double &dEdT, bool ret) {
+  const double Ye = m.Ye, iabar = m.iabar;
+  double idT;
+  const HelmCell c = helm_cell(h, m, T, idT);
+  if (tab.jh != c.jh) {
+    HelmBasis r;
+    helm_basis(c.x, c.drho, r);
+    helm_tab_load(h, c, r, tab);
+  }
+  HelmBasis t, dt, ddt;
   helm_basis(c.y, c.dT, t);
-  helm_dbasis<FMA>(c.y, c.dT, dt);
+  helm_dbasis(c.y, c.dT, idT, dt);
   double f, df_dT, df_dT2 = 0.0;
-  if (FMA) {
-    helm_ddbasis<FMA>(c.y, c.dT, ddt);
-    const HelmBasis *const RR[1] = {&r};
-    double G[1][6];
-    helm_contract_rho<1>(h, c, RR, G);
-    f = helm_contract_T(G[0], t);
-    df_dT = helm_contract_T(G[0], dt);
-    df_dT2 = helm_contract_T(G[0], ddt);
-  } else if (ret) {
-    helm_ddbasis(c.y, c.dT, ddt);
-    const HelmBasis *const RR[3] = {&r, &r, &r};
+  if (ret) {
+    helm_ddbasis(c.y, c.dT, idT, ddt);
     const HelmBasis *const TT[3] = {&t, &dt, &ddt};
     double sm[3];
-    helm_sums36<3>(h, c, RR, TT, sm);
+    helm_sums_T<3>(tab, TT, sm);
     f = sm[0];
     df_dT = sm[1];
     df_dT2 = sm[2];
   } else {
-    const HelmBasis *const RR[2] = {&r, &r};
     const HelmBasis *const TT[2] = {&t, &dt};
     double sm[2];
-    helm_sums36<2>(h, c, RR, TT, sm);
+    helm_sums_T<2>(tab, TT, sm);
     f = sm[0];
     df_dT = sm[1];
   }
@@ -555,9 +732,8 @@ __device__ __forceinline__ void helm_given2(const HelmDev &h, double rho, double
   double e = Ye * f + T * s;
   double dE_dT = T * ds_dT;
   const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
-  const double tmp = h.pig ? 0.0 : hdiv<FMA>(1.0, abar);
-  e = e + 1.5 * kHelmRgas * T * tmp + hdiv<FMA>(kHelmCrad * T4, rho);
-  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv<FMA>(4.0 * kHelmCrad * T3, rho);
+  e = e + 1.5 * kHelmRgas * T * iabar + m.rrho.div(kHelmCrad * T4);
+  dE_dT = dE_dT + 1.5 * kHelmRgas * iabar + m.rrho.div(4.0 * kHelmCrad * T3);
   E = e;
   dEdT = dE_dT;
 }
@@ -567,21 +743,29 @@ __device__ __forceinline__ void helm_given2(const HelmDev &h, double rho, double
 // one Newton step past the converged one; a T outside [Tl, Th] resets to the
 // start value and ends the loop.  Returns the iterations taken (<= 100).
 // cv_last (optional): dE/dT of the last Newton evaluation (the energy
-// predictor's slope for the next solve of the zone).
-__device__ __forceinline__ int helm_rhoe_given(const HelmDev &h, double rho, double E0,
-                                               double abar, double zbar, double &T, double &P,
-                                               double &sound, bool ret,
-                                               double *cv_last = nullptr) {
+// predictor's slope for the next solve of the zone).  start (optional): E and
+// dE/dT at the incoming T, where the caller has them already.
+__device__ __forceinline__ int helm_rhoe_given(const HelmDev &h, const HelmRho &m, HelmTab &tab,
+                                               double E0, double &T, double &P, double &sound,
+                                               bool ret,
+                                               double *cv_last = nullptr,
+                                               const double *start = nullptr) {
   const double Told = T;
+  const Recip rE0(E0);
   int iter;
   sound = 0.0;
   for (iter = 1; iter <= kHelmMaxIter; iter++) {
     double e, dEdT;
-    helm_given2(h, rho, T, abar, zbar, e, dEdT, true);
+    if (start && iter == 1) {
+      e = start[0];
+      dEdT = start[1];
+    } else {
+      helm_given2(h, m, tab, T, e, dEdT, true);
+    }
     if (cv_last) *cv_last = dEdT;
     const double res = e - E0;
-    T = T - res / dEdT;
-    double err = fabs(res / E0);
+    T = T - Recip(dEdT).div(res);
+    double err = fabs(rE0.div(res));
     if ((T < h.tl) || (T > h.th)) {
       T = Told;
       err = 1e-15;
@@ -590,27 +774,38 @@ __device__ __forceinline__ int helm_rhoe_given(const HelmDev &h, double rho, dou
   }
   if (ret) {
     double e, cv;
-    helm_full(h, rho, T, abar, zbar, P, e, sound, cv);
+    helm_full_at(h, m, T, P, e, sound, cv);
   } else {
     double dPdT;
-    helm_given1(h, rho, T, abar, zbar, P, dPdT, false);
+    HelmTab tp;
+    helm_given1(h, m, tp, T, P, dPdT, false);
   }
   return iter > kHelmMaxIter ? kHelmMaxIter : iter;
+}
+__device__ __forceinline__ int helm_rhoe_given(const HelmDev &h, double rho, double E0,
+                                               double abar, double zbar, double &T, double &P,
+                                               double &sound, bool ret,
+                                               double *cv_last = nullptr) {
+  HelmTab tab;
+  return helm_rhoe_given(h, HelmRho(h, rho, abar, zbar), tab, E0, T, P, sound, ret, cv_last);
 }
 
 // helm_rhoP_given: Newton for T(rho, P); same conventions as helm_rhoe_given.
 __device__ __forceinline__ int helm_rhoP_given(const HelmDev &h, double rho, double P0,
                                                double abar, double zbar, double &T, double &E,
                                                double &sound, bool ret) {
+  const HelmRho m(h, rho, abar, zbar);
+  HelmTab tab;
   const double Told = T;
+  const Recip rP0(P0);
   int iter;
   sound = 0.0;
   for (iter = 1; iter <= kHelmMaxIter; iter++) {
     double p, dPdT;
-    helm_given1(h, rho, T, abar, zbar, p, dPdT, true);
+    helm_given1(h, m, tab, T, p, dPdT, true);
     const double res = p - P0;
-    T = T - res / dPdT;
-    double err = fabs(res / P0);
+    T = T - Recip(dPdT).div(res);
+    double err = fabs(rP0.div(res));
     if ((T < h.tl) || (T > h.th)) {
       T = Told;
       err = 1e-15;
@@ -619,10 +814,11 @@ __device__ __forceinline__ int helm_rhoP_given(const HelmDev &h, double rho, dou
   }
   if (ret) {
     double p, cv;
-    helm_full(h, rho, T, abar, zbar, p, E, sound, cv);
+    helm_full_at(h, m, T, p, E, sound, cv);
   } else {
     double dEdT;
-    helm_given2(h, rho, T, abar, zbar, E, dEdT, false);
+    HelmTab te;
+    helm_given2(h, m, te, T, E, dEdT, false);
   }
   return iter > kHelmMaxIter ? kHelmMaxIter : iter;
 }

@@ -156,7 +156,7 @@ __device__ __forceinline__ void flux_face(const Grid &g, int i, int j, int k, do
     g.emf[DIR][f] = e0;
     g.emf[DIR][nf + f] = e1v;
     const double den = 0.5 * (qL[0] + qR[0]) * g.sc->smax;
-    const double mach = F[0] / den;
+    const double mach = Recip(den).div(F[0]);
     signed char s = 0;
     if (mach > g.mach_ct) s = 1;
     if (mach < -g.mach_ct) s = -1;
@@ -1010,12 +1010,12 @@ __device__ __forceinline__ double cell_speed(const Grid &g, const double *p, con
     double pr, ei, cv;
     helm_full(g.helm, p[0], T, abar, zbar, pr, ei, c, cv);
   } else {
-    c = sqrt(g.gm * p[SD + 1] / p[0]);
+    c = dsqrt(Recip(p[0]).div(g.gm * p[SD + 1]));
   }
   if (MHD) {
     const double bz = (SD == 3) ? b[2] : 0.0;
     const double ca2 = b[0] * b[0] + b[1] * b[1] + bz * bz;
-    c = sqrt(c * c + ca2 / p[0]);
+    c = dsqrt(c * c + Recip(p[0]).div(ca2));
   }
   const double s1 = (fabs(p[1]) + c) * g.inv_dx[0];
   const double s2 = (fabs(p[2]) + c) * g.inv_dx[1];
@@ -1222,7 +1222,7 @@ __global__ void __launch_bounds__(256)
     // EoS outputs is stored before the Helmholtz solve, so that little state
     // stays live across it.
     const double rho = S[0], m1 = S[1], m2 = S[2], m3 = (SD == 3) ? S[3] : 0.0;
-    const double ir = 1.0 / rho;
+    const double ir = Recip(rho).inv();
     double eint = S[IE] - 0.5 * (m1 * m1 + m2 * m2 + m3 * m3) * ir;
     if (MHD) eint = eint - 0.5 * (b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
     if (g.etot) eint = eint - rho * g.phi_cc[j];
@@ -1275,13 +1275,13 @@ __global__ void __launch_bounds__(256)
       double ye = 1.0, abar = 1.0;   // PIG_EOS without scalars ignores both
       if constexpr (NAS >= 2) {
         ye = p[IA];
-        abar = rho / S[IA + 1];
+        abar = Recip(S[IA + 1]).div(rho);
       }
       if constexpr (NAS >= 2) {
         // the CFL's evaluation takes abar from the stored prim, 1 / (1/abar)
         // (compute_hyperbolic_dt, source/source.F90:13801-13847)
         ye_c = p[IA];
-        abar_c = 1.0 / p[IA + 1];
+        abar_c = Recip(p[IA + 1]).inv();
       }
       const double zbar = ye * abar;
       double pr, sound;
@@ -1361,8 +1361,8 @@ __global__ void __launch_bounds__(256)
       // the mixed path leaves the FP64 pressure and gammas to k_prim_from_u
       // (an evaluation at the stored T when something reads them)
       if (g.fasteos && !MIX) {
-        g.gam[c] = pr / eint + 1.0;
-        g.gam[N + c] = sound * sound * rho / pr;
+        g.gam[c] = Recip(eint).div(pr) + 1.0;
+        g.gam[N + c] = Recip(pr).div(sound * sound * rho);
       }
       g.temp[c] = T;
       if (!MIX) g.P[IE * N + c] = pr;
@@ -1370,9 +1370,9 @@ __global__ void __launch_bounds__(256)
       sound_out = sound;
       if constexpr (MIX) {
         g.Pf[IE * N + c] = (float)(g.wb ? pr - g.eq_p_cc[j] : pr);
-        const double ge = pr / eint + 1.0;
+        const double ge = Recip(eint).div(pr) + 1.0;
         g.Pf[(NV + 3) * N + c] = (float)(g.wb ? ge - g.eq_ge_cc[j] : ge);
-        g.Pf[(NV + 4) * N + c] = (float)(sound * sound * rho / pr);
+        g.Pf[(NV + 4) * N + c] = (float)Recip(pr).div(sound * sound * rho);
       }
     }
     if (last)
@@ -1414,7 +1414,7 @@ __global__ void __launch_bounds__(256) k_prim_from_u(Grid g) {
     for (int v = 0; v < SD; v++) g.bcc[v * N + c] = b[v];
   }
   const double rho = S[0], m1 = S[1], m2 = S[2], m3 = (SD == 3) ? S[3] : 0.0;
-  const double ir = 1.0 / rho;
+  const double ir = Recip(rho).inv();
   double eint = S[IE] - 0.5 * (m1 * m1 + m2 * m2 + m3 * m3) * ir;
   if (MHD) eint = eint - 0.5 * (b[0] * b[0] + b[1] * b[1] + b[2] * b[2]);
   if (g.etot) eint = eint - rho * g.phi_cc[j];
@@ -1970,7 +1970,7 @@ __global__ void __launch_bounds__(256)
           // cons -> prim and the CFL speed, as k_update (the ideal gas without
           // a field), into the buffer that no block reads in this launch
           const double rho = S[0], m1 = S[1], m2 = S[2], m3 = (SD == 3) ? S[3] : 0.0;
-          const double ir = 1.0 / rho;
+          const double ir = Recip(rho).inv();
           double p[NV];
           double eint = S[IE] - 0.5 * (m1 * m1 + m2 * m2 + m3 * m3) * ir;
           if (g.etot) eint = eint - rho * g.phi_cc[lj];

@@ -48,11 +48,13 @@ k_mlp_data(HelmDev h, long long n, unsigned long long seed, double lrs_lo, doubl
   const double ye = ye_lo + unit01(seed, i, 3) * (ye_hi - ye_lo);
   const double rho = exp10(lrs) / ye, zbar = ye * abar;
   double e, dedt;
-  helm_given2(h, rho, exp10(lt), abar, zbar, e, dedt, false);
+  const HelmRho m(h, rho, abar, zbar);
+  HelmTab tab;
+  helm_given2(h, m, tab, exp10(lt), e, dedt, false);
   double T = helm_bracket_guess(h, rho, e, abar, zbar), P, cs;
   helm_rhoe_given(h, rho, e, abar, zbar, T, P, cs, false);
   double el, dedtl;
-  helm_given2(h, rho, T, abar, zbar, el, dedtl, true);
+  helm_given2(h, m, tab, T, el, dedtl, true);
   const double slope = dedtl * T / el;  // d ln E / d ln T at the label
   wt[i] = (float)fmin(fmax(slope * slope, 1e-8), 1e4);
   raw[4 * i + 0] = (float)log10(rho);

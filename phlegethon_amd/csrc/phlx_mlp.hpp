@@ -253,47 +253,16 @@ __device__ __forceinline__ float mlp_forward_wave(const MlpDev &m, const float x
 __device__ __forceinline__ double helm_bracket_guess(const HelmDev &h, double rho, double E0,
                                                      double abar, double zbar) {
   double lo = log10(h.tl), hi = log10(h.th);
+  const HelmRho m(h, rho, abar, zbar);
+  HelmTab tab;
 #pragma unroll 1
   for (int it = 0; it < kBracketSteps; it++) {
     const double mid = 0.5 * (lo + hi);
     double e, dedt;
-    helm_given2(h, rho, exp10(mid), abar, zbar, e, dedt, false);
+    helm_given2(h, m, tab, exp10(mid), e, dedt, false);
     if (e > E0) hi = mid; else lo = mid;
   }
   return exp10(0.5 * (lo + hi));
-}
-
-// The reference's Newton loop for T(rho, e) (helm_rhoe_given) entered with
-// the first evaluation (e1, dedt1 = E and dE/dT at the incoming T) already
-// done: identical arithmetic to helm_rhoe_given from the same T, without
-// repeating that evaluation.
-__device__ __forceinline__ int helm_rhoe_given_from(const HelmDev &h, double rho, double E0,
-                                                    double abar, double zbar, double &T,
-                                                    double &P, double &sound, bool ret,
-                                                    double e1, double dedt1) {
-  const double Told = T;
-  int iter;
-  sound = 0.0;
-  for (iter = 1; iter <= kHelmMaxIter; iter++) {
-    double e = e1, dEdT = dedt1;
-    if (iter > 1) helm_given2(h, rho, T, abar, zbar, e, dEdT, true);
-    const double res = e - E0;
-    T = T - res / dEdT;
-    double err = fabs(res / E0);
-    if ((T < h.tl) || (T > h.th)) {
-      T = Told;
-      err = 1e-15;
-    }
-    if (err < kHelmTol) break;
-  }
-  if (ret) {
-    double e, cv;
-    helm_full(h, rho, T, abar, zbar, P, e, sound, cv);
-  } else {
-    double dPdT;
-    helm_given1(h, rho, T, abar, zbar, P, dPdT, false);
-  }
-  return iter > kHelmMaxIter ? kHelmMaxIter : iter;
 }
 
 // Mixed-precision T(rho, e), linearised (opt-in, phlx_set_eos_lin_tol > 0;
@@ -311,7 +280,7 @@ __device__ __forceinline__ int helm_rhoe_lin(const HelmDev &h, double lin_tol, d
                                              double &P, double &sound, int &fallback,
                                              double &cv_out) {
   double E, cv, dPdT;
-  helm_full<true>(h, rho, T, abar, zbar, P, E, sound, cv, &dPdT);
+  helm_full_fma(h, rho, T, abar, zbar, P, E, sound, cv, &dPdT);
   cv_out = cv;
   const double res = E - E0;
   const double dT = hdiv<true>(-res, cv);
@@ -418,11 +387,13 @@ __device__ __forceinline__ int helm_rhoe_guess(const HelmDev &h, int mode, doubl
     // residual); a missing guess (tg <= 0 or NaN) falls back
     if (tg > 0.0) {
       tg = fmin(fmax(tg, h.tl * (1.0 + 1e-9)), h.th * (1.0 - 1e-9));
-      double e, dedt;
-      helm_given2(h, rho, tg, abar, zbar, e, dedt, true);
-      if (fabs((e - E0) / E0) <= (double)resid_tol) {
+      const HelmRho m(h, rho, abar, zbar);
+      double at[2];  // E and dE/dT at tg: the Newton loop's first evaluation
+      HelmTab tab;
+      helm_given2(h, m, tab, tg, at[0], at[1], true);
+      if (fabs((at[0] - E0) / E0) <= (double)resid_tol) {
         T = tg;
-        return helm_rhoe_given_from(h, rho, E0, abar, zbar, T, P, sound, ret, e, dedt);
+        return helm_rhoe_given(h, m, tab, E0, T, P, sound, ret, nullptr, at);
       }
     }
     fallback = 1;
