@@ -688,11 +688,13 @@ extern "C" int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, 
 // of whole-stage passes, which ends in the other one, is not captured.
 static bool use_fused_sweep(const phlx_ctx *ctx) {
   const Grid &g = ctx->g;
-  // measured on MI355X: without MHD the fused stage is 5-19 % faster (FP64
-  // and mixed); with MHD the split sweeps are 1-5 % faster (FP32: the
-  // column segments prefetch a cell ahead at 3-4 waves/SIMD; FP64: the
-  // fused MHD sweep spills)
-  const bool want = ctx->fused_sweep < 0 ? !ctx->g.mhd : ctx->fused_sweep != 0;
+  // measured on MI355X, us per step, fused / split: without MHD always the
+  // faster form (384^3 hydro FP64 9800 / 14400, mixed 5650 / 7650); ideal MHD
+  // from 32^3 (32^3 FP64 81 / 92, mixed 69 / 87; 256^3 7055 / 7770, 4240 /
+  // 4345); MHD with the tabulated EoS spills and is slower (128^3 FP64 2090 /
+  // 1705, 256^3 mixed 7880 / 7230), as the ideal one with two scalars does
+  const bool mhd_too = ctx->cfg.eos == PHLX_EOS_IDEAL && g.nas == 0 && g.N >= 32768;
+  const bool want = ctx->fused_sweep < 0 ? !g.mhd || mhd_too : ctx->fused_sweep != 0;
   if (!want || !ctx->kt.sweep || g.sflat) return false;
   if (!ctx->kt.update_swept) return !(ctx->step_graph && ctx->stages % 2);
   return (!g.mhd || g.n1 % kSweepT == 0) &&

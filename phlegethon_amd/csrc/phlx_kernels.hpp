@@ -347,13 +347,25 @@ __device__ __forceinline__ void seg_walk(const Grid &g, int i, int o, int f0, in
   }
   cm = c0;
   c0 = cp;
+  // cell f+1 is loaded one face ahead where its registers cost no occupancy:
+  // ideal MHD, at 2 waves per SIMD either way (256^3: x2 638 -> 574 us, x3 604 ->
+  // 559); hydro would fall from 4 waves to 3 (384^3 1152 -> 1297), MHD with
+  // scalars and gammas spill (150 x 201 x 130: 245 -> 325)
+  constexpr bool AHEAD = MHD && EK == EK_IDEAL && NAS == 0;
+  CellW cn;
+  if (AHEAD) load(f0 + 1, cn, i, o);
 #pragma unroll 1
   for (int f = f0; f < f1; f++) {
     // the column indices are re-materialised per face: hoisting every
     // address and profile value of the body out of the loop costs ~100 VGPRs
     int ii = i, oo = o;
     asm volatile("" : "+v"(ii), "+v"(oo));
-    load(f + 1, cp, ii, oo);
+    if (AHEAD) {
+      cp = cn;
+      if (f + 1 < f1) load(f + 2, cn, ii, oo);
+    } else {
+      load(f + 1, cp, ii, oo);
+    }
     double qL[NV], qR[NV], bL[3] = {0.0, 0.0, 0.0}, bR[3] = {0.0, 0.0, 0.0};
     double gL[2] = {0.0, 0.0}, gR[2] = {0.0, 0.0};
     const int rec = (SF && c0.fl) ? REC_LIM2ND : g.recon;
@@ -724,41 +736,6 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(3)))
 }
 
 // ------------------------------------------------------------------ CT
-// Face-centred EMF component `comp` (0..2 = E1..E3) of the face array of
-// direction fd at a possibly-ghost transverse position; ghosts follow the
-// EMF halo copy and EMF boundary conditions (source/source.F90:11370-11964).
-// FAST: the caller guarantees an interior position (no map).  F32: the
-// mixed path's FP32 face EMFs (emff).
-template <bool FAST = false, bool F32 = false>
-__device__ __forceinline__ void face_emf(const Grid &g, int fd, int comp, int i, int j,
-                                         int k, double &e, double &s) {
-  int ii[3] = {i, j, k};
-  const int n[3] = {g.n1, g.n2, g.n3};
-  double fac = 1.0;
-#pragma unroll
-  for (int a = 0; a < 3; a++) {
-    if (FAST || a == fd || a >= g.sd) continue;
-    int c = ii[a];
-    if (c < 0 || c >= n[a]) {
-      const int side = c < 0 ? 0 : 1;
-      if (g.bc[2 * a + side] == BC_PERIODIC) {
-        ii[a] = c < 0 ? c + n[a] : c - n[a];
-      } else {
-        ii[a] = c < 0 ? 0 : n[a] - 1;
-        if (g.bc[2 * a + side] == BC_REFLECTIVE && comp != a) fac = -fac;
-      }
-    }
-  }
-  const long long f = fix(g, fd, ii[0], ii[1], ii[2]);
-  // slot of component comp within the face array
-  int slot;
-  if (fd == 0) slot = (comp == 1) ? 0 : 1;
-  else if (fd == 1) slot = (comp == 0) ? 0 : 1;
-  else slot = (comp == 0) ? 0 : 1;
-  e = fac * (F32 ? (double)g.emff[fd][slot * g.nf[fd] + f] : g.emf[fd][slot * g.nf[fd] + f]);
-  s = (double)g.sgn[fd][f];
-}
-
 // -(v x B)_comp of a cell from v and b_cc (the reference forms it from the
 // ghost-filled prim and b_cc inside the corner loops, :11966-12185).
 template <int SD>
@@ -767,30 +744,6 @@ __device__ __forceinline__ double emf_of(int comp, const double *v, const double
   if (comp == 2) return -v1 * b[1] + v2 * b[0];
   if (comp == 0) return v3 * b[1] - v2 * b[2];
   return v1 * b[2] - v3 * b[0];
-}
-
-// Stored cell EMF of a (possibly ghost) cell.  The update kernel stores
-// -(v x B) of every interior cell; a mirrored ghost flips v_a and b_a of the
-// mirrored axis a, which negates every component but E_a (each product
-// holds exactly one axis-a factor), and IEEE negation commutes with
-// rounding, so this equals the value formed from the flipped ghost state
-// bit for bit.  F32: the mixed path's FP32 cell EMFs (ecellf).
-template <int SD, bool FAST = false, bool F32 = false>
-__device__ __forceinline__ double cell_emf(const Grid &g, int comp, int i, int j, int k) {
-  if (FAST)
-    return F32 ? (double)g.ecellf[(long long)comp * g.N + cix(g, i, j, k)]
-               : g.ecell[(long long)comp * g.N + cix(g, i, j, k)];
-  int si, sj, sk = 0;
-  const int mi = map_axis(g, 0, i, g.n1, si);
-  const int mj = map_axis(g, 1, j, g.n2, sj);
-  const int mk = (SD == 3) ? map_axis(g, 2, k, g.n3, sk) : k;
-  const long long ce = (long long)comp * g.N + cix(g, mi, mj, mk);
-  double e = F32 ? (double)g.ecellf[ce] : g.ecell[ce];
-  if (comp != 0 && si && flips(g, 0, si, cix(g, si < 0 ? 0 : g.n1 - 1, mj, mk))) e = -e;
-  if (comp != 1 && sj && flips(g, 1, sj, cix(g, mi, sj < 0 ? 0 : g.n2 - 1, mk))) e = -e;
-  if (SD == 3 && comp != 2 && sk && flips(g, 2, sk, cix(g, mi, mj, sk < 0 ? 0 : g.n3 - 1)))
-    e = -e;
-  return e;
 }
 
 // Gardiner-Stone CT-contact corner EMF (source/source.F90:11966-12027)
@@ -805,75 +758,98 @@ __device__ __forceinline__ double corner_emf(double eS, double eW, double eN, do
   return 0.25 * (eS + eW + eN + eE + dS - dN + dW - dE);
 }
 
-// The three edge EMFs whose lower end is node (i, j, k) (FAST: all eight
-// surrounding cells interior; F32: FP32 face and cell EMFs, FP64 arithmetic).
-template <int SD, bool FAST, bool F32>
-__device__ __forceinline__ void corner_node(const Grid &g, int i, int j, int k) {
-  double eN, eE, eS, eW, sS, sN, sW, sE;
-  if (k < g.n3) {  // x3-edges (emfx3_cor)
-    face_emf<FAST, F32>(g, 0, 2, i, j, k, eN, sN);
-    face_emf<FAST, F32>(g, 1, 2, i, j, k, eE, sE);
-    face_emf<FAST, F32>(g, 0, 2, i, j - 1, k, eS, sS);
-    face_emf<FAST, F32>(g, 1, 2, i - 1, j, k, eW, sW);
-    const double eSW = cell_emf<SD, FAST, F32>(g, 2, i - 1, j - 1, k);
-    const double eNW = cell_emf<SD, FAST, F32>(g, 2, i - 1, j, k);
-    const double eNE = cell_emf<SD, FAST, F32>(g, 2, i, j, k);
-    const double eSE = cell_emf<SD, FAST, F32>(g, 2, i, j - 1, k);
-    {
-      const double ec = corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE);
-      if (F32) g.corf[2][kix(g, 2, i, j, k)] = (float)ec;
-      else g.cor[2][kix(g, 2, i, j, k)] = ec;
-    }
-  }
-  if (SD == 3) {
-    if (i < g.n1) {  // x1-edges (emfx1_cor, source/source.F90:12050-12107)
-      face_emf<FAST, F32>(g, 1, 0, i, j, k, eN, sN);
-      face_emf<FAST, F32>(g, 2, 0, i, j, k, eE, sE);
-      face_emf<FAST, F32>(g, 1, 0, i, j, k - 1, eS, sS);
-      face_emf<FAST, F32>(g, 2, 0, i, j - 1, k, eW, sW);
-      const double eSW = cell_emf<SD, FAST, F32>(g, 0, i, j - 1, k - 1);
-      const double eNW = cell_emf<SD, FAST, F32>(g, 0, i, j - 1, k);
-      const double eNE = cell_emf<SD, FAST, F32>(g, 0, i, j, k);
-      const double eSE = cell_emf<SD, FAST, F32>(g, 0, i, j, k - 1);
-      {
-        const double ec = corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE);
-        if (F32) g.corf[0][kix(g, 0, i, j, k)] = (float)ec;
-        else g.cor[0][kix(g, 0, i, j, k)] = ec;
-      }
-    }
-    if (j < g.n2) {  // x2-edges (emfx2_cor, source/source.F90:12128-12185)
-      face_emf<FAST, F32>(g, 2, 1, i, j, k, eN, sN);
-      face_emf<FAST, F32>(g, 0, 1, i, j, k, eE, sE);
-      face_emf<FAST, F32>(g, 2, 1, i - 1, j, k, eS, sS);
-      face_emf<FAST, F32>(g, 0, 1, i, j, k - 1, eW, sW);
-      const double eSW = cell_emf<SD, FAST, F32>(g, 1, i - 1, j, k - 1);
-      const double eNW = cell_emf<SD, FAST, F32>(g, 1, i, j, k - 1);
-      const double eNE = cell_emf<SD, FAST, F32>(g, 1, i, j, k);
-      const double eSE = cell_emf<SD, FAST, F32>(g, 1, i - 1, j, k);
-      {
-        const double ec = corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE);
-        if (F32) g.corf[1][kix(g, 1, i, j, k)] = (float)ec;
-        else g.cor[1][kix(g, 1, i, j, k)] = ec;
-      }
-    }
-  }
-}
-
 // One thread per grid node (i,j,k) in [0,n1]x[0,n2]x[0,n3]: the three edge
-// EMFs whose lower end is that node.  A wave whose nodes all have their
-// eight surrounding cells inside the grid reads without the boundary map.
+// EMFs whose lower end is that node (F32: FP32 face, cell and edge EMFs, FP64
+// arithmetic).
+// Ghosts: an edge reads face and cell EMFs one position outside the grid.  The
+// EMF halo copy and EMF boundary conditions (source/source.F90:11370-11964)
+// wrap them or take the wall's own, negated beyond a reflecting wall since the
+// component is tangential to it; a cell EMF -(v x B) there, of a mirrored state
+// with v_a and b_a flipped, is the wall cell's negated too (each product holds
+// exactly one axis-a factor, and IEEE negation commutes with rounding), and one
+// position out both mirror to the wall's own index.  So one mapped index and
+// one sign per axis side serve every load, and the loads have no branch
+// between them (with a map per load, 36 a node, the kernel was bound by index
+// arithmetic: mixed 0.67 VALU-busy at half the copy kernel's rate).
 template <int SD, bool F32>
 __global__ void __launch_bounds__(256) k_corner(Grid g) {
+  using Re = typename std::conditional<F32, float, double>::type;
+  using Bits = typename std::conditional<F32, unsigned int, unsigned long long>::type;
+  constexpr Bits kSign = (Bits)1 << (8 * sizeof(Re) - 1);
   if (!g.sc->active) return;
+  const int n1 = g.n1, n2 = g.n2, n3 = g.n3, k = blockIdx.z;
   int i, j;
-  const int k = blockIdx.z;
-  if (!plane_coords(g.n1 + 1, g.n2 + 1, i, j)) return;
-  const bool inside = i >= 1 && i < g.n1 && j >= 1 && j < g.n2 &&
-                      (SD == 2 || (k >= 1 && k < g.n3));
-  if (__all(inside))
-    corner_node<SD, true, F32>(g, i, j, k);
-  else
-    corner_node<SD, false, F32>(g, i, j, k);
+  if (!plane_coords(n1 + 1, n2 + 1, i, j)) return;
+  // position c (-1 .. n) of axis a in the grid, and the sign of what it holds
+  auto map = [&](int a, int c, int n, Bits &flip) {
+    flip = 0;
+    if (c >= 0 && c < n) return c;
+    const int side = c < 0 ? 0 : 1, bc = g.bc[2 * a + side];
+    if (bc == BC_PERIODIC) return side ? c - n : c + n;
+    if (bc == BC_REFLECTIVE) flip = kSign;
+    return side ? n - 1 : 0;
+  };
+  auto load = [](const Re *p, unsigned o, Bits flip) {
+    return (double)__builtin_bit_cast(Re, __builtin_bit_cast(Bits, p[o]) ^ flip);
+  };
+  Bits xm, xp, ym, yp;
+  const int im = map(0, i - 1, n1, xm), ip = map(0, i, n1, xp);
+  const int jm = map(1, j - 1, n2, ym), jp = map(1, j, n2, yp);
+  // in-plane offsets: x1 faces (i, j) / (i, j-1), x2 faces (i, j) / (i-1, j),
+  // cells and x3 faces of the four columns around the node
+  const unsigned f1p = jp * (n1 + 1) + i, f1m = jm * (n1 + 1) + i;
+  const unsigned f2p = j * n1 + ip, f2m = j * n1 + im;
+  const unsigned cpp = jp * n1 + ip, cmp = jp * n1 + im, cpm = jm * n1 + ip, cmm = jm * n1 + im;
+  const long long s1 = (long long)(n1 + 1) * n2, s2 = (long long)n1 * (n2 + 1),
+                  s3 = (long long)n1 * n2;
+  // planes k and k - 1 (mapped) of the x1 faces, x2 faces and cells
+  Bits zp = 0, zm = 0;
+  const int kp = SD == 3 ? map(2, k, n3, zp) : 0, km = SD == 3 ? map(2, k - 1, n3, zm) : 0;
+  const Re *const E1 = F32 ? (const Re *)g.emff[0] : (const Re *)g.emf[0];
+  const Re *const E2 = F32 ? (const Re *)g.emff[1] : (const Re *)g.emf[1];
+  const Re *const Ec = F32 ? (const Re *)g.ecellf : (const Re *)g.ecell;
+  const signed char *const g1 = g.sgn[0] + kp * s1, *const g2 = g.sgn[1] + kp * s2;
+  auto store = [&](int d, double e) {
+    const long long x = kix(g, d, i, j, k);
+    if (F32)
+      g.corf[d][x] = (float)e;
+    else
+      g.cor[d][x] = e;
+  };
+  if (k < n3) {  // x3-edges (emfx3_cor, source/source.F90:11966-12027)
+    const Re *const z1 = E1 + g.nf[0] + kp * s1, *const z2 = E2 + g.nf[1] + kp * s2,
+             *const zc = Ec + 2 * g.N + kp * s3;
+    const double eN = load(z1, f1p, yp), eS = load(z1, f1m, ym);
+    const double eE = load(z2, f2p, xp), eW = load(z2, f2m, xm);
+    const double sN = g1[f1p], sS = g1[f1m], sE = g2[f2p], sW = g2[f2m];
+    const double eSW = load(zc, cmm, xm ^ ym), eNW = load(zc, cmp, xm ^ yp);
+    const double eNE = load(zc, cpp, xp ^ yp), eSE = load(zc, cpm, xp ^ ym);
+    store(2, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
+  }
+  if constexpr (SD == 3) {
+    const Re *const e3 = (F32 ? (const Re *)g.emff[2] : (const Re *)g.emf[2]) + k * s3;
+    const signed char *const g3 = g.sgn[2] + k * s3;
+    if (i < n1) {  // x1-edges (emfx1_cor, source/source.F90:12050-12107)
+      const double eN = load(E2 + kp * s2, f2p, zp), eS = load(E2 + km * s2, f2p, zm);
+      const double eE = load(e3, cpp, yp), eW = load(e3, cpm, ym);
+      const double sN = g2[f2p], sS = g.sgn[1][km * s2 + f2p], sE = g3[cpp], sW = g3[cpm];
+      const Re *const cp = Ec + kp * s3, *const cm = Ec + km * s3;
+      const double eSW = load(cm, cpm, zm ^ ym), eNW = load(cp, cpm, zp ^ ym);
+      const double eNE = load(cp, cpp, zp ^ yp), eSE = load(cm, cpp, zm ^ yp);
+      // cell order around the edge: SW (j-1,k-1), NW (j-1,k), NE (j,k), SE (j,k-1)
+      store(0, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
+    }
+    if (j < n2) {  // x2-edges (emfx2_cor, source/source.F90:12128-12185)
+      const Re *const y3 = e3 + g.nf[2];
+      const double eN = load(y3, cpp, xp), eS = load(y3, cmp, xm);
+      const double eE = load(E1 + kp * s1, f1p, zp), eW = load(E1 + km * s1, f1p, zm);
+      const double sN = g3[cpp], sS = g3[cmp], sE = g1[f1p], sW = g.sgn[0][km * s1 + f1p];
+      const Re *const cp = Ec + g.N + kp * s3, *const cm = Ec + g.N + km * s3;
+      const double eSW = load(cm, cmp, zm ^ xm), eNW = load(cm, cpp, zm ^ xp);
+      const double eNE = load(cp, cpp, zp ^ xp), eSE = load(cp, cmp, zp ^ xm);
+      store(1, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
+    }
+  }
 }
 
 // Face-B update b = a1*b0 + a2*b + a3*dt*curl(E) in FP64 (source/source.F90
@@ -1054,6 +1030,13 @@ __device__ __forceinline__ void xcd_cell_block(int nbx, int nby, int nk, int &bx
   bz = (int)((rest / T) * KC + kk);
   bx = (int)(t % (unsigned)nbx);
   by = (int)(t / (unsigned)nbx);
+}
+
+// Blocks are dealt round-robin to the 8 XCDs, each with its own L2: block id's
+// place in an order in which every XCD takes one contiguous range of 0 .. n-1.
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned id, unsigned n) {
+  const unsigned x = id & 7u, q = n >> 3, r = n & 7u;
+  return x * q + min(x, r) + (id >> 3);
 }
 
 // ---------------------------------------------------------------- update
@@ -1651,8 +1634,18 @@ __global__ void __launch_bounds__(256)
   __shared__ Re f2[NV * NF2];  // x2 faces: [v][face b = 0..15][column a]
   const int tid = threadIdx.x;
   const int ntx = (g.n1 + TX - 1) / TX;
-  const int i0 = (blockIdx.x % ntx) * TX, j0 = (blockIdx.x / ntx) * TY;
-  const int k0 = blockIdx.y * kc, k1 = min(k0 + kc, g.n3);
+  // FP32 rows of 16 are half a line and share it, and their halo, with the
+  // next tiles: those run on the same XCD (mixed 384^3 LHLLC 2935 -> 2882 us,
+  // 192 x 256 x 192 Helmholtz 728 -> 695, 150 x 130 x 110 147 -> 120).  FP64 rows
+  // fill their lines and lose by it (384^3 4847 -> 5072 us).
+  unsigned bt = blockIdx.x, bc = blockIdx.y;
+  if (MIX) {
+    const unsigned w = xcd_contiguous(bc * gridDim.x + bt, gridDim.x * gridDim.y);
+    bt = w % gridDim.x;
+    bc = w / gridDim.x;
+  }
+  const int i0 = (int)(bt % ntx) * TX, j0 = (int)(bt / ntx) * TY;
+  const int k0 = (int)bc * kc, k1 = min(k0 + kc, g.n3);
   const long long N = g.N;
   if (!g.sc->active) {
     if constexpr (FUSE) {
@@ -1816,6 +1809,24 @@ __global__ void __launch_bounds__(256)
   double *const out = (MIX && !fin) ? g.U0 : g.U;
   const bool from_u = MIX && first && (g.sc->flags & SC_U_CUR);
 
+  // halo cells of a plane: x1 cells -2, -1, 16, 17 of rows 0..14 by the first
+  // wave, x2 rows -2, -1, 15, 16 by the second
+  const bool halo = tid < 128 && (tid >= 64 || tid < 4 * TY);
+  int ha, hb;
+  if (tid < 64) {
+    const int s = tid & 3;
+    ha = s < 2 ? s - 2 : TX - 2 + s;
+    hb = tid >> 2;
+  } else {
+    const int s = (tid - 64) >> 4;
+    ha = tid & (TX - 1);
+    hb = s < 2 ? s - 2 : TY - 2 + s;
+  }
+  const int hcell = (hb + 2) * W + ha + 2;
+  constexpr bool kHaloAhead = !(MHD && GAM);
+  Cell h;
+  if (kHaloAhead && halo) load(i0 + ha, j0 + hb, k0, h);
+
 #pragma unroll 1
   for (int k = k0; k < k1; k++) {
     // the lane's indices re-materialised per plane: hoisting every
@@ -1831,24 +1842,19 @@ __global__ void __launch_bounds__(256)
     // last reads, of plane k-1, are behind the previous iteration's second
     // barrier); the single tile takes it after this plane's reads
     if (DB && lb < TY) put(plane(k + 1), mine, nxt);
-    // the halo of plane k (its interior is staged already): x1 halo cells
-    // -2, -1, 16, 17 of rows 0..14, x2 halo rows -2, -1, 15, 16
-    if (lt < 128 && (lt >= 64 || lt < 4 * TY)) {
-      int ha, hb;
-      if (lt < 64) {
-        const int s = lt & 3;
-        ha = s < 2 ? s - 2 : TX - 2 + s;
-        hb = lt >> 2;
-      } else {
-        const int s = (lt - 64) >> 4;
-        ha = lt & (TX - 1);
-        hb = s < 2 ? s - 2 : TY - 2 + s;
-      }
-      Cell h;
-      load(i0 + ha, j0 + hb, k, h);
-      put(tk, (hb + 2) * W + ha + 2, h);
-    }
+    // the halo of plane k (its interior is staged already), loaded a plane
+    // ahead where the registers allow it, so that no plane starts with a wait
+    // for memory (256^3 MHD: FP64 2378 -> 2268 us, mixed 1301 -> 1244; 192 x 256 x
+    // 192 Helmholtz 1272 -> 1255; with MHD and gammas, over its registers
+    // already, 1885 -> 2190 at 256^3 mixed)
+    if (!kHaloAhead && halo) load(i0 + ha, j0 + hb, k, h);
+    if (halo) put(tk, hcell, h);
     __syncthreads();
+    if (SD == 3 && kHaloAhead && halo && k + 1 < k1) {
+      int hx = i0 + ha, hy = j0 + hb;
+      asm volatile("" : "+v"(hx), "+v"(hy));
+      load(hx, hy, k + 1, h);
+    }
     // in-plane faces, one of each direction per thread: x1 the lower face
     // of cell (la, lb) (the last thread row: the upper face of row la), x2
     // the lower face of row lb (16 faces: row 15's is the tile's upper face)
