@@ -656,21 +656,21 @@ static int rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, double a3
   ctx->tdiff_valid = false;
   ProfRec r;
   int on = kbegin(ctx, KID_UPDATE, r);
-  const bool guess = ctx->kt.update_guess && needs_guess_variant(ctx->g.eos_guess, ctx->eos_stats);
+  const KernelTable &kt = ctx->kt;
+  const bool lin = ctx->cfg.precision == PHLX_PREC_MIXED && ctx->g.eos_lin_tol > 0.0;
+  auto *up = swept ? kt.update_swept : kt.update;
+  if (kt.update_guess && (lin || needs_guess_variant(ctx->g.eos_guess, ctx->eos_stats))) {
+    up = swept ? kt.update_swept_guess : kt.update_guess;
+    auto *mlp = swept ? kt.update_swept_mlp : kt.update_mlp;
+    if (mlp && !lin && ctx->g.eos_guess == GUESS_MLP && !ctx->eos_stats) up = mlp;
+  }
   // stage 1 of the mixed path starts from U when the device flags say it is
   // current (the FP64 conserved state of the last step that ran); a last
   // stage that runs sets them, so a step past tmax leaves them unchanged
   const int first = irk == 0 ? 1 : 0;
   const int fin = irk == ctx->stages - 1;
   const int last = last_stage != 0;
-  if (swept && guess)
-    ctx->kt.update_swept_guess(ctx->g, first, last, a1, a2, a3, fin, ctx->stream);
-  else if (swept)
-    ctx->kt.update_swept(ctx->g, first, last, a1, a2, a3, fin, ctx->stream);
-  else if (guess)
-    ctx->kt.update_guess(ctx->g, first, last, a1, a2, a3, fin, ctx->stream);
-  else
-    ctx->kt.update(ctx->g, first, last, a1, a2, a3, fin, ctx->stream);
+  up(ctx->g, first, last, a1, a2, a3, fin, ctx->stream);
   if (fin && ctx->kt.prims) ctx->prim_stale = true;
   kend(ctx, on, r);
   return check_launch();

@@ -22,6 +22,8 @@ struct KernelTable {
   void (*faceb)(const Grid &, int, double, double, double, hipStream_t);
   void (*update)(const Grid &, int, int, double, double, double, int, hipStream_t);
   void (*update_guess)(const Grid &, int, int, double, double, double, int, hipStream_t);
+  // mixed Helmholtz: the surrogate's start alone (null: update_guess has it)
+  void (*update_mlp)(const Grid &, int, int, double, double, double, int, hipStream_t);
   void (*cfl)(const Grid &, hipStream_t);
   void (*init)(const Grid &, int restart, hipStream_t);
   void (*divb)(const Grid &, hipStream_t);
@@ -37,6 +39,7 @@ struct KernelTable {
   int (*sweep)(const Grid &, int, int, int, double, double, double, hipStream_t);
   void (*update_swept)(const Grid &, int, int, double, double, double, int, hipStream_t);
   void (*update_swept_guess)(const Grid &, int, int, double, double, double, int, hipStream_t);
+  void (*update_swept_mlp)(const Grid &, int, int, double, double, double, int, hipStream_t);
 };
 
 bool select_kernels(int sd, int nas, bool mhd, bool helm, bool fasteos, bool mixed, bool r5,

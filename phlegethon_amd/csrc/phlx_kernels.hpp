@@ -1049,32 +1049,42 @@ __device__ __forceinline__ double flux_at(const Grid &g, int d, long long idx) {
   return MIX ? (double)g.Ff[d][idx] : g.F[d][idx];
 }
 
-// GUESS (Helmholtz only): the T(rho, e) start comes from g.eos_guess (warm,
-// surrogate or bracketed) and the Newton iterations / fallbacks are counted
-// per block.  The host admits this variant only when every thread of every
-// block is an interior cell (nx1 % 64 == 0, nx2 % 4 == 0), so the surrogate's
-// wave-wide MFMA and block barriers are reached uniformly.
-// MIX with HELM: the T(rho, e) solve is one FP64 evaluation plus a
-// linearised Newton step (helm_rhoe_lin) whenever the start's residual is
-// small, and that evaluation's sound speed also serves the CFL.
+// EV (Helmholtz only), the EoS solve the kernel holds:
+//   EV_NEWTON  from the carried T or the energy predictor, to the tolerance;
+//   EV_MLP     mixed: the same Newton from the surrogate's start;
+//   EV_ANY     any start of g.eos_guess, Newton iterations / fallbacks counted
+//              per block, and the mixed path's linearised step (g.eos_lin_tol).
+// The three are kernels of their own because a kernel's registers are those
+// of its hungriest path: 255 VGPRs with the FP64 bracketing and linearised
+// solves in it, 240-246 with the mixed Newton alone, at 2 waves per SIMD either
+// way, and a third of the scalar registers spilled.  At 256^3 mixed MHD the
+// update goes 2210 -> 2100 us with the surrogate and 1830 -> 1630 from the
+// carried T; swept at 192 x 256 x 192, 563 -> 507.  (3 waves per SIMD spill 73
+// registers and take 2890.)  The host admits the surrogate and the counting only
+// when every thread of every block is an interior cell (nx1 % 64 == 0,
+// nx2 % 4 == 0), so the wave-wide MFMA and the block barriers are reached
+// uniformly.
+enum { EV_NEWTON = 0, EV_MLP = 1, EV_ANY = 2 };
 #ifndef PHLX_HELM_UPDATE_WAVES
 #define PHLX_HELM_UPDATE_WAVES 1
 #endif
-// The GUESS variants hold the surrogate's 16 accumulation registers beside
-// the EoS state; they are held to 2 waves per SIMD (VGPRs + AGPRs <= 256),
-// which the unconstrained allocation can miss by a few registers and then
-// halve the occupancy.
-// The mixed-precision Helmholtz update (the EoS Newton on a rho-contracted
-// cell) is held to PHLX_HELM_MIX_UPDATE_WAVES waves per SIMD: left free, its
-// allocation lands a few registers above the 2-wave budget (1 wave per SIMD,
-// the table loads and the HBM streaming then overlap poorly).
+// Waves per SIMD the register allocation aims at: the EV_ANY variants are held
+// to 2 (VGPRs + AGPRs <= 256), which the unconstrained allocation can miss by a
+// few registers and then halve the occupancy.
 #ifndef PHLX_HELM_MIX_UPDATE_WAVES
 #define PHLX_HELM_MIX_UPDATE_WAVES 2
 #endif
-template <int SD, int NAS, bool MHD, bool HELM, bool MIX, bool GUESS = false, bool SWEPT = false>
+#ifndef PHLX_HELM_MLP_UPDATE_WAVES
+#define PHLX_HELM_MLP_UPDATE_WAVES 2
+#endif
+template <int SD, int NAS, bool MHD, bool HELM, bool MIX, int EV = EV_NEWTON, bool SWEPT = false>
 __global__ void __launch_bounds__(256)
     __attribute__((amdgpu_waves_per_eu(
-        HELM ? (GUESS ? 2 : (MIX ? PHLX_HELM_MIX_UPDATE_WAVES : PHLX_HELM_UPDATE_WAVES)) : 1)))
+        !HELM ? 1
+        : EV == EV_ANY ? 2
+        : EV == EV_MLP ? PHLX_HELM_MLP_UPDATE_WAVES
+        : MIX          ? PHLX_HELM_MIX_UPDATE_WAVES
+                       : PHLX_HELM_UPDATE_WAVES)))
     k_update(Grid g, int first, int last, double a1,
                                                 double a2, double c3, int fin) {
   // first: stage 1, state0 rebuilt from prim + eint (the reference), or in
@@ -1274,25 +1284,31 @@ __global__ void __launch_bounds__(256)
       const bool pred = g.eos_guess == GUESS_PRED;
       double tg = T, cvl = 0.0;
       if (pred) tg = helm_pred_start(T, e0, g.eprev[c], g.cvf[c]);
-      if constexpr (GUESS) {
+      // the surrogate's corrected warm start: T_prev * 10^(s (y_now - y_prev));
+      // the previous output is NaN before the first solve of a zone
+      auto surrogate_start = [&]() {
         __shared__ unsigned int lds[4 * kMlpLdsWaveDw];
+        float x[4];
+        bool ok;
+        mlp_inputs(g.mlp, rho, e0, abar, zbar, x, ok);
+        const float y = mlp_forward_wave(g.mlp, x, lds + threadIdx.y * kMlpLdsWaveDw);
+        const float yp = g.mlp_y[c];
+        // 10^d with d ~ the change of log10 T since the last solve:
+        // FP32 exp2 (the factor's ~1e-7 error only moves the Newton start)
+        if (ok && yp == yp)
+          tg = T * (double)__builtin_amdgcn_exp2f(g.mlp.out_scale * (y - yp) *
+                                                  3.32192809488736235f);
+        g.mlp_y[c] = ok ? y : __int_as_float(0x7fffffff);
+      };
+      if constexpr (EV == EV_MLP) {
+        static_assert(MIX, "the FP64 solve judges the guess and may fall back");
+        surrogate_start();
+        if (tg >= g.helm.tl && tg <= g.helm.th) T = tg;
+        helm_rhoe_mixed(g.helm, rho, e0, abar, zbar, T, pr, sound, cvl);
+      } else if constexpr (EV == EV_ANY) {
         __shared__ unsigned int cnt[3];
         const int mode = g.eos_guess;
-        if (mode == GUESS_MLP) {
-          // corrected warm start: T_prev * 10^(s (y_now - y_prev)); the
-          // previous output is NaN before the first solve of a zone
-          float x[4];
-          bool ok;
-          mlp_inputs(g.mlp, rho, e0, abar, zbar, x, ok);
-          const float y = mlp_forward_wave(g.mlp, x, lds + threadIdx.y * kMlpLdsWaveDw);
-          const float yp = g.mlp_y[c];
-          // 10^d with d ~ the change of log10 T since the last solve:
-          // FP32 exp2 (the factor's ~1e-7 error only moves the Newton start)
-          if (ok && yp == yp)
-            tg = T * (double)__builtin_amdgcn_exp2f(g.mlp.out_scale * (y - yp) *
-                                                    3.32192809488736235f);
-          g.mlp_y[c] = ok ? y : __int_as_float(0x7fffffff);
-        }
+        if (mode == GUESS_MLP) surrogate_start();
         int fb = 0, it;
         if constexpr (MIX) {
           if (mode == GUESS_BRACKET) tg = helm_bracket_guess(g.helm, rho, e0, abar, zbar);
@@ -1321,14 +1337,9 @@ __global__ void __launch_bounds__(256)
         }
       } else if constexpr (MIX) {
         // the reference Newton to its tolerance from the carried T (or the
-        // predictor's start), every iterate one FP64 evaluation; a positive
-        // eos_lin_tol selects the one-evaluation linearised step instead
+        // predictor's start), every iterate one FP64 evaluation
         if (tg >= g.helm.tl && tg <= g.helm.th) T = tg;
-        int fb;
-        if (g.eos_lin_tol > 0.0)
-          helm_rhoe_lin(g.helm, g.eos_lin_tol, rho, e0, abar, zbar, T, pr, sound, fb, cvl);
-        else
-          helm_rhoe_mixed(g.helm, rho, e0, abar, zbar, T, pr, sound, cvl);
+        helm_rhoe_mixed(g.helm, rho, e0, abar, zbar, T, pr, sound, cvl);
       } else {
         // without FASTEOS the last evaluation is pressure only (:13654-13655)
         if (pred && tg >= g.helm.tl && tg <= g.helm.th) T = tg;
@@ -2268,7 +2279,7 @@ struct Kern {
   static void update_guess(const Grid &g, int first, int last, double a1, double a2, double c3,
                            int fin, hipStream_t st) {
     const dim3 blk = cell_block(g);
-    k_update<SD, NAS, MHD, HELM, MIX, true><<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(
+    k_update<SD, NAS, MHD, HELM, MIX, EV_ANY><<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(
         g, first, last, a1, a2, c3, fin);
   }
   // the fused sweep, whole stages of it where nothing but cons -> prim follows
@@ -2291,7 +2302,23 @@ struct Kern {
                            int fin, hipStream_t st) {
     if constexpr (kSwept && !kWhole) {
       const dim3 blk = cell_block(g);
-      k_update<SD, NAS, MHD, HELM, MIX, false, true>
+      k_update<SD, NAS, MHD, HELM, MIX, EV_NEWTON, true>
+          <<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g, first, last, a1, a2, c3, fin);
+    }
+  }
+  static void update_mlp(const Grid &g, int first, int last, double a1, double a2, double c3,
+                         int fin, hipStream_t st) {
+    if constexpr (HELM && MIX) {
+      const dim3 blk = cell_block(g);
+      k_update<SD, NAS, MHD, HELM, MIX, EV_MLP><<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(
+          g, first, last, a1, a2, c3, fin);
+    }
+  }
+  static void update_swept_mlp(const Grid &g, int first, int last, double a1, double a2, double c3,
+                               int fin, hipStream_t st) {
+    if constexpr (kSwept && HELM && MIX) {
+      const dim3 blk = cell_block(g);
+      k_update<SD, NAS, MHD, HELM, MIX, EV_MLP, true>
           <<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g, first, last, a1, a2, c3, fin);
     }
   }
@@ -2299,7 +2326,7 @@ struct Kern {
                                  double c3, int fin, hipStream_t st) {
     if constexpr (kSwept && HELM) {
       const dim3 blk = cell_block(g);
-      k_update<SD, NAS, MHD, HELM, MIX, true, true>
+      k_update<SD, NAS, MHD, HELM, MIX, EV_ANY, true>
           <<<grid_flat(g.n1, g.n2, g.n3, blk), blk, 0, st>>>(g, first, last, a1, a2, c3, fin);
     }
   }
@@ -2343,6 +2370,7 @@ static KernelTable make_table() {
   t.faceb = &K::faceb;
   t.update = &K::update;
   t.update_guess = HELM ? &K::update_guess : nullptr;
+  t.update_mlp = HELM && MIX && NAS == 2 ? &K::update_mlp : nullptr;
   t.cfl = &K::cfl;
   t.init = &K::init;
   t.divb = &K::divb;
@@ -2352,6 +2380,7 @@ static KernelTable make_table() {
     t.sweep = &K::sweep;
     t.update_swept = K::kWhole ? nullptr : &K::update_swept;
     t.update_swept_guess = HELM ? &K::update_swept_guess : nullptr;
+    t.update_swept_mlp = HELM && MIX && NAS == 2 ? &K::update_swept_mlp : nullptr;
   }
   return t;
 }
