@@ -1482,12 +1482,12 @@ extern "C" int phlx_set_thermal_diffusion(phlx_ctx *ctx, int32_t enable, int32_t
     }
   }
   HIPCHK(hipSetDevice(ctx->device));
-  if (!g.e0) {
+  if (!g.rkl[0]) {
     const long long k3 = (g.sd == 3) ? g.n3 + 2 : 1;
     const size_t nk = (size_t)(g.n1 + 2) * (g.n2 + 2) * k3;
     int rc = dalloc(ctx, &g.kappa, nk);
-    if (!rc) rc = dalloc(ctx, &g.e0, (size_t)g.N);
-    if (!rc) rc = dalloc(ctx, &g.ejm2, (size_t)g.N);
+    if (!rc) rc = dalloc(ctx, &g.rkl[0], (size_t)g.N);
+    if (!rc) rc = dalloc(ctx, &g.rkl[1], (size_t)g.N);
     if (!rc) rc = dalloc(ctx, &g.me0, (size_t)g.N);
     if (!rc && !helm) rc = dalloc(ctx, &g.tdiff, (size_t)g.N);
     if (rc) return rc;
@@ -1567,8 +1567,8 @@ static int diffusion_step(phlx_ctx *ctx, int strang) {
   const double mut1 = (1.0 / 3.0) * w1;
   ProfRec r;
   int on = kbegin(ctx, KID_DIFF, r);
-  if (!helm && !ctx->tdiff_valid) launch_diff_t_from_p(g, ctx->stream);
-  launch_diff_stage(g, true, 0.0, 0.0, 0.0, half_dt * mut1, 0.0, ctx->stream);
+  launch_diff_stage(g, helm || ctx->tdiff_valid ? DIFF_FIRST_ARRAY : DIFF_FIRST_P, g.eint,
+                    nullptr, g.rkl[0], 0.0, 0.0, 0.0, half_dt * mut1, 0.0, ctx->stream);
   double bjm2 = 1.0 / 3.0, bjm1 = 1.0 / 3.0;
   for (int j = 2; j <= s; j++) {
     const double bj = ((double)(j * j + j) - 2.0) / (2.0 * j * (j + 1.0));
@@ -1576,13 +1576,16 @@ static int diffusion_step(phlx_ctx *ctx, int strang) {
     const double mutj = muj * w1;
     const double nuj = -(((j - 1.0) / j) * bj / bjm2);
     const double gammatj = -(1.0 - bjm1) * mutj;
-    launch_diff_temp(g, helm, ctx->stream);
-    launch_diff_stage(g, false, muj, nuj, 1.0 - muj - nuj, half_dt * mutj, half_dt * gammatj,
-                      ctx->stream);
+    // e_j over e_jm2's buffer (e_0 itself stays in g.eint)
+    double *ejm1 = g.rkl[j & 1], *ej = g.rkl[(j & 1) ^ 1];
+    if (helm) launch_diff_temp(g, ejm1, ctx->stream);
+    launch_diff_stage(g, helm ? DIFF_ARRAY : j < s ? DIFF_E : DIFF_LAST_E, ejm1,
+                      j == 2 ? g.eint : ej, ej, muj, nuj, 1.0 - muj - nuj, half_dt * mutj,
+                      half_dt * gammatj, ctx->stream);
     bjm2 = bjm1;
     bjm1 = bj;
   }
-  launch_diff_final(g, helm, ctx->stream);
+  if (helm) launch_diff_final(g, g.rkl[(s & 1) ^ 1], ctx->stream);
   if (ctx->kt.pack) {
     // the primitives moved past U
     ctx->kt.pack(g, ctx->stream);

@@ -97,14 +97,22 @@ struct Grid {
   unsigned char *sf_det, *sf_flag;
   // THERMAL_DIFFUSION_STS: kappa on cells -1 .. n (one ghost layer), the
   // temperature the residual reads (temp with Helmholtz, an own array for
-  // the ideal gas), RKL2 registers e_0, e_jm2, Me_0, wall temperatures of
+  // the ideal gas), RKL2 registers (two of the last stages
+  // in turn, Me_0), wall temperatures of
   // FIX_TEMPERATURE_AT_* (NaN: zero-gradient ghost)
-  double *kappa, *tdiff, *e0, *ejm2, *me0;
+  double *kappa, *tdiff, *rkl[2], *me0;
   double fix_t[6];
   double *red;       // per-block partial maxima of the cell-grid reductions
   int nred;          // number of partials (blocks of a cell-grid launch)
   Scalars *sc;
 };
+
+// Blocks are dealt round-robin to the 8 XCDs, each with its own L2: block id's
+// place in an order in which every XCD takes one contiguous range of 0 .. n-1.
+__device__ __forceinline__ unsigned xcd_contiguous(unsigned id, unsigned n) {
+  const unsigned x = id & 7u, q = n >> 3, r = n & 7u;
+  return x * q + min(x, r) + (id >> 3);
+}
 
 __device__ __forceinline__ long long cix(const Grid &g, int i, int j, int k) {
   return ((long long)k * g.n2 + j) * g.n1 + i;

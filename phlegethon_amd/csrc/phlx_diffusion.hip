@@ -2,17 +2,23 @@
 // the radiative diffusion of internal energy, Strang-split around the hydro
 // step (source/source.F90:6672-6688, thermal_diffusion_step :19949-20269).
 //
-// One diffusion step over dt/2 with s stages (s from dt / dt_par on the host):
-//   [k_diff_t_from_p]            ideal gas: T of the hydro state
-//   k_diff_stage<FIRST>          residual M(T), e_0 = eint, Me_0 = M, stage 1
-//   s-1 x (k_diff_temp, k_diff_stage)   eint_to_temp, residual, RKL2 stage
-//   k_diff_final                 eint_to_temp, p (Helmholtz: eint, gammas)
+// One diffusion step over dt/2 with s >= 3 stages (s from dt / dt_par on the
+// host):
+//   k_diff_stage<FIRST>          Me_0 = M(T), e_1
+//   s-1 x k_diff_stage           ideal gas: T from e_jm1 on the fly, residual,
+//                                RKL2 stage, and at the last one p and T
+//   Helmholtz: s-1 x (k_diff_temp, k_diff_stage), then k_diff_final
+// e_0 stays in g.eint until the last stage; e_j alternates between the two
+// g.rkl buffers, over e_jm2, which only the thread of its own cell reads.
 // The residual is sum_d (F(+) - F(-)) / dx_d of the face flux
 // F = (4/3) a c K_int dT/dx, K = T^3 / (rho kappa), K_int the harmonic
 // mean of the two cells; each face flux is recomputed by the two cells that
 // share it (same operands, same bits) instead of a face array round trip.
-// Every kernel is one thread per cell and HBM bound (7-point stencils of T,
-// rho and kappa from cache).
+//
+// Every kernel is one thread per cell and HBM bound: a middle stage of the ideal
+// gas moves 56 bytes per cell (e_jm1, rho, kappa, e_jm2, e_0, Me_0 in, e_j out;
+// the neighbours from cache), where a T pass and an in-place update took
+// 96 and two launches: 50 -> 24 us per stage at 128^3 (4.9 TB/s of those bytes).
 #include "phlx_internal.hpp"
 
 namespace phlx {
@@ -25,66 +31,72 @@ __device__ __forceinline__ long long kapix(const Grid &g, int i, int j, int k) {
   return ((long long)(k + k0) * (g.n2 + 2) + (j + 1)) * (g.n1 + 2) + (i + 1);
 }
 
-// (T, rho) of the cell beside (i, j, k) along axis a at offset o = -1/+1 (the
-// cell itself at o = 0); ghosts per bcs_thermal_diffusion (:20837-21068):
-// periodic copies, else rho extrapolated linearly from the wall cells and T
-// copied from the wall cell or set to 2 T_wall - T (FIX_TEMPERATURE_AT_*).
-template <int SD>
-__device__ __forceinline__ void diff_cell(const Grid &g, int i, int j, int k, int a, int o,
-                                          double &T, double &rho) {
+// Where a stage's temperatures come from: the g.tdiff array, p / (rho R / mu)
+// of the hydro state (source/source.F90:13670-13674), or eint_to_temp of the
+// ideal gas in closed form (:20271-20392).
+enum { DT_ARRAY = 0, DT_P = 1, DT_E = 2 };
+template <int SD, int TS>
+__device__ __forceinline__ double diff_temp_at(const Grid &g, const double *e, long long c,
+                                               double rho) {
+  if (TS == DT_P) return Recip(rho * kRgas * g.inv_mu).div(g.P[(long long)(SD + 1) * g.N + c]);
+  if (TS == DT_E) return Recip(g.inv_mu * rho * kRgas).div(g.gmm1 * e[c]);
+  return g.tdiff[c];
+}
+
+// (T, rho) of the cell beside (i, j, k) along axis a at offset o = -1/+1;
+// ghosts per bcs_thermal_diffusion (:20837-21068): periodic copies, else rho
+// extrapolated linearly from the wall cells and T copied from the wall cell
+// or set to 2 T_wall - T (FIX_TEMPERATURE_AT_*).
+template <int SD, int TS>
+__device__ __forceinline__ void diff_cell(const Grid &g, const double *e, int i, int j, int k,
+                                          int a, int o, double &T, double &rho) {
   int x[3] = {i, j, k};
   const int n[3] = {g.n1, g.n2, g.n3};
   x[a] += o;
-  const double *tp = g.tdiff;
-  if (x[a] >= 0 && x[a] < n[a]) {
-    const long long c = cix(g, x[0], x[1], x[2]);
-    T = tp[c];
-    rho = g.P[c];
-    return;
+  const int side = o < 0 ? 0 : 1;
+  const bool out = x[a] < 0 || x[a] >= n[a];
+  const bool wall = out && g.bc[2 * a + side] != BC_PERIODIC;
+  if (out) x[a] = (wall ? side : !side) ? n[a] - 1 : 0;
+  const long long c = cix(g, x[0], x[1], x[2]);
+  rho = g.P[c];
+  T = diff_temp_at<SD, TS>(g, e, c, rho);
+  if (wall) {
+    x[a] = side ? n[a] - 2 : 1;
+    rho = 2.0 * rho - g.P[cix(g, x[0], x[1], x[2])];
+    const double tw = g.fix_t[2 * a + side];
+    if (tw == tw) T = 2.0 * tw - T;
   }
-  const int side = x[a] < 0 ? 0 : 1;
-  if (g.bc[2 * a + side] == BC_PERIODIC) {
-    x[a] = side ? x[a] - n[a] : x[a] + n[a];
-    const long long c = cix(g, x[0], x[1], x[2]);
-    T = tp[c];
-    rho = g.P[c];
-    return;
-  }
-  x[a] = side ? n[a] - 1 : 0;
-  const long long c0 = cix(g, x[0], x[1], x[2]);
-  x[a] = side ? n[a] - 2 : 1;
-  const long long c1 = cix(g, x[0], x[1], x[2]);
-  rho = 2.0 * g.P[c0] - g.P[c1];
-  const double tw = g.fix_t[2 * a + side];
-  T = (tw == tw) ? 2.0 * tw - tp[c0] : tp[c0];
 }
 
-// Radiative flux of the face between cells m and p (:20488-20509).
-__device__ __forceinline__ double diff_face(double tm, double rm, double km, double tp,
-                                            double rp, double kp, double inv_dl) {
+// Radiative flux of the face between cells m and p from their T and K
+// (:20488-20509).
+__device__ __forceinline__ double diff_face(double tm, double km, double tp, double kp,
+                                            double inv_dl) {
   const double krad = (4.0 / 3.0) * kRad * kClight;
-  const double kmn = tm * tm * tm / (rm * km);
-  const double kpl = tp * tp * tp / (rp * kp);
-  const double kint = 2.0 * (kmn * kpl) / (kmn + kpl);
+  const double kint = Recip(km + kp).div(2.0 * (km * kp));
   const double grad = (tp - tm) * inv_dl;
   return krad * kint * grad;
 }
+__device__ __forceinline__ double diff_k(double T, double rho, double kappa) {
+  return Recip(rho * kappa).div(T * T * T);
+}
 
 // residuals_thermal_diffusion (:20394-20835), Cartesian, x1 first.
-template <int SD>
-__device__ __forceinline__ double diff_residual(const Grid &g, int i, int j, int k) {
-  const long long c = cix(g, i, j, k);
-  const double tc = g.tdiff[c], rc = g.P[c], kc = g.kappa[kapix(g, i, j, k)];
+template <int SD, int TS>
+__device__ __forceinline__ double diff_residual(const Grid &g, const double *e, int i, int j,
+                                                int k, double rc) {
+  const double tc = diff_temp_at<SD, TS>(g, e, cix(g, i, j, k), rc);
+  const double kc = diff_k(tc, rc, g.kappa[kapix(g, i, j, k)]);
   double m = 0.0;
 #pragma unroll
   for (int a = 0; a < SD; a++) {
     double tm, rm, tq, rq;
-    diff_cell<SD>(g, i, j, k, a, -1, tm, rm);
-    diff_cell<SD>(g, i, j, k, a, +1, tq, rq);
-    const double km = g.kappa[kapix(g, i - (a == 0), j - (a == 1), k - (a == 2))];
-    const double kq = g.kappa[kapix(g, i + (a == 0), j + (a == 1), k + (a == 2))];
-    const double fm = diff_face(tm, rm, km, tc, rc, kc, g.inv_dx[a]);
-    const double fp = diff_face(tc, rc, kc, tq, rq, kq, g.inv_dx[a]);
+    diff_cell<SD, TS>(g, e, i, j, k, a, -1, tm, rm);
+    diff_cell<SD, TS>(g, e, i, j, k, a, +1, tq, rq);
+    const double km = diff_k(tm, rm, g.kappa[kapix(g, i - (a == 0), j - (a == 1), k - (a == 2))]);
+    const double kq = diff_k(tq, rq, g.kappa[kapix(g, i + (a == 0), j + (a == 1), k + (a == 2))]);
+    const double fm = diff_face(tm, km, tc, kc, g.inv_dx[a]);
+    const double fp = diff_face(tc, kc, tq, kq, g.inv_dx[a]);
     const double d = (fp - fm) * g.inv_dx[a];
     m = (a == 0) ? d : m + d;
   }
@@ -99,92 +111,85 @@ __device__ __forceinline__ bool diff_coords(const Grid &g, int &i, int &j, int &
   return i < g.n1 && j < g.n2;
 }
 
-// Ideal gas: T of the hydro state, p / (rho R / mu) (:13670-13674).
-template <int SD>
-__global__ void __launch_bounds__(256) k_diff_t_from_p(Grid g) {
+// Stage 1 (FIRST): Me_0 = M, e_1 = e_0 + (dt/2 mu~_1) Me_0.
+// Stage j: e_j = mu e_jm1 + nu e_jm2 + (1 - mu - nu) e_0 + (dt/2 mu~) M
+//                + (dt/2 gamma~) Me_0 (:20129-20190).
+// LAST (ideal gas): the step's end with it, eint = e_s, eint_to_temp and p.
+// The block order gives each XCD contiguous planes, whose rows and the planes
+// beside them its L2 holds.
+template <int SD, int TS, bool FIRST, bool LAST>
+__global__ void __launch_bounds__(256)
+    k_diff_stage(Grid g, unsigned nbx, unsigned nby, const double *ejm1, const double *ejm2,
+                 double *ej, double mu, double nu, double c0, double hm, double hg) {
   if (!g.sc->active) return;
-  int i, j, k;
-  if (!diff_coords<SD>(g, i, j, k)) return;
+  const unsigned w = xcd_contiguous(blockIdx.x, gridDim.x);
+  const int i = (w % nbx) * blockDim.x + threadIdx.x;
+  const int j = (w / nbx % nby) * blockDim.y + threadIdx.y;
+  const int k = w / nbx / nby;
+  if (i >= g.n1 || j >= g.n2) return;
   const long long c = cix(g, i, j, k);
-  g.tdiff[c] = g.P[(long long)(SD + 1) * g.N + c] / (g.P[c] * kRgas * g.inv_mu);
-}
-
-// Stage 1 (FIRST): e_0 = e_jm2 = eint, Me_0 = M, eint = e_0 + (dt/2 mu~_1) Me_0.
-// Stage j: eint = mu e_jm1 + nu e_jm2 + (1 - mu - nu) e_0 + (dt/2 mu~) M
-//                 + (dt/2 gamma~) Me_0, e_jm2 = e_jm1 (:20129-20190).
-template <int SD, bool FIRST>
-__global__ void __launch_bounds__(256) k_diff_stage(Grid g, double mu, double nu, double c0,
-                                                    double hm, double hg) {
-  if (!g.sc->active) return;
-  int i, j, k;
-  if (!diff_coords<SD>(g, i, j, k)) return;
-  const long long c = cix(g, i, j, k);
-  const double m = diff_residual<SD>(g, i, j, k);
+  const double rho = g.P[c];
+  const double m = diff_residual<SD, TS>(g, ejm1, i, j, k, rho);
   if (FIRST) {
-    const double e0 = g.eint[c];
-    g.e0[c] = e0;
     g.me0[c] = m;
-    g.ejm2[c] = e0;
-    g.eint[c] = e0 + hm * m;
+    ej[c] = ejm1[c] + hm * m;
   } else {
-    const double ejm1 = g.eint[c];
-    g.eint[c] = mu * ejm1 + nu * g.ejm2[c] + c0 * g.e0[c] + hm * m + hg * g.me0[c];
-    g.ejm2[c] = ejm1;
+    const double e = mu * ejm1[c] + nu * ejm2[c] + c0 * g.eint[c] + hm * m + hg * g.me0[c];
+    if (LAST) {
+      const double T = Recip(g.inv_mu * rho * kRgas).div(g.gmm1 * e);
+      g.eint[c] = e;
+      g.tdiff[c] = T;
+      g.P[(long long)(SD + 1) * g.N + c] = kRgas * rho * T * g.inv_mu;
+    } else {
+      ej[c] = e;
+    }
   }
 }
 
-// eint_to_temp (:20271-20392): the ideal gas in closed form, Helmholtz by
-// helm_rhoe_given from the carried T.
-template <int SD, bool HELM>
+// eint_to_temp (:20271-20392) with Helmholtz: helm_rhoe_given from the
+// carried T.
 __device__ __forceinline__ double diff_eint_to_temp(const Grid &g, long long c, double rho,
-                                                    double eint) {
-  if (!HELM) return g.gmm1 * eint / (g.inv_mu * rho * kRgas);
-  double ye, abar;
-  cell_ye_abar(g, c, ye, abar);
-  const double zbar = ye * abar;
+                                                    double eint, double abar, double zbar) {
   double T = g.tdiff[c], pr, sound;
   helm_rhoe_given(g.helm, rho, eint / rho, abar, zbar, T, pr, sound, false);
   return T;
 }
 
-template <int SD, bool HELM>
-__global__ void __launch_bounds__(256) k_diff_temp(Grid g) {
+template <int SD>
+__global__ void __launch_bounds__(256) k_diff_temp(Grid g, const double *e) {
   if (!g.sc->active) return;
   int i, j, k;
   if (!diff_coords<SD>(g, i, j, k)) return;
   const long long c = cix(g, i, j, k);
-  g.tdiff[c] = diff_eint_to_temp<SD, HELM>(g, c, g.P[c], g.eint[c]);
+  double ye, abar;
+  cell_ye_abar(g, c, ye, abar);
+  g.tdiff[c] = diff_eint_to_temp(g, c, g.P[c], e[c], abar, ye * abar);
 }
 
-// The step's end (:20193-20267): eint_to_temp, then p from (rho, T); with
-// Helmholtz also eint = rho e(T) and the FASTEOS gammas.
-template <int SD, bool HELM>
-__global__ void __launch_bounds__(256) k_diff_final(Grid g) {
+// The step's end with Helmholtz (:20193-20267): eint_to_temp, then p and
+// eint = rho e(T) from (rho, T), and the FASTEOS gammas.
+template <int SD>
+__global__ void __launch_bounds__(256) k_diff_final(Grid g, const double *es) {
   if (!g.sc->active) return;
   int i, j, k;
   if (!diff_coords<SD>(g, i, j, k)) return;
   constexpr int IP = SD + 1;
   const long long c = cix(g, i, j, k), N = g.N;
   const double rho = g.P[c];
-  const double T = diff_eint_to_temp<SD, HELM>(g, c, rho, g.eint[c]);
+  double ye, abar;
+  cell_ye_abar(g, c, ye, abar);
+  const double T = diff_eint_to_temp(g, c, rho, es[c], abar, ye * abar);
   g.tdiff[c] = T;
-  if (HELM) {
-    double ye, abar;
-    cell_ye_abar(g, c, ye, abar);
-    const double zbar = abar * ye;
-    double pr, e, sound, cv;
-    helm_full(g.helm, rho, T, abar, zbar, pr, e, sound, cv);
-    helm_pin(pr);
-    helm_pin(sound);
-    const double eint = rho * e;
-    g.P[IP * N + c] = pr;
-    g.eint[c] = eint;
-    if (g.fasteos) {
-      g.gam[c] = pr / eint + 1.0;
-      g.gam[N + c] = sound * sound * rho / pr;
-    }
-  } else {
-    g.P[IP * N + c] = kRgas * rho * T * g.inv_mu;
+  double pr, e, sound, cv;
+  helm_full(g.helm, rho, T, abar, abar * ye, pr, e, sound, cv);
+  helm_pin(pr);
+  helm_pin(sound);
+  const double eint = rho * e;
+  g.P[IP * N + c] = pr;
+  g.eint[c] = eint;
+  if (g.fasteos) {
+    g.gam[c] = pr / eint + 1.0;
+    g.gam[N + c] = sound * sound * rho / pr;
   }
 }
 
@@ -217,44 +222,38 @@ static dim3 diff_grid(const Grid &g) {
   return dim3((g.n1 + b.x - 1) / b.x, (g.n2 + b.y - 1) / b.y, g.n3);
 }
 
-void launch_diff_t_from_p(const Grid &g, hipStream_t st) {
-  const dim3 blk = cell_block(g);
-  if (g.sd == 3) k_diff_t_from_p<3><<<diff_grid(g), blk, 0, st>>>(g);
-  else k_diff_t_from_p<2><<<diff_grid(g), blk, 0, st>>>(g);
-}
-
-void launch_diff_stage(const Grid &g, bool first, double mu, double nu, double c0, double hm,
-                       double hg, hipStream_t st) {
-  const dim3 blk = cell_block(g);
-  if (g.sd == 3) {
-    if (first) k_diff_stage<3, true><<<diff_grid(g), blk, 0, st>>>(g, mu, nu, c0, hm, hg);
-    else k_diff_stage<3, false><<<diff_grid(g), blk, 0, st>>>(g, mu, nu, c0, hm, hg);
-  } else {
-    if (first) k_diff_stage<2, true><<<diff_grid(g), blk, 0, st>>>(g, mu, nu, c0, hm, hg);
-    else k_diff_stage<2, false><<<diff_grid(g), blk, 0, st>>>(g, mu, nu, c0, hm, hg);
+template <int SD>
+static void diff_stage(const Grid &g, int form, const double *ejm1, const double *ejm2, double *ej,
+                       double mu, double nu, double c0, double hm, double hg, hipStream_t st) {
+  const dim3 b = cell_block(g), n = diff_grid(g), q(n.x * n.y * n.z);
+  const auto go = [&](auto kern) {
+    kern<<<q, b, 0, st>>>(g, n.x, n.y, ejm1, ejm2, ej, mu, nu, c0, hm, hg);
+  };
+  switch (form) {
+    case DIFF_FIRST_ARRAY: return go(k_diff_stage<SD, DT_ARRAY, true, false>);
+    case DIFF_FIRST_P: return go(k_diff_stage<SD, DT_P, true, false>);
+    case DIFF_ARRAY: return go(k_diff_stage<SD, DT_ARRAY, false, false>);
+    case DIFF_E: return go(k_diff_stage<SD, DT_E, false, false>);
+    default: return go(k_diff_stage<SD, DT_E, false, true>);
   }
 }
 
-void launch_diff_temp(const Grid &g, bool helm, hipStream_t st) {
-  const dim3 blk = cell_block(g);
-  if (g.sd == 3) {
-    if (helm) k_diff_temp<3, true><<<diff_grid(g), blk, 0, st>>>(g);
-    else k_diff_temp<3, false><<<diff_grid(g), blk, 0, st>>>(g);
-  } else {
-    if (helm) k_diff_temp<2, true><<<diff_grid(g), blk, 0, st>>>(g);
-    else k_diff_temp<2, false><<<diff_grid(g), blk, 0, st>>>(g);
-  }
+void launch_diff_stage(const Grid &g, int form, const double *ejm1, const double *ejm2, double *ej,
+                       double mu, double nu, double c0, double hm, double hg, hipStream_t st) {
+  if (g.sd == 3) diff_stage<3>(g, form, ejm1, ejm2, ej, mu, nu, c0, hm, hg, st);
+  else diff_stage<2>(g, form, ejm1, ejm2, ej, mu, nu, c0, hm, hg, st);
 }
 
-void launch_diff_final(const Grid &g, bool helm, hipStream_t st) {
+void launch_diff_temp(const Grid &g, const double *e, hipStream_t st) {
   const dim3 blk = cell_block(g);
-  if (g.sd == 3) {
-    if (helm) k_diff_final<3, true><<<diff_grid(g), blk, 0, st>>>(g);
-    else k_diff_final<3, false><<<diff_grid(g), blk, 0, st>>>(g);
-  } else {
-    if (helm) k_diff_final<2, true><<<diff_grid(g), blk, 0, st>>>(g);
-    else k_diff_final<2, false><<<diff_grid(g), blk, 0, st>>>(g);
-  }
+  if (g.sd == 3) k_diff_temp<3><<<diff_grid(g), blk, 0, st>>>(g, e);
+  else k_diff_temp<2><<<diff_grid(g), blk, 0, st>>>(g, e);
+}
+
+void launch_diff_final(const Grid &g, const double *es, hipStream_t st) {
+  const dim3 blk = cell_block(g);
+  if (g.sd == 3) k_diff_final<3><<<diff_grid(g), blk, 0, st>>>(g, es);
+  else k_diff_final<2><<<diff_grid(g), blk, 0, st>>>(g, es);
 }
 
 void launch_parabolic(const Grid &g, double inv_dl2, hipStream_t st) {

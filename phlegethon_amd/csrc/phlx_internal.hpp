@@ -71,11 +71,13 @@ void launch_stream_copy(const void *src, void *dst, long long n16, hipStream_t s
 void launch_shock_flags(const Grid &g, hipStream_t st);
 
 // THERMAL_DIFFUSION_STS (phlx_diffusion.hip)
-void launch_diff_t_from_p(const Grid &g, hipStream_t st);
-void launch_diff_stage(const Grid &g, bool first, double mu, double nu, double c0, double hm,
-                       double hg, hipStream_t st);
-void launch_diff_temp(const Grid &g, bool helm, hipStream_t st);
-void launch_diff_final(const Grid &g, bool helm, hipStream_t st);
+// forms of a stage: the first / a middle one with T from g.tdiff, from p, from
+// e_jm1 (ideal gas), and the ideal gas' last
+enum { DIFF_FIRST_ARRAY, DIFF_FIRST_P, DIFF_ARRAY, DIFF_E, DIFF_LAST_E };
+void launch_diff_stage(const Grid &g, int form, const double *ejm1, const double *ejm2, double *ej,
+                       double mu, double nu, double c0, double hm, double hg, hipStream_t st);
+void launch_diff_temp(const Grid &g, const double *e, hipStream_t st);
+void launch_diff_final(const Grid &g, const double *es, hipStream_t st);
 void launch_parabolic(const Grid &g, double inv_dl2, hipStream_t st);
 
 // Helmholtz EoS (phlx_helm.hip)

@@ -1032,13 +1032,6 @@ __device__ __forceinline__ void xcd_cell_block(int nbx, int nby, int nk, int &bx
   by = (int)(t / (unsigned)nbx);
 }
 
-// Blocks are dealt round-robin to the 8 XCDs, each with its own L2: block id's
-// place in an order in which every XCD takes one contiguous range of 0 .. n-1.
-__device__ __forceinline__ unsigned xcd_contiguous(unsigned id, unsigned n) {
-  const unsigned x = id & 7u, q = n >> 3, r = n & 7u;
-  return x * q + min(x, r) + (id >> 3);
-}
-
 // ---------------------------------------------------------------- update
 // One thread per cell: state0 rebuild (first stage), flux divergence,
 // gravity / heating sources, RK combine, b_cc from the updated faces,
