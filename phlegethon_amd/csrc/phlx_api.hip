@@ -695,7 +695,9 @@ static bool use_fused_sweep(const phlx_ctx *ctx) {
   // 1705, 256^3 mixed 7880 / 7230), as the ideal one with two scalars does
   const bool mhd_too = ctx->cfg.eos == PHLX_EOS_IDEAL && g.nas == 0 && g.N >= 32768;
   const bool want = ctx->fused_sweep < 0 ? !g.mhd || mhd_too : ctx->fused_sweep != 0;
-  if (!want || !ctx->kt.sweep || g.sflat) return false;
+  if (!want || !ctx->kt.sweep) return false;
+  // shock flattening has no swept form beside the whole-stage one
+  if (g.sflat && ctx->kt.update_swept) return false;
   if (!ctx->kt.update_swept) return !(ctx->step_graph && ctx->stages % 2);
   return (!g.mhd || g.n1 % kSweepT == 0) &&
          (!ctx->kt.update_guess || ctx->kt.update_swept_guess);
@@ -1617,7 +1619,7 @@ extern "C" int phlx_diffusion_stages(phlx_ctx *ctx, int32_t *stages) {
 
 // USE_SHOCK_FLATTENING with eps_sf_make (source/source.F90:8073-8131): the
 // detector needs three ghost cells, so every axis holds at least 3 cells;
-// FP64 only.  The flag arrays are made on the first enable.
+// FP64 only.  The flag array is made on the first enable.
 extern "C" int phlx_set_shock_flattening(phlx_ctx *ctx, int32_t enable, double eps_sf) {
   if (!ctx || (enable != 0 && enable != 1)) return PHLX_E_ARG;
   Grid &g = ctx->g;
@@ -1630,16 +1632,9 @@ extern "C" int phlx_set_shock_flattening(phlx_ctx *ctx, int32_t enable, double e
   if (g.n1 < 3 || g.n2 < 3 || (g.sd == 3 && g.n3 < 3)) return PHLX_E_CONFIG;
   HIPCHK(hipSetDevice(ctx->device));
   if (!g.sf_flag) {
-    const long long e3 = (g.sd == 3) ? g.n3 + 4 : 1, f3 = (g.sd == 3) ? g.n3 + 2 : 1;
-    const size_t nd = (size_t)(g.n1 + 4) * (g.n2 + 4) * e3;
-    const size_t nfl = (size_t)(g.n1 + 2) * (g.n2 + 2) * f3;
-    unsigned char *det = nullptr, *flag = nullptr;
-    int rc = dalloc(ctx, &det, nd);
+    const long long f3 = (g.sd == 3) ? g.n3 + 2 : 1;
+    const int rc = dalloc(ctx, &g.sf_flag, (size_t)(g.n1 + 2) * (g.n2 + 2) * f3);
     if (rc) return rc;
-    rc = dalloc(ctx, &flag, nfl);
-    if (rc) return rc;
-    g.sf_det = det;
-    g.sf_flag = flag;
   }
   g.eps_sf = eps_sf;
   g.sflat = 1;

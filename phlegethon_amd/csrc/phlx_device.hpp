@@ -90,11 +90,10 @@ struct Grid {
   // GUESS_PRED: each zone's last T(rho, e) target e (NaN: none) and c_v there
   double *eprev;
   float *cvf;
-  // USE_SHOCK_FLATTENING: detector bytes on cells -2 .. n+1 and flags on
-  // cells -1 .. n of every axis (x3 only in 3D); sflat 0 = off
+  // USE_SHOCK_FLATTENING: flags on cells -1 .. n of every axis (x3 only in 3D); sflat 0 = off
   int sflat;
   double eps_sf;
-  unsigned char *sf_det, *sf_flag;
+  unsigned char *sf_flag;
   // THERMAL_DIFFUSION_STS: kappa on cells -1 .. n (one ghost layer), the
   // temperature the residual reads (temp with Helmholtz, an own array for
   // the ideal gas), RKL2 registers (two of the last stages
@@ -148,10 +147,6 @@ __device__ __forceinline__ void cell_ye_abar(const Grid &g, long long c, double 
 __device__ __forceinline__ long long sfix(const Grid &g, int i, int j, int k) {
   const int k0 = (g.sd == 3) ? 1 : 0;
   return ((long long)(k + k0) * (g.n2 + 2) + (j + 1)) * (g.n1 + 2) + (i + 1);
-}
-__device__ __forceinline__ long long sdix(const Grid &g, int i, int j, int k) {
-  const int k0 = (g.sd == 3) ? 2 : 0;
-  return ((long long)(k + k0) * (g.n2 + 4) + (j + 2)) * (g.n1 + 4) + (i + 2);
 }
 
 // Map a cell-centred index along axis a into the interior.  side = -1/+1

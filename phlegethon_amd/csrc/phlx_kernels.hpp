@@ -1600,12 +1600,17 @@ __global__ void __launch_bounds__(256) k_divb(Grid g) {
 // ~10 us (101 x 93 FP64: 36 -> 22 us, 256^2 mixed 31 -> 20), and a 3D one reads
 // and writes U once less (384^3 LHLLC: FP64 12.5 -> 10.25 ms per step, mixed
 // 6.14 -> 5.89, where the mixed pass is bound by its face solves).
+// SF (FP64 whole stages): shock flattening, the flags staged beside the cells:
+// 133 x 120 x 97 224 -> 146 us per stage against the split sweeps and update,
+// 256^3 1800 -> 1117.
 // Last tiles past n1 or n2 mask their missing columns.
 template <int D>
 struct SweepDir {
   static constexpr int value = D;
 };
-// waves per SIMD the register allocation aims at (FP64; the FP32 sweeps)
+// waves per SIMD the register allocation aims at (FP64; the FP32 sweeps).  With
+// shock flattening and no scalars 3, for 8 spilled registers (256^3: 1210 ->
+// 1080 us per stage, 133 x 120 x 97 152 -> 144); two scalars would spill 127.
 #ifndef PHLX_SWEEP_WAVES
 #define PHLX_SWEEP_WAVES 2
 #endif
@@ -1613,15 +1618,17 @@ struct SweepDir {
 #define PHLX_SWEEP_WAVES_MX 2
 #endif
 
-template <int SD, int NAS, bool MHD, int EK, bool MIX, bool FUSE>
+template <int SD, int NAS, bool MHD, int EK, bool MIX, bool FUSE, bool SF = false>
 __global__ void __launch_bounds__(256)
-    __attribute__((amdgpu_waves_per_eu(MIX ? PHLX_SWEEP_WAVES_MX : PHLX_SWEEP_WAVES)))
+    __attribute__((amdgpu_waves_per_eu(
+        MIX ? PHLX_SWEEP_WAVES_MX : (SF && NAS == 0) ? 3 : PHLX_SWEEP_WAVES)))
     k_sweep(Grid g, int first, int last, int fin, double a1, double a2, double c3, int kc) {
   constexpr int NV = SD + 2 + NAS, IE = SD + 1, IA = SD + 2;
   constexpr bool GAM = EK == EK_FASTEOS;
   static_assert(EK != EK_HELM_FACE, "per-face Newton states are not staged");
   static_assert(!FUSE || (!MHD && EK == EK_IDEAL), "the stage's end without CT and EoS solve");
   static_assert(SD == 3 || FUSE, "2D stages are fused ones");
+  static_assert(!SF || (FUSE && !MIX), "shock flattening: FP64 whole stages");
   using Re = typename std::conditional<MIX, float, double>::type;
   constexpr int TX = kSweepT, TY = kSweepTy;     // cells per tile
   constexpr int W = TX + 4, WW = W * (TY + 4);   // LDS row, cells per variable
@@ -1636,6 +1643,7 @@ __global__ void __launch_bounds__(256)
   __shared__ Re tile[(DB ? 2 : 1) * NC * WW];
   __shared__ Re f1[NV * NF1];  // x1 faces: [v][row b][face a = 0..16]
   __shared__ Re f2[NV * NF2];  // x2 faces: [v][face b = 0..15][column a]
+  __shared__ unsigned char flat[SF ? (DB ? 2 : 1) * WW : 1];  // shock-flattening flags
   const int tid = threadIdx.x;
   const int ntx = (g.n1 + TX - 1) / TX;
   // FP32 rows of 16 are half a line and share it, and their halo, with the
@@ -1678,9 +1686,11 @@ __global__ void __launch_bounds__(256)
   // has no column; it takes the tile's upper x1 faces)
   const bool own = (tid >> 4) < TY;
   auto plane = [&](int kk) { return DB ? tile + (kk & 1) * NC * WW : tile; };
+  auto flags = [&](int kk) { return DB ? flat + (kk & 1) * WW : flat; };
 
   struct Cell {
     Re q[NV], b[3], ga[2];
+    int fl;
   };
   // cells past n1 + 1 and n2 + 1 (partial last tiles) are read as cell
   // n1 + 1 and row n2 + 1: no face inside the grid reaches them, and the
@@ -1689,6 +1699,12 @@ __global__ void __launch_bounds__(256)
     ii = min(ii, g.n1 + 1);
     jj = min(jj, g.n2 + 1);
     const bool in = ii >= 0 && ii < g.n1 && jj >= 0 && jj < g.n2 && kk >= 0 && kk < g.n3;
+    if constexpr (SF) {
+      // flags cover the cells beside a face of the grid (-1 .. n); the others
+      // are no face's neighbour
+      const int fi = min(max(ii, -1), g.n1), fj = min(max(jj, -1), g.n2);
+      c.fl = g.sf_flag[sfix(g, fi, fj, SD == 3 ? min(max(kk, -1), g.n3) : kk)];
+    }
     if constexpr (MIX) {
       if (__all(in))
         load_cell_f<SD, NV, MHD, GAM, true>(g, ii, jj, kk, c.q, c.b, c.ga);
@@ -1701,7 +1717,9 @@ __global__ void __launch_bounds__(256)
         load_cell<SD, NV, MHD, GAM, false>(g, ii, jj, kk, c.q, c.b, c.ga);
     }
   };
-  auto put = [&](Re *t, int cell, const Cell &c) {
+  auto put = [&](int kk, int cell, const Cell &c) {
+    Re *const t = plane(kk);
+    if (SF) flags(kk)[cell] = (unsigned char)c.fl;
 #pragma unroll
     for (int v = 0; v < NV; v++) t[v * WW + cell] = c.q[v];
     if (MHD) {
@@ -1719,31 +1737,42 @@ __global__ void __launch_bounds__(256)
     else
       face_states<false>(g.recon, lim, w, st, qL, qR);
   };
-  auto edges = [&](bool lim, Re qm, Re q0, Re qp, Re &l, Re &r) {
+  auto edges = [&](bool lim, Re qm, Re q0, Re qp, Re &l, Re &r, int fl = 0) {
     if constexpr (MIX)
       cell_edges_mx(g.recon, lim, qm, q0, qp, l, r);
     else
-      cell_edges(g.recon, lim, qm, q0, qp, l, r);
+      cell_edges(SF && fl ? REC_LIM2ND : g.recon, lim, qm, q0, qp, l, r);
   };
   auto solve = [&](auto dirc, int ii, int jj, int kk, Re *qL, Re *qR, Re *bL, Re *bR, Re *gL,
-                   Re *gR, Re *Fo) {
+                   Re *gR, Re *Fo, bool hll) {
     constexpr int DIR = decltype(dirc)::value;
     if constexpr (MIX)
       flux_face_mx<DIR, SD, NAS, MHD, GAM, true>(g, ii, jj, kk, qL, qR, bL, bR, gL, gR, Fo);
     else
-      flux_face<DIR, SD, NAS, MHD, EK, false, true>(g, ii, jj, kk, qL, qR, bL, bR, gL, gR, 0.0,
-                                                    false, Fo);
+      flux_face<DIR, SD, NAS, MHD, EK, SF, true>(g, ii, jj, kk, qL, qR, bL, bR, gL, gR, 0.0, hll,
+                                                 Fo);
   };
   // the in-plane face (DIR 0: lower x1 face of tile cell (fa, fb); DIR 1:
   // lower x2 face) from the LDS stencil, its fluxes into the LDS face array
-  auto plane_face = [&](auto dirc, const Re *t, int fa, int fb, int kk) {
+  auto plane_face = [&](auto dirc, int fa, int fb, int kk) {
+    const Re *const t = plane(kk);
     constexpr int DIR = decltype(dirc)::value;
     const int base = DIR == 0 ? (fb + 2) * W + fa : fb * W + fa + 2;
     constexpr int st = DIR == 0 ? 1 : W;
     Re qL[NV], qR[NV], bL[3] = {0, 0, 0}, bR[3] = {0, 0, 0}, gL[2] = {0, 0}, gR[2] = {0, 0};
     Re Fo[NV];
+    bool hll = false;
+    if constexpr (SF) {
+      // flattened cells take the LIM2ND slope, the faces beside them HLL
+      const bool flm = flags(kk)[base + st] != 0, flc = flags(kk)[base + 2 * st] != 0;
+      hll = flm || flc;
 #pragma unroll
-    for (int v = 0; v < NV; v++) states(v > IE, &t[v * WW + base], st, qL[v], qR[v]);
+      for (int v = 0; v < NV; v++)
+        face_states_sf<false>(g.recon, v > IE, &t[v * WW + base], st, flm, flc, qL[v], qR[v]);
+    } else {
+#pragma unroll
+      for (int v = 0; v < NV; v++) states(v > IE, &t[v * WW + base], st, qL[v], qR[v]);
+    }
     if (MHD) {
 #pragma unroll
       for (int c = 0; c < SD; c++) {
@@ -1755,7 +1784,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int c = 0; c < 2; c++) states(false, &t[(OG + c) * WW + base], st, gL[c], gR[c]);
     }
-    solve(dirc, i0 + fa, j0 + fb, kk, qL, qR, bL, bR, gL, gR, Fo);
+    solve(dirc, i0 + fa, j0 + fb, kk, qL, qR, bL, bR, gL, gR, Fo, hll);
     Re *dst = DIR == 0 ? f1 + fb * (TX + 1) + fa : f2 + fb * TX + fa;
 #pragma unroll
     for (int v = 0; v < NV; v++) {
@@ -1769,6 +1798,7 @@ __global__ void __launch_bounds__(256)
   // past n2 (a last, partial tile) only stages its ghost cells.
   Cell nxt;
   Re rq[NV], rb[3] = {0, 0, 0}, rg[2] = {0, 0}, F3m[NV];
+  int flk = 0;  // the flag of this column's cell k
   if (own) {
     const int a = tid & (TX - 1), b = tid >> 4, i = i0 + a, j = j0 + b;
     Cell cA, cB, cC;
@@ -1783,8 +1813,8 @@ __global__ void __launch_bounds__(256)
     Re l, qL[NV], qR[NV], bL[3] = {0, 0, 0}, bR[3] = {0, 0, 0}, gL[2] = {0, 0}, gR[2] = {0, 0};
 #pragma unroll
     for (int v = 0; v < NV; v++) {
-      edges(v > IE, cA.q[v], cB.q[v], cC.q[v], l, qL[v]);
-      edges(v > IE, cB.q[v], cC.q[v], nxt.q[v], qR[v], rq[v]);
+      edges(v > IE, cA.q[v], cB.q[v], cC.q[v], l, qL[v], cB.fl);
+      edges(v > IE, cB.q[v], cC.q[v], nxt.q[v], qR[v], rq[v], cC.fl);
     }
     if (MHD) {
 #pragma unroll
@@ -1801,8 +1831,10 @@ __global__ void __launch_bounds__(256)
       }
     }
     if constexpr (SD == 3)
-      if (i < g.n1 && j < g.n2) solve(SweepDir<2>{}, i, j, k0, qL, qR, bL, bR, gL, gR, F3m);
-    put(plane(k0), (b + 2) * W + a + 2, cC);
+      if (i < g.n1 && j < g.n2)
+        solve(SweepDir<2>{}, i, j, k0, qL, qR, bL, bR, gL, gR, F3m, SF && (cB.fl || cC.fl));
+    if (SF) flk = cC.fl;
+    put(k0, (b + 2) * W + a + 2, cC);
   }
 
   // the RK buffers of k_update: the FP64 path saves state0 in U0 and carries
@@ -1845,14 +1877,14 @@ __global__ void __launch_bounds__(256)
     // double tile: cell k+1 of this column into plane k+1's tile (whose
     // last reads, of plane k-1, are behind the previous iteration's second
     // barrier); the single tile takes it after this plane's reads
-    if (DB && lb < TY) put(plane(k + 1), mine, nxt);
+    if (DB && lb < TY) put(k + 1, mine, nxt);
     // the halo of plane k (its interior is staged already), loaded a plane
     // ahead where the registers allow it, so that no plane starts with a wait
     // for memory (256^3 MHD: FP64 2378 -> 2268 us, mixed 1301 -> 1244; 192 x 256 x
     // 192 Helmholtz 1272 -> 1255; with MHD and gammas, over its registers
     // already, 1885 -> 2190 at 256^3 mixed)
     if (!kHaloAhead && halo) load(i0 + ha, j0 + hb, k, h);
-    if (halo) put(tk, hcell, h);
+    if (halo) put(k, hcell, h);
     __syncthreads();
     if (SD == 3 && kHaloAhead && halo && k + 1 < k1) {
       int hx = i0 + ha, hy = j0 + hb;
@@ -1864,9 +1896,9 @@ __global__ void __launch_bounds__(256)
     // the lower face of row lb (16 faces: row 15's is the tile's upper face)
     {
       const int fa = lb < TY ? la : TX, fb = lb < TY ? lb : la;
-      if (fb < TY && i0 + fa <= g.n1 && j0 + fb < g.n2) plane_face(SweepDir<0>{}, tk, fa, fb, k);
+      if (fb < TY && i0 + fa <= g.n1 && j0 + fb < g.n2) plane_face(SweepDir<0>{}, fa, fb, k);
     }
-    if (li < g.n1 && lj <= g.n2) plane_face(SweepDir<1>{}, tk, la, lb, k);
+    if (li < g.n1 && lj <= g.n2) plane_face(SweepDir<1>{}, la, lb, k);
     // cell k+2 of this column, in flight across the barrier
     Cell cp;
     if constexpr (SD == 3)
@@ -1882,7 +1914,7 @@ __global__ void __launch_bounds__(256)
 #pragma unroll
       for (int v = 0; v < NV; v++) {
         qL[v] = rq[v];
-        edges(v > IE, qm[v * WW], DB ? q1[v * WW] : nxt.q[v], cp.q[v], qR[v], rq[v]);
+        edges(v > IE, qm[v * WW], DB ? q1[v * WW] : nxt.q[v], cp.q[v], qR[v], rq[v], nxt.fl);
       }
       if (MHD) {
 #pragma unroll
@@ -1903,8 +1935,10 @@ __global__ void __launch_bounds__(256)
       }
       // single tile: plane k's reads are done (this thread's own cell k was
       // the last, just above), so cell k+1 takes its slot
+      const bool hll3 = SF && (flk || nxt.fl);
       if (SD == 3) {
-        if (!DB && k + 1 < k1) put(tk, mine, nxt);
+        if (!DB && k + 1 < k1) put(k, mine, nxt);
+        if (SF) flk = nxt.fl;
         nxt = cp;
       }
       if (col) {
@@ -1949,7 +1983,8 @@ __global__ void __launch_bounds__(256)
             S[v] = s_buf[v * N + c];
           }
         }
-        if constexpr (SD == 3) solve(SweepDir<2>{}, li, lj, k + 1, qL, qR, bL, bR, gL, gR, F3p);
+        if constexpr (SD == 3)
+          solve(SweepDir<2>{}, li, lj, k + 1, qL, qR, bL, bR, gL, gR, F3p, hll3);
         // divergence (x1 overwrites, x2 and x3 accumulate), sources, RK
 #pragma unroll
         for (int v = 0; v < NV; v++) {
@@ -2014,94 +2049,76 @@ __global__ void __launch_bounds__(256)
 }
 
 // ------------------------------------------------------- shock flattening
-// USE_SHOCK_FLATTENING detector (source/source.F90:8073-8131).  k_sf_detect:
-// one thread per cell of -2 .. n+1 on each axis marks a cell whose summed
-// relative pressure jump sum_d |p(c+e_d) - p(c-e_d)| / p(c) exceeds eps_sf;
-// k_sf_dilate: a cell of -1 .. n is flattened when a marked cell lies in
-// its 3^sdims neighbourhood (the reference's scatter written as a gather, so
-// no flag array has to be cleared first).  Ghost pressures come through the
-// boundary map (pressure carries no sign flip); with USE_WB the full
-// pressure is the stored deviation plus the mapped row's equilibrium.
+// USE_SHOCK_FLATTENING flags (source/source.F90:8073-8131) of the cells
+// -1 .. n.  A cell of -2 .. n+1 is marked when its summed relative pressure jump
+// sum_d |p(c+e_d) - p(c-e_d)| / p(c) exceeds eps_sf; a cell is flattened when
+// a marked one lies in its 3^sdims neighbourhood (the reference's scatter
+// written as a gather, so no flag array has to be cleared first).  Ghost
+// pressures come through the boundary map (pressure carries no sign flip), row
+// and plane once per wave; with USE_WB the full pressure is the stored deviation
+// plus the mapped row's equilibrium.
+//
+// A block marches 64 x 16 cells along x3, a wave per row: a plane's pressures go
+// through LDS, the next one is in flight, the marks of a row are one ballot word
+// and the flags the OR of nine words and their shifts (60 x 12 flags per plane).
+// One launch and 8 bytes of pressure per cell: 133 x 120 x 97 27.7 -> 20.7 us,
+// 256^3 191 -> 89 against a byte per mark between two launches (now bound by
+// the round trip of each plane: 140 MB would take 30).
+constexpr int kSfRows = 16, kSfW = 60, kSfH = kSfRows - 4;
 template <int SD>
-__device__ __forceinline__ double sf_pressure(const Grid &g, int i, int j, int k) {
+__global__ void __launch_bounds__(64 * kSfRows) k_sf_flags(Grid g, int kc) {
+  if (!g.sc->active) return;
+  __shared__ double P[2][kSfRows * 64];
+  __shared__ unsigned long long mark[2][kSfRows];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int row = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // cells past the ghosts repeat the last one; no flag is taken from them
+  const int i = kSfW * (int)blockIdx.x - 3 + lane, j = kSfH * (int)blockIdx.y - 3 + row;
+  const int k0 = SD == 3 ? (int)blockIdx.z * kc - 1 : 0;
+  const int k1 = SD == 3 ? min(k0 + kc, g.n3 + 1) : 1;
   int s;
-  const int mi = map_axis(g, 0, i, g.n1, s);
-  const int mj = map_axis(g, 1, j, g.n2, s);
-  const int mk = (SD == 3) ? map_axis(g, 2, k, g.n3, s) : k;
-  const double p = g.P[(long long)(SD + 1) * g.N + cix(g, mi, mj, mk)];
-  if (!g.wb) return p;
-  const double e = g.eq_p_cc[mj];
-  return (p - e) + e;
-}
-
-// The detector of cell (i, j, k) from the full pressures of its stencil.
-template <int SD>
-__device__ __forceinline__ unsigned char sf_test(const Grid &g, double pc, double pim,
-                                                 double pip, double pjm, double pjp, double pkm,
-                                                 double pkp) {
-  const double dj = fabs(pjp - pjm), di = fabs(pip - pim);
-  double tmp;
-  if (SD == 3)
-    tmp = (fabs(pkp - pkm) + dj + di) / pc;
-  else
-    tmp = (dj + di) / pc;
-  return (tmp > g.eps_sf) ? 1 : 0;
-}
-
-template <int SD>
-__global__ void __launch_bounds__(256) k_sf_detect(Grid g) {
-  if (!g.sc->active) return;
-  int a, b;
-  if (!plane_coords(g.n1 + 4, g.n2 + 4, a, b)) return;
-  const int i = a - 2, j = b - 2, k = (SD == 3) ? (int)blockIdx.z - 2 : 0;
-  const bool inside = i >= 1 && i <= g.n1 - 2 && j >= 1 && j <= g.n2 - 2 &&
-                      (SD == 2 || (k >= 1 && k <= g.n3 - 2));
-  unsigned char d;
-  if (__all(inside)) {
-    // every stencil cell of the wave is interior: direct loads
-    const double *p = g.P + (long long)(SD + 1) * g.N;
-    const long long c = cix(g, i, j, k), sj = g.n1, sk = (long long)g.n1 * g.n2;
-    double pc = p[c], pim = p[c - 1], pip = p[c + 1], pjm = p[c - sj], pjp = p[c + sj];
-    double pkm = 0.0, pkp = 0.0;
-    if (SD == 3) {
-      pkm = p[c - sk];
-      pkp = p[c + sk];
-    }
-    if (g.wb) {
-      const double e = g.eq_p_cc[j], em = g.eq_p_cc[j - 1], ep = g.eq_p_cc[j + 1];
-      pc = (pc - e) + e;
-      pim = (pim - e) + e;
-      pip = (pip - e) + e;
-      pkm = (pkm - e) + e;
-      pkp = (pkp - e) + e;
-      pjm = (pjm - em) + em;
-      pjp = (pjp - ep) + ep;
-    }
-    d = sf_test<SD>(g, pc, pim, pip, pjm, pjp, pkm, pkp);
-  } else {
-    d = sf_test<SD>(g, sf_pressure<SD>(g, i, j, k), sf_pressure<SD>(g, i - 1, j, k),
-                    sf_pressure<SD>(g, i + 1, j, k), sf_pressure<SD>(g, i, j - 1, k),
-                    sf_pressure<SD>(g, i, j + 1, k),
-                    SD == 3 ? sf_pressure<SD>(g, i, j, k - 1) : 0.0,
-                    SD == 3 ? sf_pressure<SD>(g, i, j, k + 1) : 0.0);
+  const int ic = map_axis(g, 0, min(i, g.n1 + 2), g.n1, s);
+  const int jc = map_axis(g, 1, min(j, g.n2 + 2), g.n2, s);
+  const double *p = g.P + (long long)(SD + 1) * g.N;
+  const double eq = g.wb ? g.eq_p_cc[jc] : 0.0;
+  auto at = [&](int kk) { return p[cix(g, ic, jc, SD == 3 ? map_axis(g, 2, kk, g.n3, s) : 0)]; };
+  auto full = [&](double v) { return g.wb ? (v - eq) + eq : v; };
+  const bool out = lane >= 2 && lane < 2 + kSfW && row >= 2 && row < 2 + kSfH && i <= g.n1 &&
+                   j <= g.n2;
+  // neighbours in the tile (an edge cell reads itself: its mark is not used)
+  const int xm = lane > 0 ? tid - 1 : tid, xp = lane < 63 ? tid + 1 : tid;
+  const int ym = row > 0 ? tid - 64 : tid, yp = row < kSfRows - 1 ? tid + 64 : tid;
+  int kk = SD == 3 ? k0 - 1 : 0;
+  double pm = 0.0, pc = full(at(kk)), pn = 0.0;
+  if (SD == 3) {
+    pm = full(at(kk - 1));
+    pn = at(kk + 1);
   }
-  g.sf_det[sdix(g, i, j, k)] = d;
-}
-
-template <int SD>
-__global__ void __launch_bounds__(256) k_sf_dilate(Grid g) {
-  if (!g.sc->active) return;
-  int a, b;
-  if (!plane_coords(g.n1 + 2, g.n2 + 2, a, b)) return;
-  const int i = a - 1, j = b - 1, k = (SD == 3) ? (int)blockIdx.z - 1 : 0;
-  int any = 0;
-#pragma unroll
-  for (int dk = (SD == 3 ? -1 : 0); dk <= (SD == 3 ? 1 : 0); dk++)
-#pragma unroll
-    for (int dj = -1; dj <= 1; dj++)
-#pragma unroll
-      for (int di = -1; di <= 1; di++) any |= g.sf_det[sdix(g, i + di, j + dj, k + dk)];
-  g.sf_flag[sfix(g, i, j, k)] = (unsigned char)(any != 0);
+  unsigned long long w = 0, x0 = 0, x1 = 0;
+  // marks of plane kk, flags of plane kk - 2 (3D) or kk - 1 (2D)
+  for (int b = 0; kk <= k1 + (SD == 3 ? 1 : 0); kk++, b ^= 1) {
+    P[b][tid] = pc;
+    if (lane == 0) mark[b][row] = w;
+    __syncthreads();
+    // plane kk + 1, loaded an iteration ago; kk + 2 follows
+    const double pp = full(pn);
+    if (SD == 3 && kk < k1) pn = at(kk + 2);
+    const double di = fabs(P[b][xp] - P[b][xm]), dj = fabs(P[b][yp] - P[b][ym]);
+    const double tmp = (SD == 3) ? (fabs(pp - pm) + dj + di) / pc : (dj + di) / pc;
+    const unsigned long long wk = __ballot(tmp > g.eps_sf);
+    if (row > 0 && row < kSfRows - 1) {
+      const unsigned long long r = mark[b][row - 1] | w | mark[b][row + 1];
+      const unsigned long long x = r | r << 1 | r >> 1;
+      const int k = kk - (SD == 3 ? 2 : 1);
+      if (out && k >= k0)
+        g.sf_flag[sfix(g, i, j, k)] = (unsigned char)((x0 | x1 | x) >> lane & 1);
+      x0 = x1;
+      x1 = x;
+    }
+    w = wk;
+    pm = pc;
+    pc = pp;
+  }
 }
 
 // -------------------------------------------------------------- launchers
@@ -2285,6 +2302,13 @@ struct Kern {
     if constexpr (kSwept) {
       int kc;
       const dim3 grd = sweep_grid(g, kc);
+      if constexpr (kWhole && !MIX) {
+        if (g.sflat) {
+          k_sweep<SD, NAS, MHD, EK, MIX, true, true>
+              <<<grd, 256, 0, st>>>(g, first, last, fin, a1, a2, c3, kc);
+          return (int)(grd.x * grd.y);
+        }
+      }
       k_sweep<SD, NAS, MHD, EK, MIX, kWhole>
           <<<grd, 256, 0, st>>>(g, first, last, fin, a1, a2, c3, kc);
       return (int)(grd.x * grd.y);
