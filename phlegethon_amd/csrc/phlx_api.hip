@@ -259,8 +259,8 @@ extern "C" int phlx_create(const phlx_config *cfg, phlx_ctx **out) {
       e |= dalloc(ctx, &g.sgn[d], (size_t)g.nf[d]);
     }
     const size_t n1 = g.n1, n2 = g.n2, n3 = g.n3;
-    e |= dalloc(ctx, &g.cor[2], (n1 + 1) * (n2 + 1) * n3);
     if (g.sd == 3) {
+      e |= dalloc(ctx, &g.cor[2], (n1 + 1) * (n2 + 1) * n3);
       e |= dalloc(ctx, &g.cor[0], n1 * (n2 + 1) * (n3 + 1));
       e |= dalloc(ctx, &g.cor[1], (n1 + 1) * n2 * (n3 + 1));
     }
@@ -636,9 +636,12 @@ extern "C" int phlx_ct(phlx_ctx *ctx, int32_t irk, double a1, double a2, double 
     mode = irk == 0 ? FACEB_RK2_1 : FACEB_RK2_2;
   }
   ProfRec r;
-  int on = kbegin(ctx, KID_CORNER, r);
-  ctx->kt.corner(ctx->g, ctx->stream);
-  kend(ctx, on, r);
+  int on;
+  if (ctx->kt.corner) {
+    on = kbegin(ctx, KID_CORNER, r);
+    ctx->kt.corner(ctx->g, ctx->stream);
+    kend(ctx, on, r);
+  }
   on = kbegin(ctx, KID_FACEB, r);
   ctx->kt.faceb(ctx->g, mode, a1, a2, a3, ctx->stream);
   kend(ctx, on, r);
@@ -691,15 +694,17 @@ static bool use_fused_sweep(const phlx_ctx *ctx) {
   // measured on MI355X, us per step, fused / split: without MHD always the
   // faster form (384^3 hydro FP64 9800 / 14400, mixed 5650 / 7650); ideal MHD
   // from 32^3 (32^3 FP64 81 / 92, mixed 69 / 87; 256^3 7055 / 7770, 4240 /
-  // 4345); MHD with the tabulated EoS spills and is slower (128^3 FP64 2090 /
+  // 4345), in 2D at any size (64 x 48 FP64 RK3 60 / 74, 1024^2 332 / 413, mixed
+  // 2000 x 1500 641 / 751); MHD with the tabulated EoS spills and is slower (128^3 FP64 2090 /
   // 1705, 256^3 mixed 7880 / 7230), as the ideal one with two scalars does
-  const bool mhd_too = ctx->cfg.eos == PHLX_EOS_IDEAL && g.nas == 0 && g.N >= 32768;
+  const bool mhd_too =
+      ctx->cfg.eos == PHLX_EOS_IDEAL && g.nas == 0 && (g.sd == 2 || g.N >= 32768);
   const bool want = ctx->fused_sweep < 0 ? !g.mhd || mhd_too : ctx->fused_sweep != 0;
   if (!want || !ctx->kt.sweep) return false;
   // shock flattening has no swept form beside the whole-stage one
   if (g.sflat && ctx->kt.update_swept) return false;
   if (!ctx->kt.update_swept) return !(ctx->step_graph && ctx->stages % 2);
-  return (!g.mhd || g.n1 % kSweepT == 0) &&
+  return (!g.mhd || g.sd == 2 || g.n1 % kSweepT == 0) &&
          (!ctx->kt.update_guess || ctx->kt.update_swept_guess);
 }
 

@@ -758,10 +758,8 @@ __device__ __forceinline__ double corner_emf(double eS, double eW, double eN, do
   return 0.25 * (eS + eW + eN + eE + dS - dN + dW - dE);
 }
 
-// One thread per grid node (i,j,k) in [0,n1]x[0,n2]x[0,n3]: the three edge
-// EMFs whose lower end is that node (F32: FP32 face, cell and edge EMFs, FP64
-// arithmetic).
-// Ghosts: an edge reads face and cell EMFs one position outside the grid.  The
+// In-plane neighbourhood of the grid node (i, j), i in [0,n1], j in [0,n2].
+// An edge reads face and cell EMFs one position outside the grid.  The
 // EMF halo copy and EMF boundary conditions (source/source.F90:11370-11964)
 // wrap them or take the wall's own, negated beyond a reflecting wall since the
 // component is tangential to it; a cell EMF -(v x B) there, of a mirrored state
@@ -769,42 +767,78 @@ __device__ __forceinline__ double corner_emf(double eS, double eW, double eN, do
 // exactly one axis-a factor, and IEEE negation commutes with rounding), and one
 // position out both mirror to the wall's own index.  So one mapped index and
 // one sign per axis side serve every load, and the loads have no branch
-// between them (with a map per load, 36 a node, the kernel was bound by index
+// between them (with a map per load, 36 a node, the 3D kernel was bound by index
 // arithmetic: mixed 0.67 VALU-busy at half the copy kernel's rate).
-template <int SD, bool F32>
-__global__ void __launch_bounds__(256) k_corner(Grid g) {
+// F32: FP32 face, cell and edge EMFs, FP64 arithmetic.
+template <bool F32>
+struct CtNode {
   using Re = typename std::conditional<F32, float, double>::type;
   using Bits = typename std::conditional<F32, unsigned int, unsigned long long>::type;
-  constexpr Bits kSign = (Bits)1 << (8 * sizeof(Re) - 1);
-  if (!g.sc->active) return;
-  const int n1 = g.n1, n2 = g.n2, n3 = g.n3, k = blockIdx.z;
-  int i, j;
-  if (!plane_coords(n1 + 1, n2 + 1, i, j)) return;
+  static constexpr Bits kSign = (Bits)1 << (8 * sizeof(Re) - 1);
+  Bits xm, xp, ym, yp;
+  // x1 faces (i, j) / (i, j-1), x2 faces (i, j) / (i-1, j), cells and x3 faces
+  // of the four columns around the node
+  unsigned f1p, f1m, f2p, f2m, cpp, cmp, cpm, cmm;
   // position c (-1 .. n) of axis a in the grid, and the sign of what it holds
-  auto map = [&](int a, int c, int n, Bits &flip) {
+  static __device__ __forceinline__ int map(const Grid &g, int a, int c, int n, Bits &flip) {
     flip = 0;
     if (c >= 0 && c < n) return c;
     const int side = c < 0 ? 0 : 1, bc = g.bc[2 * a + side];
     if (bc == BC_PERIODIC) return side ? c - n : c + n;
     if (bc == BC_REFLECTIVE) flip = kSign;
     return side ? n - 1 : 0;
-  };
-  auto load = [](const Re *p, unsigned o, Bits flip) {
+  }
+  static __device__ __forceinline__ double load(const Re *p, unsigned o, Bits flip) {
     return (double)__builtin_bit_cast(Re, __builtin_bit_cast(Bits, p[o]) ^ flip);
-  };
-  Bits xm, xp, ym, yp;
-  const int im = map(0, i - 1, n1, xm), ip = map(0, i, n1, xp);
-  const int jm = map(1, j - 1, n2, ym), jp = map(1, j, n2, yp);
-  // in-plane offsets: x1 faces (i, j) / (i, j-1), x2 faces (i, j) / (i-1, j),
-  // cells and x3 faces of the four columns around the node
-  const unsigned f1p = jp * (n1 + 1) + i, f1m = jm * (n1 + 1) + i;
-  const unsigned f2p = j * n1 + ip, f2m = j * n1 + im;
-  const unsigned cpp = jp * n1 + ip, cmp = jp * n1 + im, cpm = jm * n1 + ip, cmm = jm * n1 + im;
+  }
+  __device__ __forceinline__ CtNode(const Grid &g, int i, int j) {
+    const int n1 = g.n1;
+    const int im = map(g, 0, i - 1, n1, xm), ip = map(g, 0, i, n1, xp);
+    const int jm = map(g, 1, j - 1, g.n2, ym), jp = map(g, 1, j, g.n2, yp);
+    f1p = jp * (n1 + 1) + i;
+    f1m = jm * (n1 + 1) + i;
+    f2p = j * n1 + ip;
+    f2m = j * n1 + im;
+    cpp = jp * n1 + ip;
+    cmp = jp * n1 + im;
+    cpm = jm * n1 + ip;
+    cmm = jm * n1 + im;
+  }
+  // the x3-edge of plane k (emfx3_cor, source/source.F90:11966-12027)
+  __device__ __forceinline__ double edge3(const Grid &g, int k) const {
+    const long long s1 = (long long)(g.n1 + 1) * g.n2, s2 = (long long)g.n1 * (g.n2 + 1),
+                    s3 = (long long)g.n1 * g.n2;
+    const Re *const z1 = (F32 ? (const Re *)g.emff[0] : (const Re *)g.emf[0]) + g.nf[0] + k * s1;
+    const Re *const z2 = (F32 ? (const Re *)g.emff[1] : (const Re *)g.emf[1]) + g.nf[1] + k * s2;
+    const Re *const zc = (F32 ? (const Re *)g.ecellf : (const Re *)g.ecell) + 2 * g.N + k * s3;
+    const signed char *const g1 = g.sgn[0] + k * s1, *const g2 = g.sgn[1] + k * s2;
+    const double eN = load(z1, f1p, yp), eS = load(z1, f1m, ym);
+    const double eE = load(z2, f2p, xp), eW = load(z2, f2m, xm);
+    const double sN = g1[f1p], sS = g1[f1m], sE = g2[f2p], sW = g2[f2m];
+    const double eSW = load(zc, cmm, xm ^ ym), eNW = load(zc, cmp, xm ^ yp);
+    const double eNE = load(zc, cpp, xp ^ yp), eSE = load(zc, cpm, xp ^ ym);
+    return corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE);
+  }
+};
+
+// 3D: one thread per grid node (i,j,k) in [0,n1]x[0,n2]x[0,n3], the three edge
+// EMFs whose lower end is that node.
+template <bool F32>
+__global__ void __launch_bounds__(256) k_corner(Grid g) {
+  using Re = typename CtNode<F32>::Re;
+  using Bits = typename CtNode<F32>::Bits;
+  if (!g.sc->active) return;
+  const int n1 = g.n1, n2 = g.n2, n3 = g.n3, k = blockIdx.z;
+  int i, j;
+  if (!plane_coords(n1 + 1, n2 + 1, i, j)) return;
+  const CtNode<F32> o(g, i, j);
+  auto load = [](const Re *p, unsigned x, Bits flip) { return CtNode<F32>::load(p, x, flip); };
+  const auto [xm, xp, ym, yp, f1p, f1m, f2p, f2m, cpp, cmp, cpm, cmm] = o;
   const long long s1 = (long long)(n1 + 1) * n2, s2 = (long long)n1 * (n2 + 1),
                   s3 = (long long)n1 * n2;
   // planes k and k - 1 (mapped) of the x1 faces, x2 faces and cells
-  Bits zp = 0, zm = 0;
-  const int kp = SD == 3 ? map(2, k, n3, zp) : 0, km = SD == 3 ? map(2, k - 1, n3, zm) : 0;
+  Bits zp, zm;
+  const int kp = CtNode<F32>::map(g, 2, k, n3, zp), km = CtNode<F32>::map(g, 2, k - 1, n3, zm);
   const Re *const E1 = F32 ? (const Re *)g.emff[0] : (const Re *)g.emf[0];
   const Re *const E2 = F32 ? (const Re *)g.emff[1] : (const Re *)g.emf[1];
   const Re *const Ec = F32 ? (const Re *)g.ecellf : (const Re *)g.ecell;
@@ -816,39 +850,28 @@ __global__ void __launch_bounds__(256) k_corner(Grid g) {
     else
       g.cor[d][x] = e;
   };
-  if (k < n3) {  // x3-edges (emfx3_cor, source/source.F90:11966-12027)
-    const Re *const z1 = E1 + g.nf[0] + kp * s1, *const z2 = E2 + g.nf[1] + kp * s2,
-             *const zc = Ec + 2 * g.N + kp * s3;
-    const double eN = load(z1, f1p, yp), eS = load(z1, f1m, ym);
-    const double eE = load(z2, f2p, xp), eW = load(z2, f2m, xm);
-    const double sN = g1[f1p], sS = g1[f1m], sE = g2[f2p], sW = g2[f2m];
-    const double eSW = load(zc, cmm, xm ^ ym), eNW = load(zc, cmp, xm ^ yp);
-    const double eNE = load(zc, cpp, xp ^ yp), eSE = load(zc, cpm, xp ^ ym);
-    store(2, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
+  if (k < n3) store(2, o.edge3(g, k));
+  const Re *const e3 = (F32 ? (const Re *)g.emff[2] : (const Re *)g.emf[2]) + k * s3;
+  const signed char *const g3 = g.sgn[2] + k * s3;
+  if (i < n1) {  // x1-edges (emfx1_cor, source/source.F90:12050-12107)
+    const double eN = load(E2 + kp * s2, f2p, zp), eS = load(E2 + km * s2, f2p, zm);
+    const double eE = load(e3, cpp, yp), eW = load(e3, cpm, ym);
+    const double sN = g2[f2p], sS = g.sgn[1][km * s2 + f2p], sE = g3[cpp], sW = g3[cpm];
+    const Re *const cp = Ec + kp * s3, *const cm = Ec + km * s3;
+    const double eSW = load(cm, cpm, zm ^ ym), eNW = load(cp, cpm, zp ^ ym);
+    const double eNE = load(cp, cpp, zp ^ yp), eSE = load(cm, cpp, zm ^ yp);
+    // cell order around the edge: SW (j-1,k-1), NW (j-1,k), NE (j,k), SE (j,k-1)
+    store(0, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
   }
-  if constexpr (SD == 3) {
-    const Re *const e3 = (F32 ? (const Re *)g.emff[2] : (const Re *)g.emf[2]) + k * s3;
-    const signed char *const g3 = g.sgn[2] + k * s3;
-    if (i < n1) {  // x1-edges (emfx1_cor, source/source.F90:12050-12107)
-      const double eN = load(E2 + kp * s2, f2p, zp), eS = load(E2 + km * s2, f2p, zm);
-      const double eE = load(e3, cpp, yp), eW = load(e3, cpm, ym);
-      const double sN = g2[f2p], sS = g.sgn[1][km * s2 + f2p], sE = g3[cpp], sW = g3[cpm];
-      const Re *const cp = Ec + kp * s3, *const cm = Ec + km * s3;
-      const double eSW = load(cm, cpm, zm ^ ym), eNW = load(cp, cpm, zp ^ ym);
-      const double eNE = load(cp, cpp, zp ^ yp), eSE = load(cm, cpp, zm ^ yp);
-      // cell order around the edge: SW (j-1,k-1), NW (j-1,k), NE (j,k), SE (j,k-1)
-      store(0, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
-    }
-    if (j < n2) {  // x2-edges (emfx2_cor, source/source.F90:12128-12185)
-      const Re *const y3 = e3 + g.nf[2];
-      const double eN = load(y3, cpp, xp), eS = load(y3, cmp, xm);
-      const double eE = load(E1 + kp * s1, f1p, zp), eW = load(E1 + km * s1, f1p, zm);
-      const double sN = g3[cpp], sS = g3[cmp], sE = g1[f1p], sW = g.sgn[0][km * s1 + f1p];
-      const Re *const cp = Ec + g.N + kp * s3, *const cm = Ec + g.N + km * s3;
-      const double eSW = load(cm, cmp, zm ^ xm), eNW = load(cm, cpp, zm ^ xp);
-      const double eNE = load(cp, cpp, zp ^ xp), eSE = load(cp, cmp, zp ^ xm);
-      store(1, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
-    }
+  if (j < n2) {  // x2-edges (emfx2_cor, source/source.F90:12128-12185)
+    const Re *const y3 = e3 + g.nf[2];
+    const double eN = load(y3, cpp, xp), eS = load(y3, cmp, xm);
+    const double eE = load(E1 + kp * s1, f1p, zp), eW = load(E1 + km * s1, f1p, zm);
+    const double sN = g3[cpp], sS = g3[cmp], sE = g1[f1p], sW = g.sgn[0][km * s1 + f1p];
+    const Re *const cp = Ec + g.N + kp * s3, *const cm = Ec + g.N + km * s3;
+    const double eSW = load(cm, cmp, zm ^ xm), eNW = load(cm, cpp, zm ^ xp);
+    const double eNE = load(cp, cpp, zp ^ xp), eSE = load(cp, cmp, zp ^ xm);
+    store(1, corner_emf(eS, eW, eN, eE, eSW, eNW, eNE, eSE, sS, sN, sW, sE));
   }
 }
 
@@ -889,47 +912,65 @@ __device__ __forceinline__ void faceb_set(const Grid &g, int d, long long f, int
   else
     g.bf[d][f] = out;
 }
-template <int SD, bool F32>
+// an inactive first stage of RK2: the current field in both buffers
+template <int SD>
+__device__ __forceinline__ void faceb_keep(const Grid &g, int mode, int i, int j, int k) {
+  if (mode != FACEB_RK2_1) return;
+  if (j < g.n2 && k < g.n3) g.b0f[0][fix(g, 0, i, j, k)] = g.bf[0][fix(g, 0, i, j, k)];
+  if (i < g.n1 && k < g.n3) g.b0f[1][fix(g, 1, i, j, k)] = g.bf[1][fix(g, 1, i, j, k)];
+  if (SD == 3 && i < g.n1 && j < g.n2)
+    g.b0f[2][fix(g, 2, i, j, k)] = g.bf[2][fix(g, 2, i, j, k)];
+}
+template <bool F32>
 __global__ void __launch_bounds__(256) k_faceb(Grid g, int mode, double a1, double a2,
                                                double c3) {
   int i, j;
   const int k = blockIdx.z;
   if (!plane_coords(g.n1 + 1, g.n2 + 1, i, j)) return;
   if (!g.sc->active) {
-    if (mode == FACEB_RK2_1) {
-      if (j < g.n2 && k < g.n3) g.b0f[0][fix(g, 0, i, j, k)] = g.bf[0][fix(g, 0, i, j, k)];
-      if (i < g.n1 && k < g.n3) g.b0f[1][fix(g, 1, i, j, k)] = g.bf[1][fix(g, 1, i, j, k)];
-      if (SD == 3 && i < g.n1 && j < g.n2)
-        g.b0f[2][fix(g, 2, i, j, k)] = g.bf[2][fix(g, 2, i, j, k)];
-    }
+    faceb_keep<3>(g, mode, i, j, k);
     return;
   }
   const double a3 = c3 * g.sc->dt;
   const double i1 = g.inv_dx[0], i2 = g.inv_dx[1], i3 = g.inv_dx[2];
   const EdgeEmf<F32> C1{g.cor[0], g.corf[0]}, C2{g.cor[1], g.corf[1]}, C3{g.cor[2], g.corf[2]};
   if (j < g.n2 && k < g.n3) {
-    double t;
-    if (SD == 3)
-      t = -(C2[kix(g, 1, i, j, k + 1)] - C2[kix(g, 1, i, j, k)]) * i3 +
-          (C3[kix(g, 2, i, j + 1, k)] - C3[kix(g, 2, i, j, k)]) * i2;
-    else
-      t = (C3[kix(g, 2, i, j + 1, k)] - C3[kix(g, 2, i, j, k)]) * i2;
+    const double t = -(C2[kix(g, 1, i, j, k + 1)] - C2[kix(g, 1, i, j, k)]) * i3 +
+                     (C3[kix(g, 2, i, j + 1, k)] - C3[kix(g, 2, i, j, k)]) * i2;
     faceb_set(g, 0, fix(g, 0, i, j, k), mode, a1, a2, a3, t);
   }
   if (i < g.n1 && k < g.n3) {
-    double t;
-    if (SD == 3)
-      t = (C1[kix(g, 0, i, j, k + 1)] - C1[kix(g, 0, i, j, k)]) * i3 +
-          (C3[kix(g, 2, i, j, k)] - C3[kix(g, 2, i + 1, j, k)]) * i1;
-    else
-      t = (C3[kix(g, 2, i, j, k)] - C3[kix(g, 2, i + 1, j, k)]) * i1;
+    const double t = (C1[kix(g, 0, i, j, k + 1)] - C1[kix(g, 0, i, j, k)]) * i3 +
+                     (C3[kix(g, 2, i, j, k)] - C3[kix(g, 2, i + 1, j, k)]) * i1;
     faceb_set(g, 1, fix(g, 1, i, j, k), mode, a1, a2, a3, t);
   }
-  if (SD == 3 && i < g.n1 && j < g.n2) {
+  if (i < g.n1 && j < g.n2) {
     const double t = (C2[kix(g, 1, i + 1, j, k)] - C2[kix(g, 1, i, j, k)]) * i1 -
                      (C1[kix(g, 0, i, j + 1, k)] - C1[kix(g, 0, i, j, k)]) * i2;
     faceb_set(g, 2, fix(g, 2, i, j, k), mode, a1, a2, a3, t);
   }
+}
+
+// 2D: both in one pass, a thread's two faces from their three edges, each edge
+// computed by up to four threads (from cache; a 2D stage is bound by its
+// launches: 333 x 250 FP64 RK3 109 -> 98 us per step, 84 with the fused sweep).  F32: the edge EMF is rounded to FP32 as the 3D path stores it.
+template <bool F32>
+__global__ void __launch_bounds__(256) k_ct2(Grid g, int mode, double a1, double a2, double c3) {
+  int i, j;
+  if (!plane_coords(g.n1 + 1, g.n2 + 1, i, j)) return;
+  if (!g.sc->active) {
+    faceb_keep<2>(g, mode, i, j, 0);
+    return;
+  }
+  auto edge = [&](int x, int y) {
+    const double e = CtNode<F32>(g, x, y).edge3(g, 0);
+    return F32 ? (double)(float)e : e;
+  };
+  const double a3 = c3 * g.sc->dt, e = edge(i, j);
+  if (j < g.n2)
+    faceb_set(g, 0, fix(g, 0, i, j, 0), mode, a1, a2, a3, (edge(i, j + 1) - e) * g.inv_dx[1]);
+  if (i < g.n1)
+    faceb_set(g, 1, fix(g, 1, i, j, 0), mode, a1, a2, a3, (e - edge(i + 1, j)) * g.inv_dx[0]);
 }
 
 // ----------------------------------------------------------- wave max
@@ -1627,7 +1668,7 @@ __global__ void __launch_bounds__(256)
   constexpr bool GAM = EK == EK_FASTEOS;
   static_assert(EK != EK_HELM_FACE, "per-face Newton states are not staged");
   static_assert(!FUSE || (!MHD && EK == EK_IDEAL), "the stage's end without CT and EoS solve");
-  static_assert(SD == 3 || FUSE, "2D stages are fused ones");
+  static_assert(SD == 3 || EK == EK_IDEAL, "2D: the ideal gas");
   static_assert(!SF || (FUSE && !MIX), "shock flattening: FP64 whole stages");
   using Re = typename std::conditional<MIX, float, double>::type;
   constexpr int TX = kSweepT, TY = kSweepTy;     // cells per tile
@@ -1724,7 +1765,7 @@ __global__ void __launch_bounds__(256)
     for (int v = 0; v < NV; v++) t[v * WW + cell] = c.q[v];
     if (MHD) {
 #pragma unroll
-      for (int v = 0; v < 3; v++) t[(OB + v) * WW + cell] = c.b[v];
+      for (int v = 0; v < SD; v++) t[(OB + v) * WW + cell] = c.b[v];
     }
     if (GAM) {
       t[OG * WW + cell] = c.ga[0];
@@ -1964,7 +2005,7 @@ __global__ void __launch_bounds__(256)
           if (SD == 3) S0[3] = rho * v3;
           double E = g.eint[c] + 0.5 * rho * (v1 * v1 + v2 * v2 + v3 * v3);
           if (MHD) {
-            const double b1 = g.bcc[c], b2 = g.bcc[N + c], b3 = g.bcc[2 * N + c];
+            const double b1 = g.bcc[c], b2 = g.bcc[N + c], b3 = (SD == 3) ? g.bcc[2 * N + c] : 0.0;
             E = E + 0.5 * (b1 * b1 + b2 * b2 + b3 * b3);
           }
           if (g.etot) E = E + rho * g.phi_cc[lj];
@@ -2273,12 +2314,14 @@ struct Kern {
   }
   static void corner(const Grid &g, hipStream_t st) {
     const dim3 blk(64, 4, 1);
-    k_corner<SD, MIX><<<grid_plane(g.n1 + 1, g.n2 + 1, SD == 3 ? g.n3 + 1 : 1), blk, 0, st>>>(g);
+    k_corner<MIX><<<grid_plane(g.n1 + 1, g.n2 + 1, g.n3 + 1), blk, 0, st>>>(g);
   }
   static void faceb(const Grid &g, int mode, double a1, double a2, double c3, hipStream_t st) {
-    const dim3 blk(64, 4, 1);
-    k_faceb<SD, MIX><<<grid_plane(g.n1 + 1, g.n2 + 1, SD == 3 ? g.n3 + 1 : 1), blk, 0, st>>>(
-        g, mode, a1, a2, c3);
+    const dim3 blk(64, 4, 1), grd = grid_plane(g.n1 + 1, g.n2 + 1, SD == 3 ? g.n3 + 1 : 1);
+    if constexpr (SD == 3)
+      k_faceb<MIX><<<grd, blk, 0, st>>>(g, mode, a1, a2, c3);
+    else
+      k_ct2<MIX><<<grd, blk, 0, st>>>(g, mode, a1, a2, c3);
   }
   static void update(const Grid &g, int first, int last, double a1, double a2, double c3,
                      int fin, hipStream_t st) {
@@ -2296,7 +2339,8 @@ struct Kern {
   // the RK combination (kWhole), else the sweep and the update that finishes
   // its stage after CT (2nd-order reconstructions, ideal / FASTEOS states)
   static constexpr bool kWhole = !R5 && !MHD && EK == EK_IDEAL;
-  static constexpr bool kSwept = (SD == 3 || kWhole) && !R5 && EK != EK_HELM_FACE;
+  static constexpr bool kSwept =
+      (SD == 3 || kWhole || (EK == EK_IDEAL && NAS == 0)) && !R5 && EK != EK_HELM_FACE;
   static int sweep(const Grid &g, int first, int last, int fin, double a1, double a2, double c3,
                    hipStream_t st) {
     if constexpr (kSwept) {
@@ -2383,7 +2427,7 @@ static KernelTable make_table() {
   KernelTable t{};
   t.flux = &K::flux;
   if constexpr (R5) return t;
-  t.corner = &K::corner;
+  t.corner = SD == 3 ? &K::corner : nullptr;  // 2D: faceb computes its edges
   t.faceb = &K::faceb;
   t.update = &K::update;
   t.update_guess = HELM ? &K::update_guess : nullptr;
