@@ -29,7 +29,7 @@ enum { FLUX_HLLC = 0, FLUX_LHLLC = 1, FLUX_HLLD = 2, FLUX_LHLLD = 3 };
 // Device-resident step control: dt/time/smax never round-trip to the host.
 struct Scalars {
   double time, dt, smax, tmax, cfl;
-  unsigned long long spare;
+  double par;  // thermal diffusion: 1 / dt_par of the last evaluation
   long long step;
   int active;  // 0 once time >= tmax: the step's kernels return at once
   int flags;   // mixed precision: SC_U_CUR | SC_P_STALE (set by the kernels that ran)
