@@ -18,7 +18,7 @@
 // Every kernel is one thread per cell and HBM bound: a middle stage of the ideal
 // gas moves 56 bytes per cell (e_jm1, rho, kappa, e_jm2, e_0, Me_0 in, e_j out;
 // the neighbours from cache), where a T pass and an in-place update took
-// 96 and two launches: 50 -> 24 us per stage at 128^3 (4.9 TB/s of those bytes).
+// 96 and two launches: 50 -> 37 us per stage at 128^3.
 #include "phlx_internal.hpp"
 
 namespace phlx {
