@@ -88,10 +88,14 @@ def kernel_bytes(cfg, name: str, swept: bool = False) -> float:
         # the fused sweep, averaged over the two RK2 stages: the cell inputs
         # and the normal face B once; stage 1 the prim, eint, b_cc of the
         # state0 rebuild, stage 2 state0 and the stage state; the new state
-        # (and state0 at stage 1), 2 EMFs + sign per face (MHD) out
+        # (and state0 at stage 1), 2 EMFs + sign per face (MHD) out; the ideal
+        # gas without a field ends its stage here: the new prim and eint (FP32
+        # prim in the mixed path) out too
         st = nv + 1 + (sd if mhd else 0)
         rd = N * cell_in + (sum(nf[:sd]) * 8 if mhd else 0) + 0.5 * N * 8 * (st + 2 * nv)
         wr = (sum(nf[:sd]) * 17 if mhd else 0) + 1.5 * N * 8 * nv
+        if not mhd and not helm:
+            wr += N * (4 * nv if cfg.precision == 1 else 8 * (nv + 1))
         return rd + wr
     if name == "update" and swept:
         # cons -> prim after the fused sweep: U and the face B (Helmholtz: T)
@@ -126,29 +130,27 @@ def kernel_bytes(cfg, name: str, swept: bool = False) -> float:
         pf = 4 * (nv + 5) if mix else 0
         return rd + N * (8 * words + pf)
     if name == "misc" and cfg.shock_flattening:
-        # shock-flattening flags: pressure in, detector bytes out and in
-        # (cells -2..n+1), flag bytes out (cells -1..n)
-        e = [nx + 4, ny + 4, nz + 4 if sd == 3 else 1]
+        # shock-flattening flags: pressure in, flag bytes out (cells -1..n)
         f = [nx + 2, ny + 2, nz + 2 if sd == 3 else 1]
-        return N * 8 + 2 * e[0] * e[1] * e[2] + f[0] * f[1] * f[2]
+        return N * 8 + f[0] * f[1] * f[2]
     return 0.0
 
 
 def diffusion_bytes(cfg, stages: int) -> float:
     """Algorithmic bytes of one thermal-diffusion step (RKL2, s stages):
-    stage 1 reads T, rho, kappa, eint and writes e_0, Me_0, e_jm2, eint;
-    every further stage converts eint to T (eint, rho in, T out; Helmholtz
-    also Ye, 1/abar and the carried T in) and reads T, rho, kappa, eint,
-    e_jm2, e_0, Me_0, writing eint and e_jm2; the end converts once more and
-    writes T and p (Helmholtz also eint and the FASTEOS gammas)."""
+    stage 1 reads p (Helmholtz T), rho, kappa, eint and writes Me_0 and e_1;
+    every further stage of the ideal gas reads e_jm1, rho, kappa, e_jm2, e_0,
+    Me_0 and writes e_j, the last one eint, T and p instead.  Helmholtz
+    converts before each (eint, rho, Ye, 1/abar and the carried T in, T out)
+    and reads T besides; its end converts once more and writes T, p, eint and
+    the FASTEOS gammas."""
     nz, ny, nx = cfg.shape
     N = nx * ny * nz
-    helm = cfg.eos == 1
-    to_t = 24 + (24 if helm else 0)
-    stage = 24 + 32 + 16
-    first = 24 + 8 + 32 + (0 if helm else 24)   # + T from p for the ideal gas
-    final = to_t + 8 + (24 if helm and cfg.fasteos else (8 if helm else 0))
-    return N * (first + (stages - 1) * (to_t + stage) + final)
+    first = 32 + 16
+    if cfg.eos != 1:
+        return N * (first + (stages - 2) * 56 + 72)
+    to_t = 48
+    return N * (first + (stages - 1) * (to_t + 64) + to_t + (32 if cfg.fasteos else 16))
 
 
 def b_zu(cfg) -> int:

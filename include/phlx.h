@@ -162,10 +162,11 @@ int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, double a3,
  * cons -> prim and the CFL maximum included) into one pass that stages a
  * pencil tile in LDS and keeps the face fluxes out of HBM: mode 1 wherever the
  * run admits it, 0 never, -1 (the default) where it is the faster form: runs
- * without MHD.  It applies with LIM2ND or PPH and no shock flattening to 3D
- * runs with the ideal or the FASTEOS Helmholtz state and to 2D runs of the
- * ideal gas without MHD; with MHD, nx1 has to be a multiple of 16 (other runs
- * take the separate sweeps).  Either way the results are bit for bit the
+ * without MHD, and ideal MHD without scalars in 2D and from 32768 cells in 3D.
+ * It applies with LIM2ND or PPH to 3D runs with the ideal or the FASTEOS
+ * Helmholtz state (with MHD, nx1 has to be a multiple of 16) and to 2D runs of
+ * the ideal gas (with MHD: without scalars); with shock flattening to the
+ * ideal gas without MHD.  Other runs take the separate sweeps.  Either way the results are bit for bit the
  * same.  No counterpart in the reference (its hydro_step is one routine either
  * way): for A/B timing and for callers that want the per-direction kernels. */
 int phlx_set_fused_sweep(phlx_ctx *ctx, int32_t mode);
