@@ -44,3 +44,33 @@ def test_two_steps_bitwise(oracle_mod, dims, ratio, stages):
             assert np.array_equal(got[name], ref[name]), (n, name)
     sim.close()
     r.close()
+
+
+@pytest.mark.parametrize("dims", [(33, 9, 1601), (64, 16, 1024)])
+def test_marching_chunks_bitwise(oracle_mod, dims):
+    """3D grids large enough for chunks of two and three planes, the last one
+    short: the carried x3 flux and the prefetched planes, walls and wraps."""
+    from phlegethon_amd.runtime import Simulation
+    wall = dims[0] % 2 == 1
+    bc = (BC_REFLECTIVE, BC_OUTFLOW, 0, 0, BC_OUTFLOW, BC_REFLECTIVE) if wall else (0,) * 6
+    fix = (None, 1.2e7, None, None, 0.9e7, None) if wall else None
+    cfg = PhlxConfig(sdims=3, nx1=dims[0], nx2=dims[1], nx3=dims[2], x1u=1e8, x2u=8e7, x3u=1e9,
+                     bc=bc, thermal_diffusion=True, fix_temperature=fix)
+    pb = _random_T(cfg, amp=0.02)
+    r = oracle_mod.OracleRun(pb)
+    r.init()
+    dtp = r.parabolic_dt()
+    r.set_scalar("dt", 5.0 * dtp)
+    sim = Simulation(cfg)
+    sim.setup(pb)
+    sim.init()
+    sc = sim.scalars()
+    assert sim.parabolic_dt() == dtp
+    sim.set_scalars(sc["time"], 5.0 * dtp, sc["smax"], sc["step"])
+    r.diffusion_step(1)
+    sim.diffusion_step(1)
+    got, ref = sim.download(), r.state()
+    sim.close()
+    r.close()
+    for name in ("eint", "temp", "prim"):
+        assert np.array_equal(got[name], ref[name]), name
