@@ -695,8 +695,9 @@ static bool use_fused_sweep(const phlx_ctx *ctx) {
   // faster form (384^3 hydro FP64 9800 / 14400, mixed 5650 / 7650); ideal MHD
   // from 32^3 (32^3 FP64 81 / 92, mixed 69 / 87; 256^3 7055 / 7770, 4240 /
   // 4345), in 2D at any size (64 x 48 FP64 RK3 60 / 74, 1024^2 332 / 413, mixed
-  // 2000 x 1500 641 / 751); MHD with the tabulated EoS spills and is slower (128^3 FP64 2090 /
-  // 1705, 256^3 mixed 7880 / 7230), as the ideal one with two scalars does
+  // 2000 x 1500 641 / 751); MHD with the tabulated EoS spills and is slower
+  // (128^3 FP64 2090 / 1705, 256^3 mixed 7880 / 7230), as the ideal one with
+  // two scalars does
   const bool mhd_too =
       ctx->cfg.eos == PHLX_EOS_IDEAL && g.nas == 0 && (g.sd == 2 || g.N >= 32768);
   const bool want = ctx->fused_sweep < 0 ? !g.mhd || mhd_too : ctx->fused_sweep != 0;

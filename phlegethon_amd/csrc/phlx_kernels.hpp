@@ -5,6 +5,7 @@
 //   k_flux<x1>, k_flux<x2>, k_flux<x3>   face states -> Riemann fluxes (+EMF, sign)
 //   k_corner                             CT-contact corner EMFs      (MHD)
 //   k_faceb                              face-B update (FP64)         (MHD)
+//   (2D: k_ct2                           both)
 //   k_update                             flux divergence + sources + RK combine
 //                                        + cons->prim (+ CFL max at the last stage)
 // or, fused (k_sweep, the 2nd-order reconstructions),
@@ -185,7 +186,7 @@ __device__ __forceinline__ void flux_face(const Grid &g, int i, int j, int k, do
 // flux correction and the ETOT potential flux.  MHD faces also store the
 // two tangential EMF components and the contact-upwind sign used by CT.
 // EK: EoS kind of the face states (EK_IDEAL, EK_FASTEOS, EK_HELM_FACE).
-// SF: USE_SHOCK_FLATTENING -- the flags of cells f-1 and f (k_sf_dilate)
+// SF: USE_SHOCK_FLATTENING -- the flags of cells f-1 and f (k_sf_flags)
 // select LIM2ND for a flattened cell and the HLL flux for the face.
 template <int DIR, int SD, int NAS, bool MHD, int EK, bool R5, bool SF = false>
 __global__ void __launch_bounds__(256) k_flux(Grid g) {
@@ -953,7 +954,8 @@ __global__ void __launch_bounds__(256) k_faceb(Grid g, int mode, double a1, doub
 
 // 2D: both in one pass, a thread's two faces from their three edges, each edge
 // computed by up to four threads (from cache; a 2D stage is bound by its
-// launches: 333 x 250 FP64 RK3 109 -> 98 us per step, 84 with the fused sweep).  F32: the edge EMF is rounded to FP32 as the 3D path stores it.
+// launches: 333 x 250 FP64 RK3 109 -> 98 us per step, 84 with the fused sweep).
+// F32: the edge EMF is rounded to FP32 as the 3D path stores it.
 template <bool F32>
 __global__ void __launch_bounds__(256) k_ct2(Grid g, int mode, double a1, double a2, double c3) {
   int i, j;
