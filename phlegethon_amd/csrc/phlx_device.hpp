@@ -281,7 +281,9 @@ __device__ __forceinline__ void rec_lim2nd(double qm, double qc, double qp, doub
   // harmonic-mean limited slope, source/source.F90:8141-8181
   double sf = qp - qc, sb = qc - qm;
   double prod = sf * sb, slope = 0.0;
-  if (prod > 0.0) slope = Recip(sf + sb).div(prod);
+  // prod is no zero and no NaN; where it or the sum is infinite the edges are
+  // infinite or NaN either way
+  if (prod > 0.0) slope = Recip(sf + sb).div_finite(prod);
   double h = 0.5 * slope;
   l = qc - h;
   r = qc + h;

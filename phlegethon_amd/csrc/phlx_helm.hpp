@@ -20,6 +20,8 @@
 
 #include <hip/hip_runtime.h>
 
+#include "phlx_fp64.hpp"
+
 namespace phlx {
 
 constexpr double kHelmRgas = 8.31446261815324e7;  // source/source.F90:605-616
@@ -55,48 +57,6 @@ struct HelmCell {
 // evaluation into the conditional stores that follow (one copy per branch),
 // which holds every table value of the evaluation live at once.
 __device__ __forceinline__ void helm_pin(double &v) { asm volatile("" : "+v"(v)); }
-
-// Correctly rounded FP64 quotients of one denominator, the bits of a / b, in
-// fewer instructions than the compiler's expansion of it (v_div_scale twice,
-// reciprocal, four FMAs, product, remainder, v_div_fmas, v_div_fixup: 11 per
-// quotient, nothing shared).  The hardware reciprocal (relative error e <
-// 2^-24.4) is refined in one third-order step, r (1 + e + e^2), to half an ulp;
-// each quotient is the product with it corrected by its exact FMA remainder
-// (Markstein's theorem).  4 instructions and 3 per quotient (2 for 1 / b).
-// Without the scaling the remainder must stay a normal number: b normal and
-// finite, |a| in [2^-960, 2^960] or 0 and a / b in that range too.  No operand
-// of a physical state leaves it (b = 0 gives NaN where a / b is inf: the
-// callers' denominators are densities, speeds, cell widths, temperatures).
-// Checked bit for bit against a / b and 1 / b on 1.6e10 pairs with exponents
-// to +-480, mantissas next to all-ones and all-zeros among them.
-struct Recip {
-  double b, r;
-  __device__ __forceinline__ explicit Recip(double v) : b(v) {
-    const double r0 = __builtin_amdgcn_rcp(v);
-    const double e = fma(-v, r0, 1.0);
-    r = fma(r0, fma(e, e, e), r0);
-  }
-  __device__ __forceinline__ double div(double a) const {
-    const double q = a * r;
-    return fma(fma(-b, q, a), r, q);
-  }
-  __device__ __forceinline__ double inv() const { return fma(fma(-b, r, 1.0), r, r); }
-};
-// The correctly rounded square root, the bits of sqrt(x), for x = 0 or x in
-// [2^-960, 2^960] (NaN for x < 0): Goldschmidt's iteration from the hardware's
-// reciprocal root and two exact-remainder corrections, without the compiler's
-// rescaling and its tests of the ends of the range (13 instructions instead
-// of 19).  Checked on the same sample.
-__device__ __forceinline__ double dsqrt(double x) {
-  const double y = __builtin_amdgcn_rsq(x);
-  double s = x * y, h = 0.5 * y;
-  const double r = fma(-h, s, 0.5);
-  s = fma(s, r, s);
-  h = fma(h, r, h);
-  s = fma(fma(-s, s, x), h, s);
-  s = fma(fma(-s, s, x), h, s);
-  return x == 0.0 ? x : s;
-}
 
 // a / b; FAST (the mixed-precision EoS step only): the hardware reciprocal
 // refined by two Newton steps (~1 ulp) instead of the correctly rounded form.
