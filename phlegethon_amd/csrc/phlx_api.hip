@@ -20,6 +20,16 @@ struct ProfRec {
   hipEvent_t a, b;
 };
 
+// A captured step and what it was captured with: the grid descriptor (every
+// kernel argument but the per-stage constants), the sweep form and the Newton
+// counting.  after: the descriptor the step leaves, its buffers swapped.
+struct StepGraph {
+  hipGraph_t graph = nullptr;
+  hipGraphExec_t exec = nullptr;
+  Grid g{}, after{};
+  bool fused = false, stats = false;
+};
+
 struct phlx_ctx {
   phlx_config cfg;
   Grid g;
@@ -62,14 +72,9 @@ struct phlx_ctx {
   // RK2 with MHD: between a step's two CT calls the stage-1 face field
   // lives in the b0f buffers and g.bf / g.b0f are swapped (k_faceb)
   bool b_swapped = false;
-  // phlx_run's captured step (phlx_set_step_graph) and what it was
-  // captured with: the grid descriptor (every kernel argument but the
-  // per-stage constants), the sweep form and the Newton counting
+  // phlx_run's captured steps (phlx_set_step_graph)
   bool step_graph = false;
-  hipGraph_t sg_graph = nullptr;
-  hipGraphExec_t sg_exec = nullptr;
-  Grid sg_g{};
-  bool sg_fused = false, sg_stats = false;
+  StepGraph sg[2];
   double dt_par = 0.0;
   int diff_stages = 0;  // stages of the last diffusion step
   // profiling
@@ -320,12 +325,18 @@ extern "C" int phlx_create(const phlx_config *cfg, phlx_ctx **out) {
   return PHLX_OK;
 }
 
+static void drop_step_graph(StepGraph &s) {
+  if (s.exec) (void)hipGraphExecDestroy(s.exec);
+  if (s.graph) (void)hipGraphDestroy(s.graph);
+  s.exec = nullptr;
+  s.graph = nullptr;
+}
+
 extern "C" int phlx_destroy(phlx_ctx *ctx) {
   if (!ctx) return PHLX_E_ARG;
   (void)hipSetDevice(ctx->device);
   if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
-  if (ctx->sg_exec) (void)hipGraphExecDestroy(ctx->sg_exec);
-  if (ctx->sg_graph) (void)hipGraphDestroy(ctx->sg_graph);
+  for (auto &s : ctx->sg) drop_step_graph(s);
   for (auto &r : ctx->recs) {
     (void)hipEventDestroy(r.a);
     (void)hipEventDestroy(r.b);
@@ -687,8 +698,7 @@ extern "C" int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, 
 
 // Whether hydro_step takes the fused sweep: a family that has one and no shock
 // flattening (its flagged cells switch scheme per face); with MHD, x1 tiles
-// that divide the grid.  A captured step keeps its buffers, so an odd number
-// of whole-stage passes, which ends in the other one, is not captured.
+// that divide the grid.
 static bool use_fused_sweep(const phlx_ctx *ctx) {
   const Grid &g = ctx->g;
   // measured on MI355X, us per step, fused / split: without MHD always the
@@ -704,7 +714,7 @@ static bool use_fused_sweep(const phlx_ctx *ctx) {
   if (!want || !ctx->kt.sweep) return false;
   // shock flattening has no swept form beside the whole-stage one
   if (g.sflat && ctx->kt.update_swept) return false;
-  if (!ctx->kt.update_swept) return !(ctx->step_graph && ctx->stages % 2);
+  if (!ctx->kt.update_swept) return true;
   return (!g.mhd || g.sd == 2 || g.n1 % kSweepT == 0) &&
          (!ctx->kt.update_guess || ctx->kt.update_swept_guess);
 }
@@ -860,28 +870,39 @@ extern "C" int phlx_set_step_graph(phlx_ctx *ctx, int32_t on) {
   return PHLX_OK;
 }
 
-static void drop_step_graph(phlx_ctx *ctx) {
-  if (ctx->sg_exec) (void)hipGraphExecDestroy(ctx->sg_exec);
-  if (ctx->sg_graph) (void)hipGraphDestroy(ctx->sg_graph);
-  ctx->sg_exec = nullptr;
-  ctx->sg_graph = nullptr;
-}
-
-// The executable graph of one step (step begin, hydro_step with the CFL,
-// step end), captured from the same launch sequence as the eager loop.  It
-// holds only kernel nodes.  Captured again when the grid descriptor, the
-// sweep form or the Newton counting differ from the capture's.
-static int step_graph_ready(phlx_ctx *ctx) {
+// The executable graph of one step from the current buffers (step begin,
+// hydro_step with the CFL, step end), captured from the same launch sequence as
+// the eager loop.  It holds only kernel nodes.  A step of an odd number of
+// whole-stage passes ends in the other buffer, so two graphs alternate.
+// Captured again when the grid descriptor, the sweep form or the Newton counting
+// differ from both captures'.
+static int step_graph_ready(phlx_ctx *ctx, StepGraph *&out) {
   const bool fused = use_fused_sweep(ctx);
-  if (ctx->sg_exec && ctx->sg_fused == fused && ctx->sg_stats == ctx->eos_stats &&
-      std::memcmp(&ctx->sg_g, &ctx->g, sizeof(Grid)) == 0)
-    return PHLX_OK;
-  drop_step_graph(ctx);
+  const auto current = [&](const StepGraph &s) {
+    return s.exec && s.fused == fused && s.stats == ctx->eos_stats;
+  };
+  for (auto &s : ctx->sg)
+    if (current(s) && std::memcmp(&s.g, &ctx->g, sizeof(Grid)) == 0) {
+      out = &s;
+      return PHLX_OK;
+    }
+  // beside the graph whose step led here, else in place of the first
+  const bool follows =
+      current(ctx->sg[0]) && std::memcmp(&ctx->sg[0].after, &ctx->g, sizeof(Grid)) == 0;
+  StepGraph &s = ctx->sg[follows ? 1 : 0];
+  if (s.exec) HIPCHK(hipStreamSynchronize(ctx->stream));  // its launches end first
+  drop_step_graph(s);
+  s.g = ctx->g;
+  const bool b_swapped = ctx->b_swapped;
   HIPCHK(hipStreamBeginCapture(ctx->stream, hipStreamCaptureModeThreadLocal));
   launch_step_begin(ctx->g.sc, ctx->stream);
   int n_cfl;
   const int rc = do_hydro_step(ctx, true, &n_cfl);
   launch_step_end(ctx->g, n_cfl, 1, 0, ctx->stream);
+  // nothing has run yet
+  s.after = ctx->g;
+  ctx->g = s.g;
+  ctx->b_swapped = b_swapped;
   hipGraph_t gr = nullptr;
   const hipError_t e = hipStreamEndCapture(ctx->stream, &gr);
   if (rc || e != hipSuccess) {
@@ -889,15 +910,15 @@ static int step_graph_ready(phlx_ctx *ctx) {
     (void)hipGetLastError();
     return rc ? rc : PHLX_E_HIP;
   }
-  ctx->sg_graph = gr;
-  if (hipGraphInstantiate(&ctx->sg_exec, gr, nullptr, nullptr, 0) != hipSuccess) {
-    ctx->sg_exec = nullptr;
-    drop_step_graph(ctx);
+  s.graph = gr;
+  if (hipGraphInstantiate(&s.exec, gr, nullptr, nullptr, 0) != hipSuccess) {
+    s.exec = nullptr;
+    drop_step_graph(s);
     return PHLX_E_HIP;
   }
-  ctx->sg_g = ctx->g;
-  ctx->sg_fused = fused;
-  ctx->sg_stats = ctx->eos_stats;
+  s.fused = fused;
+  s.stats = ctx->eos_stats;
+  out = &s;
   return PHLX_OK;
 }
 
@@ -907,12 +928,16 @@ extern "C" int phlx_run(phlx_ctx *ctx, int32_t nsteps) {
   HIPCHK(hipSetDevice(ctx->device));
   const bool diff = ctx->diff_on;
   if (ctx->step_graph && nsteps > 0 && !diff && !ctx->prof && !ctx->b_swapped) {
-    const int rc = step_graph_ready(ctx);
-    if (rc) return rc;
-    for (int s = 0; s < nsteps; s++) HIPCHK(hipGraphLaunch(ctx->sg_exec, ctx->stream));
-    // the host-side records an eager step leaves
-    ctx->tdiff_valid = false;
-    if (ctx->kt.prims) ctx->prim_stale = true;
+    for (int s = 0; s < nsteps; s++) {
+      StepGraph *sg = nullptr;
+      const int rc = step_graph_ready(ctx, sg);
+      if (rc) return rc;
+      HIPCHK(hipGraphLaunch(sg->exec, ctx->stream));
+      // the host-side records an eager step leaves
+      ctx->g = sg->after;
+      ctx->tdiff_valid = false;
+      if (ctx->kt.prims) ctx->prim_stale = true;
+    }
     return PHLX_OK;
   }
   if (nsteps > 0) launch_step_begin(ctx->g.sc, ctx->stream);
