@@ -69,6 +69,8 @@ struct phlx_ctx {
   // hydro_step's fused sweep: -1 = where it is the faster form, 0 = never,
   // 1 = wherever the kernel family has one
   int fused_sweep = -1;
+  // whole-stage passes: the axis whose flux buffer takes the next primitives
+  int pn_dir = 0;
   // RK2 with MHD: between a step's two CT calls the stage-1 face field
   // lives in the b0f buffers and g.bf / g.b0f are swapped (k_faceb)
   bool b_swapped = false;
@@ -236,20 +238,25 @@ extern "C" int phlx_create(const phlx_config *cfg, phlx_ctx **out) {
   }
   const size_t N = (size_t)g.N, nv = (size_t)g.nv;
   int e = 0;
-  e |= dalloc(ctx, &g.P, nv * N);
+  // whole-stage passes write the new primitives into the buffer of the fluxes
+  // along the longest axis, which they leave alone, and the two change roles
+  // (next_prims): either is large enough for both
+  const bool whole = ctx->kt.sweep && !ctx->kt.update_swept, mix = cfg->precision == PHLX_PREC_MIXED;
+  for (int d = 1; d < g.sd; d++)
+    if (g.nf[d] < g.nf[ctx->pn_dir]) ctx->pn_dir = d;
+  const size_t nvf = whole ? nv * (size_t)g.nf[ctx->pn_dir] : 0;
+  e |= dalloc(ctx, &g.P, mix ? nv * N : std::max(nv * N, nvf));
   e |= dalloc(ctx, &g.U, nv * N);
   e |= dalloc(ctx, &g.U0, nv * N);
   e |= dalloc(ctx, &g.eint, N);
-  if (cfg->precision == PHLX_PREC_MIXED) e |= dalloc(ctx, &g.Pf, (nv + 5) * N);
-  if (ctx->kt.sweep && !ctx->kt.update_swept) {
-    if (cfg->precision == PHLX_PREC_MIXED)
-      e |= dalloc(ctx, &g.Pfn, nv * N);
-    else
-      e |= dalloc(ctx, &g.Pn, nv * N);
-  }
+  if (mix) e |= dalloc(ctx, &g.Pf, std::max((nv + 5) * N, nvf));
   for (int d = 0; d < g.sd; d++) {
     e |= dalloc(ctx, &g.F[d], nv * (size_t)g.nf[d]);
     g.Ff[d] = (float *)g.F[d];  // the mixed path stores FP32 fluxes in the same buffer
+  }
+  if (whole) {
+    g.Pn = mix ? nullptr : g.F[ctx->pn_dir];
+    g.Pfn = mix ? g.Ff[ctx->pn_dir] : nullptr;
   }
   if (g.mhd) {
     e |= dalloc(ctx, &g.bcc, 3 * N);
@@ -747,6 +754,22 @@ static int materialize(phlx_ctx *ctx) {
   return check_launch();
 }
 
+// After a whole-stage pass: its primitives are the current ones, and their
+// buffer before it is that of the fluxes (of FP32 fluxes alone in the mixed path).
+static void next_prims(phlx_ctx *ctx) {
+  Grid &g = ctx->g;
+  const int d = ctx->pn_dir;
+  if (g.Pfn) {
+    std::swap(g.Pf, g.Pfn);
+    g.Ff[d] = g.Pfn;
+    g.F[d] = nullptr;
+  } else {
+    std::swap(g.P, g.Pn);
+    g.F[d] = g.Pn;
+    g.Ff[d] = nullptr;
+  }
+}
+
 // n_cfl: the partials of the CFL maximum that the last stage leaves.
 static int do_hydro_step(phlx_ctx *ctx, bool with_cfl, int *n_cfl = nullptr) {
   const bool fused = use_fused_sweep(ctx);
@@ -766,11 +789,7 @@ static int do_hydro_step(phlx_ctx *ctx, bool with_cfl, int *n_cfl = nullptr) {
       rc = check_launch();
       if (rc) return rc;
       if (whole) {
-        Grid &g = ctx->g;
-        if (g.Pfn)
-          std::swap(g.Pf, g.Pfn);
-        else
-          std::swap(g.P, g.Pn);
+        next_prims(ctx);
         ctx->tdiff_valid = false;
         if (fin && ctx->kt.prims) ctx->prim_stale = true;
         if (n_cfl) *n_cfl = blocks;

@@ -56,8 +56,9 @@ struct Grid {
   // the update (and k_pack_f), read by the mixed flux kernels
   float *Pf;
   // ideal hydro in whole-stage passes (k_sweep): the buffer the next stage's
-  // primitives go to (FP64; the FP32 sweep inputs in the mixed path); the
-  // host swaps it with P / Pf after the launch
+  // primitives go to (FP64; the FP32 sweep inputs in the mixed path), that of
+  // one axis' fluxes, which these passes do not store; the host swaps it with
+  // P / Pf after the launch
   double *Pn;
   float *Pfn;
   double *bf[3], *b0f[3];
