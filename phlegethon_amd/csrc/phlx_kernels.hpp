@@ -291,6 +291,12 @@ struct CellW {
 // every row end, a third of them at n1 = 133).  2D, where a row is all there
 // is: 64 cells of it per wave, one segment per wave of the block.  False past
 // the grid.
+// The segment's bounds must stay the same in all lanes.  With 2D columns times
+// segments numbered flat, so that a wave's lanes could walk two segments, the
+// flattened sweep of the per-face Newton (256 VGPRs and 148 AGPRs, 135 scalar
+// registers spilled) gave wrong fluxes, and no speed over this form; nothing in
+// the walk depends on other lanes, and the cause was not found.  Cells of
+// several rows in a wave (3D) are right (tests/test_gpu_face_newton_3d.py).
 template <int DIR, int SD>
 __device__ __forceinline__ bool seg_coords(const Grid &g, int segf, int &i, int &o, int &f0) {
   if (SD == 2) {
