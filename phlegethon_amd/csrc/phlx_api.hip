@@ -155,10 +155,17 @@ static int validate(const phlx_config *c) {
   return PHLX_OK;
 }
 
+// A failure is returned, and leaves no error for the next launch's check.
+static int dev_malloc(void **p, size_t bytes) {
+  if (hipMalloc(p, bytes) == hipSuccess) return PHLX_OK;
+  (void)hipGetLastError();
+  return PHLX_E_NOMEM;
+}
+
 template <typename T>
 static int dalloc(phlx_ctx *ctx, T **p, size_t n) {
   void *q = nullptr;
-  if (hipMalloc(&q, n * sizeof(T) + 256) != hipSuccess) return PHLX_E_NOMEM;
+  if (const int rc = dev_malloc(&q, n * sizeof(T) + 256)) return rc;
   if (hipMemsetAsync(q, 0, n * sizeof(T) + 256, ctx->stream) != hipSuccess) return PHLX_E_HIP;
   ctx->allocs.push_back(q);
   *p = (T *)q;
@@ -1044,8 +1051,8 @@ extern "C" int phlx_stream_copy(phlx_ctx *ctx, int64_t nbytes, int32_t reps, dou
   HIPCHK(hipSetDevice(ctx->device));
   const long long n16 = nbytes / 16;
   void *a = nullptr, *b = nullptr;
-  if (hipMalloc(&a, n16 * 16) != hipSuccess) return PHLX_E_NOMEM;
-  if (hipMalloc(&b, n16 * 16) != hipSuccess) {
+  if (dev_malloc(&a, n16 * 16)) return PHLX_E_NOMEM;
+  if (dev_malloc(&b, n16 * 16)) {
     (void)hipFree(a);
     return PHLX_E_NOMEM;
   }
@@ -1125,7 +1132,7 @@ static int load_table(phlx_ctx *ctx, const double *f9, const double *c4, int32_t
   const size_t node_b = sizeof(double) * nodes.size();
   const size_t stage_b = sizeof(double) * 13 * np;
   void *buf = nullptr;
-  if (hipMalloc(&buf, rec_b + node_b + stage_b + 512) != hipSuccess) return PHLX_E_NOMEM;
+  if (dev_malloc(&buf, rec_b + node_b + stage_b + 512)) return PHLX_E_NOMEM;
   char *base = (char *)buf;
   double *tab = (double *)base;
   double *nd = (double *)(base + rec_b);
@@ -1212,7 +1219,7 @@ static int mlp_alloc(phlx_ctx *ctx) {
   const size_t bytes =
       floats * sizeof(float) + (kMlpW2aShorts + kMlpW1aShorts) * sizeof(unsigned short) + 4096;
   void *buf = nullptr;
-  if (hipMalloc(&buf, bytes) != hipSuccess) return PHLX_E_NOMEM;
+  if (dev_malloc(&buf, bytes)) return PHLX_E_NOMEM;
   HIPCHK(hipMemsetAsync(buf, 0, bytes, ctx->stream));
   float *f = (float *)buf;
   ctx->mlp_theta = f; f += P;
@@ -1363,7 +1370,7 @@ extern "C" int phlx_mlp_train(phlx_ctx *ctx, int64_t nsamples, int32_t epochs, i
     if (!(box[1] > box[0]) || !(box[3] > box[2])) return PHLX_E_ARG;
   }
   float *data = nullptr;
-  if (hipMalloc(&data, sizeof(float) * 11 * (size_t)n) != hipSuccess) return PHLX_E_NOMEM;
+  if (dev_malloc((void **)&data, sizeof(float) * 11 * (size_t)n)) return PHLX_E_NOMEM;
   float *raw = data, *label = data + 4 * n, *xn = data + 5 * n, *tn = data + 9 * n,
         *wt = data + 10 * n;
   launch_mlp_data(h, n, seed, box, raw, label, wt, ctx->stream);
@@ -1548,17 +1555,17 @@ extern "C" int phlx_set_thermal_diffusion(phlx_ctx *ctx, int32_t enable, int32_t
     }
   }
   HIPCHK(hipSetDevice(ctx->device));
-  if (!g.rkl[0]) {
-    const long long k3 = (g.sd == 3) ? g.n3 + 2 : 1;
-    const size_t nk = (size_t)(g.n1 + 2) * (g.n2 + 2) * k3;
-    int rc = dalloc(ctx, &g.kappa, nk);
-    if (!rc) rc = dalloc(ctx, &g.rkl[0], (size_t)g.N);
-    if (!rc) rc = dalloc(ctx, &g.rkl[1], (size_t)g.N);
-    if (!rc) rc = dalloc(ctx, &g.me0, (size_t)g.N);
-    if (!rc && !helm) rc = dalloc(ctx, &g.tdiff, (size_t)g.N);
-    if (rc) return rc;
-    if (helm) g.tdiff = g.temp;
-  }
+  const long long k3 = (g.sd == 3) ? g.n3 + 2 : 1;
+  const size_t nk = (size_t)(g.n1 + 2) * (g.n2 + 2) * k3;
+  // what an earlier call could not get is asked for again
+  const auto need = [&](double *&p, size_t n) { return p ? PHLX_OK : dalloc(ctx, &p, n); };
+  if (helm) g.tdiff = g.temp;
+  int rc = need(g.kappa, nk);
+  if (!rc) rc = need(g.rkl[0], (size_t)g.N);
+  if (!rc) rc = need(g.rkl[1], (size_t)g.N);
+  if (!rc) rc = need(g.me0, (size_t)g.N);
+  if (!rc) rc = need(g.tdiff, (size_t)g.N);
+  if (rc) return rc;
   for (int i = 0; i < 6; i++) g.fix_t[i] = ft[i];
   ctx->diff_eval = evaluate_dt != 0;
   ctx->diff_on = true;
