@@ -710,9 +710,10 @@ extern "C" int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, 
   return rk_update(ctx, irk, a1, a2, a3, last_stage, false);
 }
 
-// Whether hydro_step takes the fused sweep: a family that has one and no shock
-// flattening (its flagged cells switch scheme per face); with MHD, x1 tiles
-// that divide the grid.
+// Whether hydro_step takes the fused sweep: a family that has one; shock
+// flattening, whose flagged cells switch scheme per face, in whole stages alone;
+// 3D MHD only where the x1 tiles divide the grid (partial ones, which hydro and
+// 2D MHD take, have not been run or timed there).
 static bool use_fused_sweep(const phlx_ctx *ctx) {
   const Grid &g = ctx->g;
   // measured on MI355X, us per step, fused / split: without MHD always the
@@ -726,7 +727,6 @@ static bool use_fused_sweep(const phlx_ctx *ctx) {
       ctx->cfg.eos == PHLX_EOS_IDEAL && g.nas == 0 && (g.sd == 2 || g.N >= 32768);
   const bool want = ctx->fused_sweep < 0 ? !g.mhd || mhd_too : ctx->fused_sweep != 0;
   if (!want || !ctx->kt.sweep) return false;
-  // shock flattening has no swept form beside the whole-stage one
   if (g.sflat && ctx->kt.update_swept) return false;
   if (!ctx->kt.update_swept) return true;
   return (!g.mhd || g.sd == 2 || g.n1 % kSweepT == 0) &&

@@ -87,20 +87,21 @@ __device__ __forceinline__ double diff_k(double T, double rho, double kappa) {
   return Recip(rho * kappa).div(T * T * T);
 }
 
-// residuals_thermal_diffusion (:20394-20835), Cartesian, x1 first.
-template <int SD, int TS>
+// residuals_thermal_diffusion (:20394-20835), Cartesian, x1 first: 2D (3D:
+// k_diff_march's).
+template <int TS>
 __device__ __forceinline__ double diff_residual(const Grid &g, const double *e, int i, int j,
-                                                int k, double rc) {
-  const double tc = diff_temp_at<SD, TS>(g, e, cix(g, i, j, k), rc);
-  const double kc = diff_k(tc, rc, g.kappa[kapix(g, i, j, k)]);
+                                                double rc) {
+  const double tc = diff_temp_at<2, TS>(g, e, cix(g, i, j, 0), rc);
+  const double kc = diff_k(tc, rc, g.kappa[kapix(g, i, j, 0)]);
   double m = 0.0;
 #pragma unroll
-  for (int a = 0; a < SD; a++) {
+  for (int a = 0; a < 2; a++) {
     double tm, rm, tq, rq;
-    diff_cell<SD, TS>(g, e, i, j, k, a, -1, tm, rm);
-    diff_cell<SD, TS>(g, e, i, j, k, a, +1, tq, rq);
-    const double km = diff_k(tm, rm, g.kappa[kapix(g, i - (a == 0), j - (a == 1), k - (a == 2))]);
-    const double kq = diff_k(tq, rq, g.kappa[kapix(g, i + (a == 0), j + (a == 1), k + (a == 2))]);
+    diff_cell<2, TS>(g, e, i, j, 0, a, -1, tm, rm);
+    diff_cell<2, TS>(g, e, i, j, 0, a, +1, tq, rq);
+    const double km = diff_k(tm, rm, g.kappa[kapix(g, i - (a == 0), j - (a == 1), 0)]);
+    const double kq = diff_k(tq, rq, g.kappa[kapix(g, i + (a == 0), j + (a == 1), 0)]);
     const double fm = diff_face(tm, km, tc, kc, g.inv_dx[a]);
     const double fp = diff_face(tc, kc, tq, kq, g.inv_dx[a]);
     const double d = (fp - fm) * g.inv_dx[a];
@@ -141,22 +142,21 @@ __device__ __forceinline__ void diff_combine(const Grid &g, long long c, double 
   }
 }
 
-// The block order gives each XCD contiguous planes, whose rows and the planes
-// beside them its L2 holds.
-template <int SD, int TS, bool FIRST, bool LAST>
+// The 2D stage, flat.  The block order gives each XCD contiguous rows, and the
+// rows beside them to its L2.
+template <int TS, bool FIRST, bool LAST>
 __global__ void __launch_bounds__(256)
-    k_diff_stage(Grid g, unsigned nbx, unsigned nby, const double *ejm1, const double *ejm2,
-                 double *ej, double mu, double nu, double c0, double hm, double hg) {
+    k_diff_stage(Grid g, unsigned nbx, const double *ejm1, const double *ejm2, double *ej,
+                 double mu, double nu, double c0, double hm, double hg) {
   if (!g.sc->active) return;
   const unsigned w = xcd_contiguous(blockIdx.x, gridDim.x);
   const int i = (w % nbx) * blockDim.x + threadIdx.x;
-  const int j = (w / nbx % nby) * blockDim.y + threadIdx.y;
-  const int k = w / nbx / nby;
+  const int j = (w / nbx) * blockDim.y + threadIdx.y;
   if (i >= g.n1 || j >= g.n2) return;
-  const long long c = cix(g, i, j, k);
+  const long long c = cix(g, i, j, 0);
   const double rho = g.P[c];
-  const double m = diff_residual<SD, TS>(g, ejm1, i, j, k, rho);
-  diff_combine<SD, FIRST, LAST>(g, c, rho, m, ejm1[c], ejm2, ej, mu, nu, c0, hm, hg);
+  const double m = diff_residual<TS>(g, ejm1, i, j, rho);
+  diff_combine<2, FIRST, LAST>(g, c, rho, m, ejm1[c], ejm2, ej, mu, nu, c0, hm, hg);
 }
 
 // The 3D stage, marching: a block takes kDiffX x kDiffY columns through kc
@@ -355,8 +355,8 @@ static void diff_stage(const Grid &g, const double *ejm1, const double *ejm2, do
                                                                   mu, nu, c0, hm, hg);
   } else {
     const dim3 b = cell_block(g), n = diff_grid(g);
-    k_diff_stage<SD, TS, FIRST, LAST>
-        <<<n.x * n.y * n.z, b, 0, st>>>(g, n.x, n.y, ejm1, ejm2, ej, mu, nu, c0, hm, hg);
+    k_diff_stage<TS, FIRST, LAST>
+        <<<n.x * n.y, b, 0, st>>>(g, n.x, ejm1, ejm2, ej, mu, nu, c0, hm, hg);
   }
 }
 template <int SD>

@@ -58,11 +58,9 @@ struct HelmCell {
 // which holds every table value of the evaluation live at once.
 __device__ __forceinline__ void helm_pin(double &v) { asm volatile("" : "+v"(v)); }
 
-// a / b; FAST (the mixed-precision EoS step only): the hardware reciprocal
-// refined by two Newton steps (~1 ulp) instead of the correctly rounded form.
-template <bool FAST>
+// a / b of the mixed-precision EoS step: the hardware reciprocal refined by two
+// Newton steps (~1 ulp) instead of Recip's corrected quotient.
 __device__ __forceinline__ double hdiv(double a, double b) {
-  if (!FAST) return Recip(b).div(a);
   double r = __builtin_amdgcn_rcp(b);
   double e = fma(-b, r, 1.0);
   r = fma(r, e, r);
@@ -95,31 +93,25 @@ __device__ __forceinline__ int helm_index(double x, double l1, double d, double 
   return i < 0 ? 0 : (i > n - 2 ? n - 2 : i);
 }
 
-// FAST (the mixed-precision EoS step only): the index from the FP32 base-2
+// The cell of the mixed-precision EoS step: the index from the FP32 base-2
 // logarithm (v_log_f32); within ~1e-5 of a node it may pick the neighbouring
 // cell, whose quintic Hermite interpolant matches value, slope and curvature
 // there, and the offsets x, y are still formed in FP64 from the table's nodes.
-template <bool FAST = false>
 __device__ __forceinline__ HelmCell helm_locate(const HelmDev &h, double rhos, double T) {
   HelmCell c;
-  if (FAST) {
-    constexpr float kLog10of2 = 0.30102999566398120f;
-    const float lr = __builtin_amdgcn_logf((float)rhos) * kLog10of2;
-    const float lt = __builtin_amdgcn_logf((float)T) * kLog10of2;
-    c.ih = (int)((lr - (float)h.lrho1) * __builtin_amdgcn_rcpf((float)h.dr));
-    c.jh = (int)((lt - (float)h.lT1) * __builtin_amdgcn_rcpf((float)h.dt));
-    c.ih = c.ih < 0 ? 0 : (c.ih > h.nr - 2 ? h.nr - 2 : c.ih);
-    c.jh = c.jh < 0 ? 0 : (c.jh > h.nt - 2 ? h.nt - 2 : c.jh);
-  } else {
-    c.ih = helm_index(rhos, h.lrho1, h.dr, h.idr, h.nr);
-    c.jh = helm_index(T, h.lT1, h.dt, h.idt, h.nt);
-  }
+  constexpr float kLog10of2 = 0.30102999566398120f;
+  const float lr = __builtin_amdgcn_logf((float)rhos) * kLog10of2;
+  const float lt = __builtin_amdgcn_logf((float)T) * kLog10of2;
+  c.ih = (int)((lr - (float)h.lrho1) * __builtin_amdgcn_rcpf((float)h.dr));
+  c.jh = (int)((lt - (float)h.lT1) * __builtin_amdgcn_rcpf((float)h.dt));
+  c.ih = c.ih < 0 ? 0 : (c.ih > h.nr - 2 ? h.nr - 2 : c.ih);
+  c.jh = c.jh < 0 ? 0 : (c.jh > h.nt - 2 ? h.nt - 2 : c.jh);
   double tmp = h.rho[c.ih];
   c.drho = h.rho[c.ih + 1] - tmp;
-  c.x = hdiv<FAST>(rhos - tmp, c.drho);
+  c.x = hdiv(rhos - tmp, c.drho);
   tmp = h.T[c.jh];
   c.dT = h.T[c.jh + 1] - tmp;
-  c.y = hdiv<FAST>(T - tmp, c.dT);
+  c.y = hdiv(T - tmp, c.dT);
   return c;
 }
 
@@ -329,13 +321,13 @@ __device__ __forceinline__ double helm_sum16(const HelmDev &h, const HelmCell &c
 __device__ __forceinline__ void helm_full_fma(const HelmDev &h, double rho, double T, double abar,
                                               double zbar, double &P, double &E, double &sound,
                                               double &cv, double *dPdT_out) {
-  const double Ye = h.pig ? 1.0 : hdiv<true>(zbar, abar), rhos = rho * Ye;
-  const HelmCell c = helm_locate<true>(h, rhos, T);
+  const double Ye = h.pig ? 1.0 : hdiv(zbar, abar), rhos = rho * Ye;
+  const HelmCell c = helm_locate(h, rhos, T);
   HelmBasis r, dr, t, dt, ddt;
   helm_basis(c.x, c.drho, r);
-  helm_dbasis(c.x, c.drho, hdiv<true>(1.0, c.drho), dr);
+  helm_dbasis(c.x, c.drho, hdiv(1.0, c.drho), dr);
   helm_basis(c.y, c.dT, t);
-  const double idT = hdiv<true>(1.0, c.dT);
+  const double idT = hdiv(1.0, c.dT);
   helm_dbasis(c.y, c.dT, idT, dt);
   helm_ddbasis(c.y, c.dT, idT, ddt);
   const HelmBasis *const RR[2] = {&r, &dr};
@@ -356,7 +348,7 @@ __device__ __forceinline__ void helm_full_fma(const HelmDev &h, double rho, doub
   const double ds_dT = -Ye * df_dT2;
   double e = Ye * f + T * s;
   double dE_dT = T * ds_dT;
-  tmp = h.pig ? 0.0 : hdiv<true>(1.0, abar);
+  tmp = h.pig ? 0.0 : hdiv(1.0, abar);
   const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
   const double pion = kHelmRgas * rho * T * tmp;
   const double dpiondt = kHelmRgas * rho * tmp;
@@ -364,18 +356,18 @@ __device__ __forceinline__ void helm_full_fma(const HelmDev &h, double rho, doub
   p = p + pion + kHelmCrad * T4 * (1.0 / 3.0);
   dP_dT = dP_dT + dpiondt + (4.0 / 3.0) * kHelmCrad * T3;
   dP_drho = dP_drho + dpiondd;
-  e = e + 1.5 * kHelmRgas * T * tmp + hdiv<true>(kHelmCrad * T4, rho);
-  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv<true>(4.0 * kHelmCrad * T3, rho);
-  const double zz = hdiv<true>(p, rho);
-  const double chiT = hdiv<true>(T, p) * dP_dT;
-  const double chirho = hdiv<true>(dP_drho, zz);
-  const double x = hdiv<true>(zz * chiT, T * dE_dT);
+  e = e + 1.5 * kHelmRgas * T * tmp + hdiv(kHelmCrad * T4, rho);
+  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv(4.0 * kHelmCrad * T3, rho);
+  const double zz = hdiv(p, rho);
+  const double chiT = hdiv(T, p) * dP_dT;
+  const double chirho = hdiv(dP_drho, zz);
+  const double x = hdiv(zz * chiT, T * dE_dT);
   const double gam1 = chiT * x + chirho;
-  const double z = 1.0 + hdiv<true>(e + kHelmClight2, zz);
+  const double z = 1.0 + hdiv(e + kHelmClight2, zz);
   P = p;
   E = e;
   cv = dE_dT;
-  sound = kHelmClight * sqrt(hdiv<true>(gam1, z));
+  sound = kHelmClight * sqrt(hdiv(gam1, z));
   if (dPdT_out) *dPdT_out = dP_dT;
 }
 
@@ -398,7 +390,7 @@ struct HelmMx {
 };
 
 __device__ __forceinline__ void helm_mx_contract(const HelmDev &h, double T, HelmMx &m) {
-  const HelmCell c = helm_locate<true>(h, m.rhos, T);
+  const HelmCell c = helm_locate(h, m.rhos, T);
   m.ih = c.ih;
   m.jh = c.jh;
   m.x = c.x;
@@ -407,7 +399,7 @@ __device__ __forceinline__ void helm_mx_contract(const HelmDev &h, double T, Hel
   m.Tj = h.T[c.jh];
   HelmBasis r, dr;
   helm_basis(c.x, c.drho, r);
-  helm_dbasis(c.x, c.drho, hdiv<true>(1.0, c.drho), dr);
+  helm_dbasis(c.x, c.drho, hdiv(1.0, c.drho), dr);
   {
     const HelmBasis *const RR[2] = {&r, &dr};
     double G[2][6];
@@ -442,9 +434,9 @@ __device__ __forceinline__ void helm_mx_contract(const HelmDev &h, double T, Hel
 
 __device__ __forceinline__ void helm_mx_setup(const HelmDev &h, double rho, double T, double abar,
                                               double zbar, HelmMx &m) {
-  m.Ye = h.pig ? 1.0 : hdiv<true>(zbar, abar);
+  m.Ye = h.pig ? 1.0 : hdiv(zbar, abar);
   m.rhos = rho * m.Ye;
-  m.iabar = h.pig ? 0.0 : hdiv<true>(1.0, abar);
+  m.iabar = h.pig ? 0.0 : hdiv(1.0, abar);
   helm_mx_contract(h, T, m);
 }
 
@@ -460,15 +452,15 @@ struct HelmMxAt {
 
 __device__ __forceinline__ void helm_mx_energy(const HelmDev &h, HelmMx &m, double rho, double T,
                                                HelmMxAt &a, double &E, double &cv) {
-  double y = hdiv<true>(T - m.Tj, m.dT);
+  double y = hdiv(T - m.Tj, m.dT);
   if (y < -0.01 || y > 1.01) {
     helm_mx_contract(h, T, m);
-    y = hdiv<true>(T - m.Tj, m.dT);
+    y = hdiv(T - m.Tj, m.dT);
   }
   a.y = y;
   HelmBasis ddt;
   helm_basis(y, m.dT, a.t);
-  const double idT = hdiv<true>(1.0, m.dT);
+  const double idT = hdiv(1.0, m.dT);
   helm_dbasis(y, m.dT, idT, a.dt);
   helm_ddbasis(y, m.dT, idT, ddt);
   const double f = helm_contract_T(m.Gr, a.t);
@@ -480,8 +472,8 @@ __device__ __forceinline__ void helm_mx_energy(const HelmDev &h, HelmMx &m, doub
   double e = Ye * f + T * s;
   double dE_dT = T * ds_dT;
   const double T2 = T * T, T3 = T2 * T, T4 = T3 * T;
-  e = e + 1.5 * kHelmRgas * T * tmp + hdiv<true>(kHelmCrad * T4, rho);
-  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv<true>(4.0 * kHelmCrad * T3, rho);
+  e = e + 1.5 * kHelmRgas * T * tmp + hdiv(kHelmCrad * T4, rho);
+  dE_dT = dE_dT + 1.5 * kHelmRgas * tmp + hdiv(4.0 * kHelmCrad * T3, rho);
   E = e;
   cv = dE_dT;
 }
@@ -508,15 +500,15 @@ __device__ __forceinline__ void helm_mx_pressure(const HelmMx &m, double rho, do
   p = p + pion + kHelmCrad * T4 * (1.0 / 3.0);
   dP_dT = dP_dT + dpiondt + (4.0 / 3.0) * kHelmCrad * T3;
   dP_drho = dP_drho + dpiondd;
-  const double zz = hdiv<true>(p, rho);
-  const double chiT = hdiv<true>(T, p) * dP_dT;
-  const double chirho = hdiv<true>(dP_drho, zz);
-  const double xx = hdiv<true>(zz * chiT, T * cv);
+  const double zz = hdiv(p, rho);
+  const double chiT = hdiv(T, p) * dP_dT;
+  const double chirho = hdiv(dP_drho, zz);
+  const double xx = hdiv(zz * chiT, T * cv);
   const double gam1 = chiT * xx + chirho;
-  const double z = 1.0 + hdiv<true>(E + kHelmClight2, zz);
+  const double z = 1.0 + hdiv(E + kHelmClight2, zz);
   P = p;
   dPdT = dP_dT;
-  sound = kHelmClight * sqrt(hdiv<true>(gam1, z));
+  sound = kHelmClight * sqrt(hdiv(gam1, z));
 }
 
 // ---------------------------------------------------------------------------

@@ -30,8 +30,8 @@ struct KernelTable {
   // mixed precision: refresh the FP32 sweep inputs from the FP64 state
   void (*pack)(const Grid &, hipStream_t);
   void (*prims)(const Grid &, hipStream_t);   // mixed: FP64 prim / eint / b_cc from U
-  // fused sweep (2nd-order reconstructions, ideal / FASTEOS states, 3D or 2D
-  // ideal hydro; null otherwise): one pass forms the stage's conserved state
+  // fused sweep (2nd-order reconstructions, ideal / FASTEOS states, 3D, or the
+  // 2D ideal gas; null otherwise): one pass forms the stage's conserved state
   // and the swept updates finish it after CT; without update_swept (ideal
   // hydro) the pass is the whole stage, its new primitives in the other
   // buffer (Grid::Pn / Pfn).  Returns the blocks launched (partials of the CFL

@@ -1626,7 +1626,8 @@ __global__ void __launch_bounds__(256) k_divb(Grid g) {
 // ------------------------------------------------------------ fused sweep
 // One RK stage's reconstruction, Riemann fluxes and flux divergence in one
 // pass (the 2nd-order reconstructions, ideal or FASTEOS states; FP64 or the
-// mixed-precision policy; 3D, and 2D ideal hydro as the one plane).  A block of
+// mixed-precision policy; 3D, and the 2D ideal gas as the one plane, with MHD
+// without scalars).  A block of
 // 256 threads owns a 16 x 15 (x1, x2) tile of columns and walks a chunk of kc
 // planes along x3 (sweep_grid).
 // Per plane the tile plus a 2-cell halo of sweep inputs (WB deviations,
@@ -1652,8 +1653,8 @@ __global__ void __launch_bounds__(256) k_divb(Grid g) {
 // 100 -> 60 B per cell of the mixed ideal gas).
 // FUSE (the ideal gas without a field, where nothing stands between the RK
 // combination and cons -> prim): the pass is the whole stage.  The new
-// primitives go to a second buffer, since neighbouring blocks still read the
-// old ones, and the host swaps the two.  A 2D step is then three launches of
+// primitives go to another buffer, since neighbouring blocks still read the
+// old ones: that of one axis' fluxes, and the host swaps the two (next_prims).  A 2D step is then three launches of
 // ~10 us (101 x 93 FP64: 36 -> 22 us, 256^2 mixed 31 -> 20), and a 3D one reads
 // and writes U once less (384^3 LHLLC: FP64 12.5 -> 10.25 ms per step, mixed
 // 6.14 -> 5.89, where the mixed pass is bound by its face solves).
@@ -1718,7 +1719,7 @@ __global__ void __launch_bounds__(256)
   const long long N = g.N;
   if (!g.sc->active) {
     if constexpr (FUSE) {
-      // the other buffer becomes the current one (sweep_swap): it takes the
+      // the other buffer becomes the current one (next_prims): it takes the
       // state unchanged
       const int i = i0 + (tid & (TX - 1)), j = j0 + (tid >> 4);
       if ((tid >> 4) < TY && i < g.n1 && j < g.n2) {

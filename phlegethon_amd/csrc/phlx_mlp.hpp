@@ -283,10 +283,10 @@ __device__ __forceinline__ int helm_rhoe_lin(const HelmDev &h, double lin_tol, d
   helm_full_fma(h, rho, T, abar, zbar, P, E, sound, cv, &dPdT);
   cv_out = cv;
   const double res = E - E0;
-  const double dT = hdiv<true>(-res, cv);
+  const double dT = hdiv(-res, cv);
   const double T1 = T + dT;
   const bool inside = (T1 >= h.tl) && (T1 <= h.th);
-  if (fabs(hdiv<true>(res, E0)) < lin_tol && inside) {
+  if (fabs(hdiv(res, E0)) < lin_tol && inside) {
     T = T1;
     P = P + dPdT * dT;
     fallback = 0;
@@ -324,8 +324,8 @@ __device__ __forceinline__ int helm_rhoe_mixed(const HelmDev &h, double rho, dou
     helm_mx_energy(h, m, rho, T, at, E, cv);
     it++;
     const double res = E - E0;
-    double Tn = T - hdiv<true>(res, cv);
-    double err = fabs(hdiv<true>(res, E0));
+    double Tn = T - hdiv(res, cv);
+    double err = fabs(hdiv(res, E0));
     bool reset = false;
     if ((Tn < h.tl) || (Tn > h.th)) {
       Tn = Told;
@@ -361,7 +361,7 @@ __device__ __forceinline__ double helm_pred_start(double T, double e0, double e_
                                                   float cvf) {
   const double cv = (double)cvf;
   if (!(cv > 0.0) || !(e_prev == e_prev)) return T;
-  const double tg = T + hdiv<true>(e0 - e_prev, cv);
+  const double tg = T + hdiv(e0 - e_prev, cv);
   return (fabs(tg - T) <= 0.1 * T) ? tg : T;
 }
 

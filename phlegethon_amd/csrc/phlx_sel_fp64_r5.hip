@@ -12,6 +12,7 @@ bool select_fp64_r5(int sd, int nas, bool mhd, bool helm, bool fasteos, KernelTa
   base.sweep = nullptr;  // the fused sweep stages the 2nd-order stencil only
   base.update_swept = nullptr;
   base.update_swept_guess = nullptr;
+  base.update_swept_mlp = nullptr;
   t = base;
   return true;
 }
