@@ -1,6 +1,6 @@
 // phlx_fp64.hpp -- FP64 quotients and square roots of the kernels: the bits of
 // a / b and sqrt(x) in fewer instructions than the compiler's expansions.
-// Host code that provides the four hardware functions can include it too (the
+// Host code that provides the three hardware functions can include it too (the
 // arithmetic is checked that way, with seeds of any error up to the bound).
 #pragma once
 
@@ -16,8 +16,6 @@ PHLX_FP64_FN double hw_rsq(double x) { return __builtin_amdgcn_rsq(x); }
 PHLX_FP64_FN double hw_div_fixup(double q, double b, double a) {
   return __builtin_amdgcn_div_fixup(q, b, a);
 }
-// v_cmp_class_f64: -0, +0 or +infinity
-PHLX_FP64_FN bool hw_own_root(double x) { return __builtin_amdgcn_class(x, 0x260); }
 }  // namespace phlx
 #else
 #include <cmath>
@@ -26,7 +24,6 @@ namespace phlx {
 double hw_rcp(double x);
 double hw_rsq(double x);
 double hw_div_fixup(double q, double b, double a);
-bool hw_own_root(double x);
 using std::fma;
 }  // namespace phlx
 #endif
@@ -39,9 +36,9 @@ namespace phlx {
 // refined in one third-order step, r (1 + e + e^2), to half an ulp; a quotient is
 // the product with it corrected by its exact FMA remainder (Markstein's
 // theorem), and v_div_fixup puts zeros, infinities and NaN right: 4 instructions
-// and 4 per quotient (3 for 1 / b).  (Without v_div_fixup, which made an infinite
-// EoS target and a face with a zero sound speed NaN, 256^3 MHD runs 1.2 % faster
-// and the flattened 133 x 120 x 97 hydro 1.5 %.)
+// and 4 per quotient (3 for 1 / b).  (Without v_div_fixup an infinite
+// EoS target and a face with a zero sound speed came out NaN; it costs 256^3 MHD
+// 0.8 % of a step, 133 x 120 x 97 flattened hydro 1.0 %, 512^3 Helmholtz MHD 1.3 %.)
 // What the missing scaling and the single step cost:
 //   - 2^-1020 <= |b| <= 2^1020, or b a zero, an infinity or NaN.  A subnormal b
 //     gives NaN, or 0 for a = 0.  The callers' denominators are densities, speeds
@@ -59,12 +56,13 @@ struct Recip {
     r = fma(r0, fma(e, e, e), r0);
   }
   PHLX_FP64_FN double div(double a) const { return hw_div_fixup(div_finite(a), b, a); }
-  // div for a and b that are neither a zero nor an infinity nor NaN
+  // for a normal b and a finite a
   PHLX_FP64_FN double div_finite(double a) const {
     const double q = a * r;
     return fma(fma(-b, q, a), r, q);
   }
-  PHLX_FP64_FN double inv() const { return hw_div_fixup(fma(fma(-b, r, 1.0), r, r), b, 1.0); }
+  PHLX_FP64_FN double inv() const { return hw_div_fixup(inv_finite(), b, 1.0); }
+  PHLX_FP64_FN double inv_finite() const { return fma(fma(-b, r, 1.0), r, r); }
 };
 
 // The square root: two steps of Goldschmidt's iteration from the hardware's
@@ -77,13 +75,17 @@ struct Recip {
 PHLX_FP64_FN double dsqrt(double x) {
   const double y = hw_rsq(x);
   double s = x * y, h = 0.5 * y;
+  // y is an infinity or 0: x is -0, +0 or infinite, its own root (v_cmp_class on x
+  // would hold its mask in a register: 2D hydro at 4 waves per SIMD instead of 5,
+  // 3000^2 992 -> 1060 us per step)
+  const bool own = h == y;
   double r = fma(-h, s, 0.5);
   s = fma(s, r, s);
   h = fma(h, r, h);
   r = fma(-h, s, 0.5);
   s = fma(s, r, s);
   s = fma(fma(-s, s, x), h, s);
-  return hw_own_root(x) ? x : s;
+  return own ? x : s;
 }
 
 }  // namespace phlx

@@ -535,8 +535,9 @@ struct HelmRho {
     const double lo = h.rho[ih];
     drho = h.rho[ih + 1] - lo;
     const Recip rd(drho);
-    x = rd.div(rhos - lo);
-    idrho = rd.inv();
+    // an infinite offset makes the basis NaN either way
+    x = rd.div_finite(rhos - lo);
+    idrho = rd.inv_finite();
   }
 };
 
@@ -551,8 +552,8 @@ __device__ __forceinline__ HelmCell helm_cell(const HelmDev &h, const HelmRho &m
   const double lo = h.T[c.jh];
   c.dT = h.T[c.jh + 1] - lo;
   const Recip rd(c.dT);
-  c.y = rd.div(T - lo);
-  idT = rd.inv();
+  c.y = rd.div_finite(T - lo);
+  idT = rd.inv_finite();
   return c;
 }
 
@@ -591,17 +592,19 @@ __device__ __forceinline__ void helm_full_at(const HelmDev &h, const HelmRho &m,
   dP_drho = dP_drho + dpiondd;
   e = e + 1.5 * kHelmRgas * T * iabar + m.rrho.div(kHelmCrad * T4);
   dE_dT = dE_dT + 1.5 * kHelmRgas * iabar + m.rrho.div(4.0 * kHelmCrad * T3);
-  const double zz = m.rrho.div(p);
-  const double chiT = Recip(p).div(T) * dP_dT;
+  // a zero rho or p makes the sound speed NaN whichever of these is infinite,
+  // and c_v is positive
+  const double zz = m.rrho.div_finite(p);
+  const double chiT = Recip(p).div_finite(T) * dP_dT;
   const Recip rz(zz);
-  const double chirho = rz.div(dP_drho);
-  const double x = Recip(T * dE_dT).div(zz * chiT);
+  const double chirho = rz.div_finite(dP_drho);
+  const double x = Recip(T * dE_dT).div_finite(zz * chiT);
   const double gam1 = chiT * x + chirho;
-  const double z = 1.0 + rz.div(e + kHelmClight2);
+  const double z = 1.0 + rz.div_finite(e + kHelmClight2);
   P = p;
   E = e;
   cv = dE_dT;
-  sound = kHelmClight * dsqrt(Recip(z).div(gam1));
+  sound = kHelmClight * dsqrt(Recip(z).div_finite(gam1));
 }
 __device__ __forceinline__ void helm_full(const HelmDev &h, double rho, double T, double abar,
                                           double zbar, double &P, double &E, double &sound,
@@ -717,7 +720,7 @@ __device__ __forceinline__ int helm_rhoe_given(const HelmDev &h, const HelmRho &
     if (cv_last) *cv_last = dEdT;
     const double res = e - E0;
     T = T - Recip(dEdT).div(res);
-    double err = fabs(rE0.div(res));
+    double err = fabs(rE0.div_finite(res));  // infinite or NaN: not converged
     if ((T < h.tl) || (T > h.th)) {
       T = Told;
       err = 1e-15;
@@ -757,7 +760,7 @@ __device__ __forceinline__ int helm_rhoP_given(const HelmDev &h, double rho, dou
     helm_given1(h, m, tab, T, p, dPdT, true);
     const double res = p - P0;
     T = T - Recip(dPdT).div(res);
-    double err = fabs(rP0.div(res));
+    double err = fabs(rP0.div_finite(res));
     if ((T < h.tl) || (T > h.th)) {
       T = Told;
       err = 1e-15;

@@ -21,7 +21,6 @@ double hw_div_fixup(double q, double b, double a) {
   if (std::isinf(b) || a == 0.0) return sg * 0.0;
   return std::copysign(q, sg);
 }
-bool hw_own_root(double x) { return x == 0.0 || x == std::numeric_limits<double>::infinity(); }
 }  // namespace phlx
 
 using phlx::dsqrt;
