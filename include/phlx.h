@@ -166,18 +166,19 @@ int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, double a3,
  * It applies with LIM2ND or PPH to 3D runs with the ideal or the FASTEOS
  * Helmholtz state (with MHD, nx1 has to be a multiple of 16) and to 2D runs of
  * the ideal gas (with MHD: without scalars); with shock flattening to the
- * ideal gas without MHD.  Other runs take the separate sweeps.  Either way the results are bit for bit the
- * same.  No counterpart in the reference (its hydro_step is one routine either
- * way): for A/B timing and for callers that want the per-direction kernels. */
+ * ideal gas without MHD.  Other runs take the separate sweeps.  Either way the
+ * results are bit for bit the same.  No counterpart in the reference (its
+ * hydro_step is one routine either way): for A/B timing and for callers that
+ * want the per-direction kernels. */
 int phlx_set_fused_sweep(phlx_ctx *ctx, int32_t mode);
 /* Whether phlx_run replays one captured HIP graph per step (on = 1) instead
  * of launching the step's kernels one by one (0, the default).  The step is
- * captured on the first phlx_run that needs it and again whenever a setting
+ * captured on the first phlx_run that needs it (RK3 without MHD in two graphs,
+ * since its steps end in either of two buffers) and again whenever a setting
  * that changes its kernels or their arguments has changed; runs with
  * thermal diffusion or profiling launch eagerly.  The results are bit for
- * bit the same.  Measured on MI355X it is not faster (2D 256^2, where
- * each step is a dozen short kernels: 0.090 against 0.085 ms per step), so
- * it is off by default; it is for callers that embed the step in their own
+ * bit the same.  Measured on MI355X it is not faster (128^3 RK3 hydro 495
+ * against 490 us per step), so it is off by default; it is for callers that embed the step in their own
  * graphs or want one launch per step.  No counterpart in the reference. */
 int phlx_set_step_graph(phlx_ctx *ctx, int32_t on);
 

@@ -712,8 +712,10 @@ extern "C" int phlx_rk_update(phlx_ctx *ctx, int32_t irk, double a1, double a2, 
 
 // Whether hydro_step takes the fused sweep: a family that has one; shock
 // flattening, whose flagged cells switch scheme per face, in whole stages alone;
-// 3D MHD only where the x1 tiles divide the grid (partial ones, which hydro and
-// 2D MHD take, have not been run or timed there).
+// 3D MHD only where the x1 tiles divide the grid.  (On partial tiles it gives the
+// same bits, but a ragged row costs more than it saves on some grids: FP64 fused /
+// split 250^3 7242 / 7994 us per step, 150^3 1662 / 1743, 100 x 90 x 80 432 / 416,
+// 50 x 64 x 60 169 / 158.)
 static bool use_fused_sweep(const phlx_ctx *ctx) {
   const Grid &g = ctx->g;
   // measured on MI355X, us per step, fused / split: without MHD always the

@@ -45,7 +45,9 @@ namespace phlx {
 //     and their differences, cell widths, temperatures, energies, conductivities,
 //     and the limiter's sum of two slopes whose product is positive (> 2^-538).
 //   - for 2^-960 <= |a|, |a / b| <= 2^1000 the bits of a / b, unless that lies
-//     within 2^-45 ulp of the midpoint of two numbers: there either of the two.
+//     within 2^-45 ulp of the midpoint of two numbers: there either of the two
+//     (none of 1.6e10 pairs differed on gfx950, exponents to +-480, mantissas next
+//     to all ones and all zeros among them; nor did their roots).
 //   - below, where the remainder underflows, within 1.5 ulp of a / b: a product of
 //     slopes under 1e-289 (the limiter in a decaying tail), a field as small.
 struct Recip {

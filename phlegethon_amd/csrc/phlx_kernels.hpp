@@ -1659,16 +1659,16 @@ __global__ void __launch_bounds__(256) k_divb(Grid g) {
 // and writes U once less (384^3 LHLLC: FP64 12.5 -> 10.25 ms per step, mixed
 // 6.14 -> 5.89, where the mixed pass is bound by its face solves).
 // SF (FP64 whole stages): shock flattening, the flags staged beside the cells:
-// 133 x 120 x 97 224 -> 146 us per stage against the split sweeps and update,
-// 256^3 1800 -> 1117.
+// 133 x 120 x 97 224 -> 147 us per stage against the split sweeps and update,
+// 256^3 1910 -> 1120.
 // Last tiles past n1 or n2 mask their missing columns.
 template <int D>
 struct SweepDir {
   static constexpr int value = D;
 };
 // waves per SIMD the register allocation aims at (FP64; the FP32 sweeps).  With
-// shock flattening and no scalars 3, for 8 spilled registers (256^3: 1210 ->
-// 1080 us per stage, 133 x 120 x 97 152 -> 144); two scalars would spill 127.
+// shock flattening and no scalars 3, for 8 spilled registers (a tenth off the
+// time of 2 waves at 256^3, 5 % at 133 x 120 x 97); two scalars would spill 127.
 #ifndef PHLX_SWEEP_WAVES
 #define PHLX_SWEEP_WAVES 2
 #endif
