@@ -261,9 +261,12 @@ extern "C" int phlx_create(const phlx_config *cfg, phlx_ctx **out) {
     e |= dalloc(ctx, &g.F[d], nv * (size_t)g.nf[d]);
     g.Ff[d] = (float *)g.F[d];  // the mixed path stores FP32 fluxes in the same buffer
   }
-  if (whole) {
-    g.Pn = mix ? nullptr : g.F[ctx->pn_dir];
-    g.Pfn = mix ? g.Ff[ctx->pn_dir] : nullptr;
+  if (whole && mix) {
+    g.Pfn = g.Ff[ctx->pn_dir];
+    g.F[ctx->pn_dir] = nullptr;
+  } else if (whole) {
+    g.Pn = g.F[ctx->pn_dir];
+    g.Ff[ctx->pn_dir] = nullptr;
   }
   if (g.mhd) {
     e |= dalloc(ctx, &g.bcc, 3 * N);
@@ -771,11 +774,9 @@ static void next_prims(phlx_ctx *ctx) {
   if (g.Pfn) {
     std::swap(g.Pf, g.Pfn);
     g.Ff[d] = g.Pfn;
-    g.F[d] = nullptr;
   } else {
     std::swap(g.P, g.Pn);
     g.F[d] = g.Pn;
-    g.Ff[d] = nullptr;
   }
 }
 
