@@ -54,6 +54,24 @@ def test_unreachable_eos_targets(oracle_mod, ret):
         eos.close()
 
 
+def test_eos_of_no_matter_and_no_limit(oracle_mod):
+    """rho = 0 (an infinite specific energy and c_v from the radiation), T = 0,
+    and infinite ones."""
+    from phlegethon_amd.runtime import HelmEoS
+    table = H.default_table()
+    eos, orc = HelmEoS(table), oracle_mod.OracleHelm(table)
+    v = np.array([0.0, 1.0, 1e7, np.inf])
+    rho, T = (x.ravel() for x in np.meshgrid(v, v))
+    abar, zbar = np.full(rho.size, 12.0), np.full(rho.size, 6.0)
+    try:
+        got, ref = eos.full(rho, T, abar, zbar), orc.full(rho, T, abar, zbar)
+        assert np.any(np.isinf(ref[1])) and np.any(np.isfinite(ref[1]))
+        for a, b in zip(got, ref):
+            assert _equal(a, b)
+    finally:
+        eos.close()
+
+
 def _run_both(pb, oracle_mod, nsteps=1):
     from phlegethon_amd.runtime import Simulation
     out = []
